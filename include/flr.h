@@ -279,6 +279,22 @@ typedef struct {
 int flr_gb_generate(const flr_gb_source *sources, int num_sources, int64_t total_samples,
                     double dt, int format, void *out, void *stream);
 
+/* ------------------------------------------------------------------ packed series
+ * No counterpart in the reference. Statistics of the sources of a packed series, and its
+ * conversion to the 8-byte input formats of the mixed kernels. `offsets` (device, num_sources + 1
+ * sample indexes) may be NULL for one source of max_len samples; max_len is the longest source.
+ * stats (device): 4 doubles per source, max |h|, max(|Re h|, |Im h|), sum |h|^2 and
+ * sum |h[i+1] - h[i]|^2 (NaN where a sample is NaN), the same whatever else runs; `format` is the
+ * series' (FLR_GB_*). work: flr_series_work doubles of device memory. */
+int64_t flr_series_work(int num_sources, int64_t max_len);
+int flr_series_stats(const void *h, int format, const int64_t *offsets, int num_sources,
+                     int64_t max_len, double *work, int64_t work_len, double *stats, void *stream);
+/* Pack complex128 h with those statistics: FLR_GB_COMPLEX64 stores h * (1 / max |h|), FLR_GB_Q31
+ * round(x * ((2^31 - 1) / max(|Re h|, |Im h|))) per component; a scale that is not positive is
+ * taken as 1. */
+int flr_series_pack(const double *h, const int64_t *offsets, int num_sources, int64_t max_len,
+                    const double *stats, int format, void *out, void *stream);
+
 /* Stencil form used by the drop-in entry points flr_get_response / flr_get_tdi_delays:
  * nonzero (default) the reference operation order, bitwise equal to the FP64 CPU path;
  * 0 the faster reciprocal-free form (equal to ~1e-15 relative per stencil). */

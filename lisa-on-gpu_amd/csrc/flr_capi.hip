@@ -1384,6 +1384,52 @@ int flr_gb_generate(const flr_gb_source *sources, int num_sources, int64_t total
     return FLR_OK;
 }
 
+namespace {
+
+int series_args(const void *h, int num_sources, const int64_t *offsets, int64_t max_len)
+{
+    if (!h || num_sources < 1) return fail(FLR_ERR_INVALID_ARGUMENT, "no series");
+    if (!offsets && num_sources > 1)
+        return fail(FLR_ERR_INVALID_ARGUMENT, "several sources need their offsets");
+    if (max_len < 1 || series_chunks(max_len) > INT32_MAX)
+        return fail(FLR_ERR_INVALID_ARGUMENT, "bad series length");
+    return FLR_OK;
+}
+
+}  // namespace
+
+int64_t flr_series_work(int num_sources, int64_t max_len)
+{
+    return num_sources < 1 || max_len < 1 ? 0 : 4 * (int64_t)num_sources * series_chunks(max_len);
+}
+
+int flr_series_stats(const void *h, int format, const int64_t *offsets, int num_sources,
+                     int64_t max_len, double *work, int64_t work_len, double *stats, void *stream)
+{
+    int st = series_args(h, num_sources, offsets, max_len);
+    if (st) return st;
+    if (format != FLR_GB_COMPLEX128 && format != FLR_GB_COMPLEX64 && format != FLR_GB_Q31)
+        return fail(FLR_ERR_INVALID_ARGUMENT, "unknown series format");
+    if (!work || !stats || work_len < flr_series_work(num_sources, max_len))
+        return fail(FLR_ERR_INVALID_ARGUMENT, "work is smaller than flr_series_work doubles");
+    hipError_t e = launch_series_stats(h, format, offsets, num_sources, max_len, work, stats,
+                                       (hipStream_t)stream);
+    return e != hipSuccess ? hip_fail(e, "series statistics launch") : FLR_OK;
+}
+
+int flr_series_pack(const double *h, const int64_t *offsets, int num_sources, int64_t max_len,
+                    const double *stats, int format, void *out, void *stream)
+{
+    int st = series_args(h, num_sources, offsets, max_len);
+    if (st) return st;
+    if (format != FLR_GB_COMPLEX64 && format != FLR_GB_Q31)
+        return fail(FLR_ERR_INVALID_ARGUMENT, "a series packs into complex64 or q31");
+    if (!stats || !out) return fail(FLR_ERR_INVALID_ARGUMENT, "NULL statistics or output");
+    hipError_t e = launch_series_pack(h, offsets, num_sources, max_len, stats, format, out,
+                                      (hipStream_t)stream);
+    return e != hipSuccess ? hip_fail(e, "series pack launch") : FLR_OK;
+}
+
 int flr_response_set_exact(flr_response *r, int exact)
 {
     if (!r) return fail(FLR_ERR_INVALID_ARGUMENT, "response is NULL");

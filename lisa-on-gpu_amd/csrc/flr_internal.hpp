@@ -231,6 +231,14 @@ hipError_t launch_inner_reduce(const double *part, const int *tile_start, int nu
 // Galactic-binary generator (flr_waveform.hip).
 hipError_t launch_gb(const flr_gb_source *sources, int num_sources, int64_t total, double dt,
                      int format, void *out, hipStream_t stream);
+// Statistics and 8-byte formats of a packed series (flr_pack.hip); series_chunks(max_len): the
+// partial records (4 doubles each) per source that the statistics need as work space.
+int64_t series_chunks(int64_t max_len);
+hipError_t launch_series_stats(const void *h, int format, const int64_t *offsets, int num_sources,
+                               int64_t max_len, double *work, double *stats, hipStream_t stream);
+hipError_t launch_series_pack(const void *h, const int64_t *offsets, int num_sources,
+                              int64_t max_len, const double *stats, int format, void *out,
+                              hipStream_t stream);
 hipError_t launch_orbit_eval(const OrbitView &orb, const double *t, int n, int row, int sc,
                              double *ltt_out, double *pos_out, hipStream_t stream);
 hipError_t launch_clear(int *word, hipStream_t stream);

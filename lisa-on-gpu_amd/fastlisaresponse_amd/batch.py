@@ -70,12 +70,76 @@ def storage_error_estimate(f, precision: str, armlength: float = 2.5e9):
     return est if est.ndim else float(est)
 
 
+_SERIES_FORMATS = {torch.complex128: _capi.FLR_GB_COMPLEX128,
+                   torch.complex64: _capi.FLR_GB_COMPLEX64, torch.int32: _capi.FLR_GB_Q31}
+
+
+def _on_device(h) -> bool:
+    """Whether the statistics and conversions of h run in the HIP kernels: a GPU tensor of one of
+    the stored formats that no gradient is recorded for. Host tensors take the torch forms."""
+    return (type(h) is torch.Tensor and h.is_cuda and h.dim() == 1 and h.dtype in _SERIES_FORMATS
+            and not h.requires_grad)
+
+
+def _flat(h: torch.Tensor) -> torch.Tensor:
+    """h's values in memory order (a conjugated or strided view is written out)."""
+    return h.resolve_conj().resolve_neg().contiguous()
+
+
+class _SeriesStats:
+    """Per-source statistics of a packed device series: max |h|, max(|Re|, |Im|), sum |h|^2 and
+    sum |h[i+1] - h[i]|^2 (flr_series_stats), enqueued on the current stream."""
+
+    def __init__(self, h: torch.Tensor, lengths: Sequence[int]):
+        self.h = _flat(h)
+        self.num = len(lengths)
+        self.max_len = max(lengths)
+        with torch.cuda.device(h.device):
+            self.offsets = None
+            if self.num > 1:
+                self.offsets = torch.as_tensor(np.concatenate([[0], np.cumsum(lengths)]),
+                                               dtype=torch.int64).to(h.device)
+            self.stats = torch.empty((self.num, 4), dtype=torch.float64, device=h.device)
+            nwork = int(lib().flr_series_work(self.num, self.max_len))
+            work = torch.empty(nwork, dtype=torch.float64, device=h.device)
+            check(lib().flr_series_stats(self.h.data_ptr(), _SERIES_FORMATS[h.dtype], self._offs(),
+                                         self.num, self.max_len, work.data_ptr(), nwork,
+                                         self.stats.data_ptr(), current_stream()))
+
+    def _offs(self):
+        return None if self.offsets is None else self.offsets.data_ptr()
+
+    def pack(self, fmt: int) -> torch.Tensor:
+        """The complex128 series as complex64 or q31 (flr_series_pack), on the current stream."""
+        n = self.h.numel()
+        with torch.cuda.device(self.h.device):
+            out = (torch.empty(2 * n, dtype=torch.int32, device=self.h.device)
+                   if fmt == _capi.FLR_GB_Q31 else
+                   torch.empty(n, dtype=torch.complex64, device=self.h.device))
+            check(lib().flr_series_pack(self.h.data_ptr(), self._offs(), self.num, self.max_len,
+                                        self.stats.data_ptr(), fmt, out.data_ptr(),
+                                        current_stream()))
+        return out
+
+
+def _rms(p, d, lengths, dt: float) -> np.ndarray:
+    """RMS frequencies from the sums of |h|^2 and of |h[i+1] - h[i]|^2 per source."""
+    p, d = p / np.maximum(lengths, 1), d / np.maximum(lengths - 1, 1)
+    with np.errstate(divide="ignore", invalid="ignore"):
+        r = np.sqrt(np.where(p > 0.0, d / np.maximum(p, 1e-300), 0.0))
+    return 2.0 * np.arcsin(np.minimum(r, 2.0) / 2.0) / (2.0 * np.pi * dt)
+
+
 def rms_frequencies(h: torch.Tensor, lengths: Sequence[int], dt: float) -> np.ndarray:
     """RMS frequency (Hz) of each source of a packed complex series: with r^2 = mean |h[i+1] -
     h[i]|^2 / mean |h[i]|^2 over the source, f = 2 arcsin(r / 2) / (2 pi dt), which is exact for a
-    single complex sinusoid. One pass over the samples (per-source sums by index), one host
-    sync."""
+    single complex sinusoid. One pass over the samples (flr_series_stats on the device, sums by
+    index for host tensors), one host sync."""
     lengths = np.asarray([int(n) for n in lengths], dtype=np.int64)
+    if _on_device(h) and len(lengths) and lengths.min() > 0 and \
+            int(lengths.sum()) == h.numel() // (2 if h.dtype == torch.int32 else 1):
+        st = _SeriesStats(h, lengths.tolist()).stats.cpu().numpy()
+        return _rms(st[:, 2], st[:, 3], lengths, dt)
     if h.dtype == torch.int32:  # q31 pairs
         h = torch.view_as_complex(h.view(-1, 2).to(torch.float64).contiguous())
     h = h.to(torch.complex128) if h.dtype != torch.complex128 else h
@@ -89,10 +153,7 @@ def rms_frequencies(h: torch.Tensor, lengths: Sequence[int], dt: float) -> np.nd
         diff = (h[1:] - h[:-1]).abs().square()
         same = ids[1:] == ids[:-1]  # no differences across source boundaries
         d.index_add_(0, ids[1:][same], diff[same])
-    p, d = p.cpu().numpy() / np.maximum(lengths, 1), d.cpu().numpy() / np.maximum(lengths - 1, 1)
-    with np.errstate(divide="ignore", invalid="ignore"):
-        r = np.sqrt(np.where(p > 0.0, d / np.maximum(p, 1e-300), 0.0))
-    return 2.0 * np.arcsin(np.minimum(r, 2.0) / 2.0) / (2.0 * np.pi * dt)
+    return _rms(p.cpu().numpy(), d.cpu().numpy(), lengths, dt)
 
 
 def check_storage(h: torch.Tensor, lengths: Sequence[int], dt: float, precision: str,
@@ -104,8 +165,13 @@ def check_storage(h: torch.Tensor, lengths: Sequence[int], dt: float, precision:
         raise ValueError("action must be 'warn', 'raise' or 'off'")
     if action == "off" or STORAGE_K[precision] == 0.0:
         return np.zeros(len(lengths))
-    est = np.atleast_1d(storage_error_estimate(rms_frequencies(h, lengths, dt), precision,
-                                               armlength))
+    return _storage_verdict(rms_frequencies(h, lengths, dt), precision, armlength, tol, action, 4)
+
+
+def _storage_verdict(rms, precision: str, armlength: float, tol: float, action: str,
+                     stacklevel: int):
+    """The estimates at the sources' RMS frequencies, with check_storage's warning or error."""
+    est = np.atleast_1d(storage_error_estimate(rms, precision, armlength))
     bad = np.flatnonzero(est > tol)
     if bad.size:
         msg = (f"precision={precision!r}: {bad.size} of {len(est)} source(s) have an estimated "
@@ -115,8 +181,40 @@ def check_storage(h: torch.Tensor, lengths: Sequence[int], dt: float, precision:
                "error at the same speed")
         if action == "raise":
             raise ValueError(msg)
-        warnings.warn(msg, StorageErrorWarning, stacklevel=3)
+        warnings.warn(msg, StorageErrorWarning, stacklevel=stacklevel)
     return est
+
+
+def pack_checked(h: torch.Tensor, dt: float, precision: str, armlength: float, action: str):
+    """One source's complex128 series in the 8-byte format of `precision` ("mixed" or "mixed-q31")
+    and its scale, after check_storage's verdict on it: one pass for the statistics, one for the
+    conversion, one transfer to the host."""
+    pack = pack_q31 if precision == "mixed-q31" else pack_mixed
+    n = len(h)
+    if not (_on_device(h) and h.dtype == torch.complex128 and n):
+        check_storage(h, [n], dt, precision, armlength, action=action)
+        stored, scales = pack(h, [n])
+        return stored, scales[0]
+    series = _SeriesStats(h, [n])
+    stored = series.pack(_capi.FLR_GB_Q31 if precision == "mixed-q31" else _capi.FLR_GB_COMPLEX64)
+    st = series.stats.cpu().numpy()
+    if action != "off":
+        _storage_verdict(_rms(st[:, 2], st[:, 3], np.asarray([n]), dt), precision, armlength,
+                         STORAGE_TOL, action, 4)
+    return stored, _scales(st, precision)[0]
+
+
+def _scales(stats: np.ndarray, precision: str):
+    """The scales of the packed formats from the statistics (pack_mixed, pack_q31)."""
+    top = stats[:, 1 if precision == "mixed-q31" else 0]
+    top = [float(v) if v > 0.0 else 1.0 for v in top]
+    return [v / float(2 ** 31 - 1) for v in top] if precision == "mixed-q31" else top
+
+
+def _pack_on_device(h: torch.Tensor, lengths: Sequence[int], precision: str):
+    series = _SeriesStats(h, lengths)
+    stored = series.pack(_capi.FLR_GB_Q31 if precision == "mixed-q31" else _capi.FLR_GB_COMPLEX64)
+    return stored, _scales(series.stats.cpu().numpy(), precision)
 
 
 def pack_mixed(h: torch.Tensor, lengths: Sequence[int]):
@@ -127,6 +225,8 @@ def pack_mixed(h: torch.Tensor, lengths: Sequence[int]):
     lengths = [int(n) for n in lengths]
     if sum(lengths) != h.numel():
         raise ValueError("lengths do not add up to the number of samples")
+    if _on_device(h) and lengths and min(lengths) > 0:
+        return _pack_on_device(h, lengths, "mixed")
     out = torch.empty(h.numel(), dtype=torch.complex64, device=h.device)
     scales = []
     o = 0
@@ -150,6 +250,8 @@ def pack_q31(h: torch.Tensor, lengths: Sequence[int]):
     lengths = [int(n) for n in lengths]
     if sum(lengths) != h.numel():
         raise ValueError("lengths do not add up to the number of samples")
+    if _on_device(h) and lengths and min(lengths) > 0:
+        return _pack_on_device(h, lengths, "mixed-q31")
     full = float(2 ** 31 - 1)
     out = torch.empty(2 * h.numel(), dtype=torch.int32, device=h.device)
     scales = []

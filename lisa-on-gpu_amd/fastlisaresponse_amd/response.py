@@ -335,15 +335,12 @@ class pyResponseTDI:
         h = h.to(device=self.device, dtype=torch.complex128).contiguous()
         self._input_keepalive = h
         if self.precision != "fp64":
-            from .batch import check_storage, pack_mixed, pack_q31
             if self.precision == "mixed-c128":
                 stored, scale = h, 1.0
             else:
-                check_storage(h, [len(h)], self.dt, self.precision,
-                              self.response_orbits.armlength, action=self.storage_check)
-                pack = pack_q31 if self.precision == "mixed-q31" else pack_mixed
-                stored, scales = pack(h, [len(h)])
-                scale = scales[0]
+                from .batch import pack_checked
+                stored, scale = pack_checked(h, self.dt, self.precision,
+                                             self.response_orbits.armlength, self.storage_check)
             self._mixed = (stored, scale, k, u, v)
             self.y_gw_flat = None
             self.y_gw_length = self.num_pts
