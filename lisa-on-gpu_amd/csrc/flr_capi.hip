@@ -158,6 +158,8 @@ struct flr_batch {
     int *d_proj_tiles = nullptr;  // [num_sources + 1] prefix sums
     int *d_tdi_tiles = nullptr;
     int proj_tiles = 0, tdi_tiles = 0;
+    int proj_min_start = 0, tdi_min_start = 0;  // smallest start index over the sources
+    int fused_min_start = 0;      // smallest tdi_start over the bound sources
     bool fused = false;           // one fused launch over d_fused / d_fused_tiles
     FusedSource *d_fused = nullptr;
     int *d_fused_tiles = nullptr;
@@ -972,6 +974,12 @@ int flr_batch_create(flr_response *r, const flr_source *sources, int num_sources
     b->fs = sampling_frequency;
     b->num_sources = num_sources;
     b->samples = samples;
+    b->proj_min_start = ps[0].start;
+    b->tdi_min_start = ts[0].start;
+    for (int s = 1; s < num_sources; ++s) {
+        b->proj_min_start = std::min(b->proj_min_start, ps[s].start);
+        b->tdi_min_start = std::min(b->tdi_min_start, ts[s].start);
+    }
     b->proj_tiles = pt[num_sources];
     b->tdi_tiles = tt[num_sources];
     hipError_t e = hipMalloc(&b->d_proj, sizeof(ProjSource) * num_sources);
@@ -1180,6 +1188,9 @@ int flr_fused_bind(flr_batch *b, const flr_source *sources, int num_sources, con
                            hipMemcpyHostToDevice, st));
     b->num_sources = num_sources;
     b->samples = samples;
+    b->fused_min_start = fs[0].tdi_start;
+    for (int s = 1; s < num_sources; ++s)
+        b->fused_min_start = std::min(b->fused_min_start, fs[s].tdi_start);
     b->fused_tiles = ft[num_sources];
     b->out_base = out_all;
     if (!same_refs) b->lti_version = ~0ull;  // new sources: their filters are built now
@@ -1251,7 +1262,8 @@ int fused_launch(flr_batch *b, hipStream_t s, const void *data, double *sums)
         b->inner_cap = b->fused_tiles;
     }
     if ((st = lti_refresh(b, s))) return st;
-    Batch<FusedSource> bf{b->d_fused, b->d_fused_tiles, b->num_sources, b->fused_tiles};
+    Batch<FusedSource> bf{b->d_fused, b->d_fused_tiles, b->num_sources, b->fused_tiles,
+                          b->fused_min_start};
     tc.lti_fir = b->d_lti;
     if ((b->flags & FLR_FLAG_MIXED) && stock.generation != 0 && stock.equal_arm &&
         r->order == 25) {
@@ -1323,8 +1335,9 @@ int flr_batch_run(flr_batch *b, void *stream)
     if (st) return st;
     st = make_tdi_config(r, b->dt, b->fs, b->flags, tc, stock);
     if (st) return st;
-    Batch<ProjSource> bp{b->d_proj, b->d_proj_tiles, b->num_sources, b->proj_tiles};
-    Batch<TdiSource> bt{b->d_tdi, b->d_tdi_tiles, b->num_sources, b->tdi_tiles};
+    Batch<ProjSource> bp{b->d_proj, b->d_proj_tiles, b->num_sources, b->proj_tiles,
+                         b->proj_min_start};
+    Batch<TdiSource> bt{b->d_tdi, b->d_tdi_tiles, b->num_sources, b->tdi_tiles, b->tdi_min_start};
     hipError_t e = launch_projection_batch(pc, bp, r->orbits->view(), r->lagrange(), exact,
                                            r->orbits->equal_arm, b->grid_per_cu, s);
     if (e != hipSuccess) return hip_fail(e, "batch projection launch");
@@ -1552,9 +1565,11 @@ int flr_fused_run_static(flr_response *r, const flr_source *sources, int num_sou
     // validate every source before anything is enqueued
     const int zero_edges = (flags & FLR_FLAG_ZERO_EDGES) ? 1 : 0;
     int64_t tiles = 0;
+    int min_start = INT32_MAX;
     for (int q = 0; q < num_sources; ++q) {
         FusedSource f;
         if ((st = fused_source_record(sources[q], q, flags, h_all, out_all, f))) return st;
+        min_start = std::min(min_start, f.tdi_start);
         tiles += tiles_for(f.num_pts, f.tdi_start, zero_edges, tc.tile);
         if (tiles > INT32_MAX) return fail(FLR_ERR_UNSUPPORTED, "batch has too many tiles");
     }
@@ -1578,7 +1593,7 @@ int flr_fused_run_static(flr_response *r, const flr_source *sources, int num_sou
         hipLaunchKernelGGL(stage_sources_kernel, dim3(1), dim3(64), 0, s, chunk, d_src, d_prefix);
         FLR_HIP(hipGetLastError());
     }
-    Batch<FusedSource> bf{d_src, d_prefix, num_sources, prefix};
+    Batch<FusedSource> bf{d_src, d_prefix, num_sources, prefix, min_start};
     const LagrangeView lg = r->lagrange();
     const OrbitView orb = r->orbits->view();
     if (mixed) {

@@ -48,6 +48,30 @@ __device__ __forceinline__ double div_rcp(double a, double b, double y)
     return __builtin_fma(r, y, q);
 }
 
+// ------------------------------------------------------------------ exact quotients
+// A tap pair's two quotients, up / F + down / G, and what they need of F and G.
+template <int FORM>
+struct PairDiv {
+    double F, G, yF, yG;
+    __device__ __forceinline__ PairDiv(double F_, double G_)
+        : F(F_), G(G_), yF(rcp_nr2(F_)), yG(rcp_nr2(G_))
+    {
+    }
+    __device__ __forceinline__ double sum(double up, double down) const
+    {
+        return div_rcp(up, F, yF) + div_rcp(down, G, yG);
+    }
+};
+template <>
+struct PairDiv<kExact2> {
+    Recip rF, rG;
+    __device__ __forceinline__ PairDiv(double F, double G) { recip_pair(F, G, rF, rG); }
+    __device__ __forceinline__ double sum(double up, double down) const
+    {
+        return div_recip(up, rF) + div_recip(down, rG);
+    }
+};
+
 // ------------------------------------------------------------------ orbit interpolation
 // Uniform-grid linear interpolation of the orbit tables (the lisatools Orbits methods called
 // at LISAResponse.cu:331,565,570,576): window k = int(t/dt), clamped to [0, N-2], value
@@ -58,18 +82,20 @@ struct OrbitNode {
     double tau;       // t - dt*k
 };
 
-// EXACT: the window index from t / dt as the CPU path; otherwise from t * (1/dt), which can
-// pick the neighbouring window at a node -- the interpolant is continuous there.
-template <bool EXACT = true>
+// EXACT: the window index from t / dt as the CPU path (the quotient by the table's spacing from its
+// reciprocal, div_rcp: 3 operations instead of the full division's ~14 issue slots); otherwise from
+// t * (1/dt), which can pick the neighbouring window at a node -- the interpolant is continuous
+// there.
+template <int EXACT = kExact>
 __device__ __forceinline__ int orbit_window(const OrbitView &o, double t)
 {
-    double q = EXACT ? t / o.dt : t * o.inv_dt;
+    double q = EXACT ? div_rcp(t, o.dt, o.inv_dt) : t * o.inv_dt;
     if (!(q >= 0.0)) return 0;
     if (q >= (double)(o.N - 1)) return o.N - 2;
     return (int)q;
 }
 
-template <bool EXACT = true>
+template <int EXACT = kExact>
 __device__ __forceinline__ OrbitNode orbit_node(const OrbitView &o, double t)
 {
     const int w = orbit_window<EXACT>(o, t);
@@ -140,7 +166,7 @@ __device__ __forceinline__ double dot3(const double *a, const double *b)
 // The fast forms' link geometry (unit vector, projections): the same dot product with fused
 // multiply-adds (equal to the exact form up to rounding). Arrival times t - (k.x)/c keep the
 // exact form in both: at t ~ 1e7 s one rounding step of t moves the signal by ~1e-10 of itself.
-template <bool EXACT>
+template <int EXACT>
 __device__ __forceinline__ double dot3_form(const double *a, const double *b)
 {
     if constexpr (EXACT)
@@ -276,7 +302,7 @@ __device__ __forceinline__ double lagrange_weight(const LagrangeView &lg, double
 // and S = T/P with the running product P = prod Q_j and T_j = T_{j-1} Q_j + E_{j-1} n_j P_{j-1},
 // so one reciprocal per stencil replaces 2(h-1) divisions.
 
-template <int H>
+template <int FORM, int H>
 __device__ __forceinline__ double stencil_exact(const double *x, double e, const LagrangeView &lg,
                                                 double y_deps)
 {
@@ -294,7 +320,7 @@ __device__ __forceinline__ double stencil_exact(const double *x, double e, const
         double G = j + (1 - e);
         double up = x[1 + j];
         double down = x[-j];
-        sum += E * (div_rcp(up, F, rcp_nr2(F)) + div_rcp(down, G, rcp_nr2(G)));
+        sum += E * PairDiv<FORM>(F, G).sum(up, down);
     }
     return A * (B * x[1] + C * x[0] + D * sum);
 }
@@ -326,7 +352,7 @@ __device__ __forceinline__ double stencil_fast(const X &x, double e, const Lagra
 }
 
 // Complex: the h+ and hx sums share each denominator's reciprocal.
-template <int H>
+template <int FORM, int H>
 __device__ __forceinline__ double2 stencil_exact_c(const double2 *x, double e, const LagrangeView &lg,
                                                    double y_deps)
 {
@@ -342,12 +368,11 @@ __device__ __forceinline__ double2 stencil_exact_c(const double2 *x, double e, c
         double E = lg.E[j - 1];
         double F = j + e;
         double G = j + (1 - e);
-        double yF = rcp_nr2(F);
-        double yG = rcp_nr2(G);
+        const PairDiv<FORM> q(F, G);
         double2 up = x[1 + j];
         double2 down = x[-j];
-        sum_re += E * (div_rcp(up.x, F, yF) + div_rcp(down.x, G, yG));
-        sum_im += E * (div_rcp(up.y, F, yF) + div_rcp(down.y, G, yG));
+        sum_re += E * q.sum(up.x, down.x);
+        sum_im += E * q.sum(up.y, down.y);
     }
     double2 up = x[1];
     double2 down = x[0];
@@ -490,22 +515,22 @@ __device__ __forceinline__ double2 stencil_fold_c_lo(const double2 *lo, double e
     return out;
 }
 
-template <bool EXACT, int H>
+template <int EXACT, int H>
 __device__ __forceinline__ double stencil(const double *x, double e, const LagrangeView &lg,
                                           double y_deps)
 {
     if constexpr (EXACT)
-        return stencil_exact<H>(x, e, lg, y_deps);
+        return stencil_exact<EXACT, H>(x, e, lg, y_deps);
     else
         return stencil_fast<H>(x, e, lg);
 }
 
-template <bool EXACT, int H>
+template <int EXACT, int H>
 __device__ __forceinline__ double2 stencil_c(const double2 *x, double e, const LagrangeView &lg,
                                              double y_deps)
 {
     if constexpr (EXACT)
-        return stencil_exact_c<H>(x, e, lg, y_deps);
+        return stencil_exact_c<EXACT, H>(x, e, lg, y_deps);
     else
         return stencil_fast_c<H>(x, e, lg);
 }

@@ -162,7 +162,7 @@ __device__ __forceinline__ void fused_store(const TdiConfig &tc, const FusedSour
 
 // The composite filters' reference for source src: its first TDI sample
 // (t0 + tdi_start * dt) and the arm length there.
-template <int NX, bool EXACT>
+template <int NX, int EXACT>
 __device__ __forceinline__ double lti_source_reference(const TdiConfig &tc, const FusedSource &src,
                                                        const OrbitView &orb, const RowMap &rm,
                                                        LtiRef<NX> &lref)
@@ -383,7 +383,7 @@ __device__ __forceinline__ void utv_mfma(const TdiConfig &tc, const FusedSource 
 // cannot be cleared as a whole are compiled in. Without them (when the host has proved that
 // every tile clears, tc.lti_uniform) the kernel is smaller and its projection loop keeps its
 // operands in registers; a tile that fails anyway is reported (kErrLti) and written as NaN.
-template <bool EXACT, int MODE, int NX, typename HT, typename OT, int PASSES, int TPB = kBlock,
+template <int EXACT, int MODE, int NX, typename HT, typename OT, int PASSES, int TPB = kBlock,
           bool SAMPLE_PASS = true, bool STAGED = false>
 __device__ __forceinline__ void fused_tile(const ProjConfig &pc, const TdiConfig &tc,
                                            const FusedSource &src, int s, int tile,
@@ -584,7 +584,7 @@ __device__ __forceinline__ void fused_tile(const ProjConfig &pc, const TdiConfig
     if (bad) atomicOr(tc.err, kErrWindow);
 }
 
-template <bool EXACT, int MODE, int NX, typename HT, typename OT, int PASSES>
+template <int EXACT, int MODE, int NX, typename HT, typename OT, int PASSES>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
 void fused_batch_kernel(ProjConfig pc, TdiConfig tc,
                                                              Batch<FusedSource> batch,
@@ -779,7 +779,7 @@ void fused_utv_kernel(ProjConfig pc, TdiConfig tc, Batch<FusedSource> batch, Orb
 
 // Launch one fused variant over a batch: the TDI mode follows the table (stock + equal arms:
 // groups for exact stencils, linear merging for fast ones; otherwise unit by unit).
-template <bool EXACT, typename HT, typename OT, int PASSES>
+template <int EXACT, typename HT, typename OT, int PASSES>
 hipError_t launch_fused_variant(const ProjConfig &pc, const TdiConfig &tc, const Batch<FusedSource> &b,
                                 const OrbitView &orb, const LagrangeView &lg, const StockTdi &st,
                                 int grid_per_cu, hipStream_t stream)

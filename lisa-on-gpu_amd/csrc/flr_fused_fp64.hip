@@ -9,11 +9,12 @@ hipError_t launch_fused_fp64(const ProjConfig &pc, const TdiConfig &tc,
                              const LagrangeView &lg, bool exact, int grid_per_cu,
                              const StockTdi &st, hipStream_t stream)
 {
-    if (exact)
-        return launch_fused_variant<true, double2, double, 2>(pc, tc, b, orb, lg, st, grid_per_cu,
-                                                              stream);
-    return launch_fused_variant<false, double2, double, 2>(pc, tc, b, orb, lg, st, grid_per_cu,
-                                                           stream);
+    // the projection's windows reach lowest: the TDI window's start less the projection's halo
+    const int64_t lowest = (int64_t)b.min_start - tc.halo_lo - pc.halo_lo;
+    return by_form(stencil_form(exact, lowest, lg.h), [&](auto form) {
+        return launch_fused_variant<decltype(form)::value, double2, double, 2>(
+            pc, tc, b, orb, lg, st, grid_per_cu, stream);
+    });
 }
 
 }  // namespace flr

@@ -5,6 +5,7 @@
 #include <cstdint>
 
 #include "../../include/flr.h"
+#include "flr_quotient.hpp"
 
 namespace flr {
 
@@ -19,6 +20,22 @@ constexpr int kBlock = 256;       // threads per workgroup (4 wave64) = samples 
 // followed by their 15 slopes (v[k+1] - v[k]) / dt, so that one node's data sits in 240 B.
 constexpr int kOrbitVals = 15;
 constexpr int kOrbitStride = 2 * kOrbitVals;
+
+// Stencil forms (flr_device.hpp). kFast: no per-tap divisions. kExact: the reference's operation
+// sequence, each quotient in three operations from its denominator's reciprocal. kExact2: the same
+// quotients, bit for bit, in two (div_recip) -- for stencils at sample positions of at least
+// exact2_min_position(h).
+constexpr int kFast = 0;
+constexpr int kExact = 1;
+constexpr int kExact2 = 2;
+
+// The form of a launch whose staged windows start at sample `lowest` or later: every stencil that
+// passes its window test sits at least h - 1 samples above its window's start.
+inline int stencil_form(bool exact, int64_t lowest, int h)
+{
+    if (!exact) return kFast;
+    return lowest + h - 1 >= exact2_min_position(h) ? kExact2 : kExact;
+}
 
 // Device error word bits.
 constexpr int kErrWindow = 1;     // stencil outside the staged window (or the input array)
@@ -143,6 +160,7 @@ struct Batch {
     const int *tile_start;
     int num_sources;
     int total_tiles;
+    int min_start = 0;  // the smallest first computed sample of the sources (stencil_form)
 };
 
 // Tiles a source needs: one per `tile` samples of [start, n - start), or of [0, n) when the

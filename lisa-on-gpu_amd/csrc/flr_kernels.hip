@@ -25,7 +25,7 @@ namespace flr {
 
 // ------------------------------------------------------------------ projection
 
-template <bool EXACT, int H, bool EQ>
+template <int EXACT, int H, bool EQ>
 __device__ __forceinline__ void projection_tile(const ProjConfig &cfg, const ProjSource &src,
                                                 int tile, const OrbitView &orb,
                                                 const LagrangeView &lg, double2 *hwin)
@@ -114,7 +114,7 @@ __device__ __forceinline__ bool tdi_stage(const TdiConfig &cfg, const TdiSource 
     return true;
 }
 
-template <bool EXACT, int H>
+template <int EXACT, int H>
 __device__ __forceinline__ void tdi_tile(const TdiConfig &cfg, const TdiSource &src, int tile,
                                          const OrbitView &orb, const LagrangeView &lg,
                                          double *smem)
@@ -158,7 +158,7 @@ __device__ __forceinline__ void tdi_tile(const TdiConfig &cfg, const TdiSource &
 // (fast form) are shared by the units of that length -- 8 groups instead of 48 units for 2nd
 // generation, with bit-identical results.
 
-template <int NX, bool EXACT, bool EQ>
+template <int NX, int EXACT, bool EQ>
 __device__ __forceinline__ void tdi_stock_tile(const TdiConfig &cfg, const TdiSource &src,
                                                int tile, const OrbitView &orb,
                                                const LagrangeView &lg, const RowMap &rm,
@@ -201,7 +201,7 @@ __device__ __forceinline__ void tdi_stock_tile(const TdiConfig &cfg, const TdiSo
 
 // ------------------------------------------------------------------ kernels
 
-template <bool EXACT, int H, bool EQ>
+template <int EXACT, int H, bool EQ>
 __global__ __launch_bounds__(kBlock) void projection_kernel(ProjConfig cfg, ProjSource src,
                                                             OrbitView orb, LagrangeView lg)
 {
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kBlock) void projection_kernel(ProjConfig cfg, Proj
     projection_tile<EXACT, H, EQ>(cfg, src, blockIdx.x, orb, lg, hwin);
 }
 
-template <bool EXACT, int H, bool EQ>
+template <int EXACT, int H, bool EQ>
 __global__ __launch_bounds__(kBlock) void projection_batch_kernel(ProjConfig cfg,
                                                                   Batch<ProjSource> batch,
                                                                   OrbitView orb, LagrangeView lg)
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(kBlock) void projection_batch_kernel(ProjConfig cfg
     FLR_BATCH_LOOP(batch, (projection_tile<EXACT, H, EQ>(cfg, src, tile, orb, lg, hwin)));
 }
 
-template <bool EXACT, int H>
+template <int EXACT, int H>
 __global__ __launch_bounds__(kBlock) void tdi_kernel(TdiConfig cfg, TdiSource src, OrbitView orb,
                                                      LagrangeView lg)
 {
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(kBlock) void tdi_kernel(TdiConfig cfg, TdiSource sr
     tdi_tile<EXACT, H>(cfg, src, blockIdx.x, orb, lg, smem);
 }
 
-template <bool EXACT, int H>
+template <int EXACT, int H>
 __global__ __launch_bounds__(kBlock) void tdi_batch_kernel(TdiConfig cfg, Batch<TdiSource> batch,
                                                            OrbitView orb, LagrangeView lg)
 {
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kBlock) void tdi_batch_kernel(TdiConfig cfg, Batch<
     FLR_BATCH_LOOP(batch, (tdi_tile<EXACT, H>(cfg, src, tile, orb, lg, smem)));
 }
 
-template <int NX, bool EXACT, bool EQ>
+template <int NX, int EXACT, bool EQ>
 __global__ __launch_bounds__(kBlock) void tdi_stock_kernel(TdiConfig cfg, TdiSource src,
                                                                OrbitView orb, LagrangeView lg,
                                                                RowMap rm)
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void tdi_stock_kernel(TdiConfig cfg, TdiSou
     tdi_stock_tile<NX, EXACT, EQ>(cfg, src, blockIdx.x, orb, lg, rm, smem);
 }
 
-template <int NX, bool EXACT, bool EQ>
+template <int NX, int EXACT, bool EQ>
 __global__ __launch_bounds__(kBlock) void tdi_stock_batch_kernel(TdiConfig cfg,
                                                                      Batch<TdiSource> batch,
                                                                      OrbitView orb,
@@ -298,14 +298,14 @@ hipError_t launch_projection(const ProjConfig &cfg, const ProjSource &src, const
 {
     const int nb = tiles_for(src.num_delays, src.start, cfg.zero_edges);
     const size_t shm = proj_lds(cfg);
-    if (lg.h == 13 && equal_arm)
-        return exact ? launch(projection_kernel<true, 13, true>, nb, shm, stream, cfg, src, orb, lg)
-                     : launch(projection_kernel<false, 13, true>, nb, shm, stream, cfg, src, orb, lg);
-    if (lg.h == 13)
-        return exact ? launch(projection_kernel<true, 13, false>, nb, shm, stream, cfg, src, orb, lg)
-                     : launch(projection_kernel<false, 13, false>, nb, shm, stream, cfg, src, orb, lg);
-    return exact ? launch(projection_kernel<true, 0, false>, nb, shm, stream, cfg, src, orb, lg)
-                 : launch(projection_kernel<false, 0, false>, nb, shm, stream, cfg, src, orb, lg);
+    return by_form(stencil_form(exact, (int64_t)src.start - cfg.halo_lo, lg.h), [&](auto form) {
+        constexpr int F = decltype(form)::value;
+        if (lg.h == 13 && equal_arm)
+            return launch(projection_kernel<F, 13, true>, nb, shm, stream, cfg, src, orb, lg);
+        if (lg.h == 13)
+            return launch(projection_kernel<F, 13, false>, nb, shm, stream, cfg, src, orb, lg);
+        return launch(projection_kernel<F, 0, false>, nb, shm, stream, cfg, src, orb, lg);
+    });
 }
 
 hipError_t launch_projection_batch(const ProjConfig &cfg, const Batch<ProjSource> &b,
@@ -314,14 +314,14 @@ hipError_t launch_projection_batch(const ProjConfig &cfg, const Batch<ProjSource
 {
     const int nb = batch_grid(b.total_tiles, grid_per_cu);
     const size_t shm = proj_lds(cfg);
-    if (lg.h == 13 && equal_arm)
-        return exact ? launch(projection_batch_kernel<true, 13, true>, nb, shm, stream, cfg, b, orb, lg)
-                     : launch(projection_batch_kernel<false, 13, true>, nb, shm, stream, cfg, b, orb, lg);
-    if (lg.h == 13)
-        return exact ? launch(projection_batch_kernel<true, 13, false>, nb, shm, stream, cfg, b, orb, lg)
-                     : launch(projection_batch_kernel<false, 13, false>, nb, shm, stream, cfg, b, orb, lg);
-    return exact ? launch(projection_batch_kernel<true, 0, false>, nb, shm, stream, cfg, b, orb, lg)
-                 : launch(projection_batch_kernel<false, 0, false>, nb, shm, stream, cfg, b, orb, lg);
+    return by_form(stencil_form(exact, (int64_t)b.min_start - cfg.halo_lo, lg.h), [&](auto form) {
+        constexpr int F = decltype(form)::value;
+        if (lg.h == 13 && equal_arm)
+            return launch(projection_batch_kernel<F, 13, true>, nb, shm, stream, cfg, b, orb, lg);
+        if (lg.h == 13)
+            return launch(projection_batch_kernel<F, 13, false>, nb, shm, stream, cfg, b, orb, lg);
+        return launch(projection_batch_kernel<F, 0, false>, nb, shm, stream, cfg, b, orb, lg);
+    });
 }
 
 // The stock kernels keep the light travel times in registers; the generic one in LDS.
@@ -334,22 +334,21 @@ hipError_t launch_tdi(const TdiConfig &cfg, const TdiSource &src, const OrbitVie
                       const LagrangeView &lg, bool exact, const StockTdi &st, hipStream_t stream)
 {
     const int nb = tiles_for(src.num_delays, src.start, cfg.zero_edges);
-    if (use_stock(st, lg)) {
-        const size_t shm = tdi_lds(cfg, true);
-        const RowMap &rm = st.rows;
-#define FLR_STOCK(NX, EQ)                                                                   \
-    (exact ? launch(tdi_stock_kernel<NX, true, EQ>, nb, shm, stream, cfg, src, orb, lg, rm) \
-           : launch(tdi_stock_kernel<NX, false, EQ>, nb, shm, stream, cfg, src, orb, lg, rm))
-        if (st.equal_arm) return st.generation == 1 ? FLR_STOCK(8, true) : FLR_STOCK(16, true);
-        return st.generation == 1 ? FLR_STOCK(8, false) : FLR_STOCK(16, false);
+    const RowMap &rm = st.rows;
+    return by_form(stencil_form(exact, (int64_t)src.start - cfg.halo_lo, lg.h), [&](auto form) {
+        constexpr int F = decltype(form)::value;
+        if (use_stock(st, lg)) {
+            const size_t shm = tdi_lds(cfg, true);
+#define FLR_STOCK(NX, EQ) \
+    launch(tdi_stock_kernel<NX, F, EQ>, nb, shm, stream, cfg, src, orb, lg, rm)
+            if (st.equal_arm) return st.generation == 1 ? FLR_STOCK(8, true) : FLR_STOCK(16, true);
+            return st.generation == 1 ? FLR_STOCK(8, false) : FLR_STOCK(16, false);
 #undef FLR_STOCK
-    }
-    const size_t shm = tdi_lds(cfg, false);
-    if (lg.h == 13)
-        return exact ? launch(tdi_kernel<true, 13>, nb, shm, stream, cfg, src, orb, lg)
-                     : launch(tdi_kernel<false, 13>, nb, shm, stream, cfg, src, orb, lg);
-    return exact ? launch(tdi_kernel<true, 0>, nb, shm, stream, cfg, src, orb, lg)
-                 : launch(tdi_kernel<false, 0>, nb, shm, stream, cfg, src, orb, lg);
+        }
+        const size_t shm = tdi_lds(cfg, false);
+        if (lg.h == 13) return launch(tdi_kernel<F, 13>, nb, shm, stream, cfg, src, orb, lg);
+        return launch(tdi_kernel<F, 0>, nb, shm, stream, cfg, src, orb, lg);
+    });
 }
 
 hipError_t launch_tdi_batch(const TdiConfig &cfg, const Batch<TdiSource> &b, const OrbitView &orb,
@@ -357,22 +356,21 @@ hipError_t launch_tdi_batch(const TdiConfig &cfg, const Batch<TdiSource> &b, con
                             int grid_per_cu, hipStream_t stream)
 {
     const int nb = batch_grid(b.total_tiles, grid_per_cu);
-    if (use_stock(st, lg)) {
-        const size_t shm = tdi_lds(cfg, true);
-        const RowMap &rm = st.rows;
-#define FLR_STOCK(NX, EQ)                                                                        \
-    (exact ? launch(tdi_stock_batch_kernel<NX, true, EQ>, nb, shm, stream, cfg, b, orb, lg, rm)  \
-           : launch(tdi_stock_batch_kernel<NX, false, EQ>, nb, shm, stream, cfg, b, orb, lg, rm))
-        if (st.equal_arm) return st.generation == 1 ? FLR_STOCK(8, true) : FLR_STOCK(16, true);
-        return st.generation == 1 ? FLR_STOCK(8, false) : FLR_STOCK(16, false);
+    const RowMap &rm = st.rows;
+    return by_form(stencil_form(exact, (int64_t)b.min_start - cfg.halo_lo, lg.h), [&](auto form) {
+        constexpr int F = decltype(form)::value;
+        if (use_stock(st, lg)) {
+            const size_t shm = tdi_lds(cfg, true);
+#define FLR_STOCK(NX, EQ) \
+    launch(tdi_stock_batch_kernel<NX, F, EQ>, nb, shm, stream, cfg, b, orb, lg, rm)
+            if (st.equal_arm) return st.generation == 1 ? FLR_STOCK(8, true) : FLR_STOCK(16, true);
+            return st.generation == 1 ? FLR_STOCK(8, false) : FLR_STOCK(16, false);
 #undef FLR_STOCK
-    }
-    const size_t shm = tdi_lds(cfg, false);
-    if (lg.h == 13)
-        return exact ? launch(tdi_batch_kernel<true, 13>, nb, shm, stream, cfg, b, orb, lg)
-                     : launch(tdi_batch_kernel<false, 13>, nb, shm, stream, cfg, b, orb, lg);
-    return exact ? launch(tdi_batch_kernel<true, 0>, nb, shm, stream, cfg, b, orb, lg)
-                 : launch(tdi_batch_kernel<false, 0>, nb, shm, stream, cfg, b, orb, lg);
+        }
+        const size_t shm = tdi_lds(cfg, false);
+        if (lg.h == 13) return launch(tdi_batch_kernel<F, 13>, nb, shm, stream, cfg, b, orb, lg);
+        return launch(tdi_batch_kernel<F, 0>, nb, shm, stream, cfg, b, orb, lg);
+    });
 }
 
 hipError_t launch_orbit_eval(const OrbitView &orb, const double *t, int n, int row, int sc,

@@ -38,7 +38,7 @@ __device__ __forceinline__ TileRange tile_range(int tile, int num_delays, int st
 // folded stencil and one-Newton-step reciprocals of the float32-output forms. STAGED (fast
 // forms): orbit nodes from the tile's LDS stage `ost` (orbit_node_staged; a lookup outside it
 // makes the sample's links NaN and returns true).
-template <bool EXACT, int H, bool EQ, bool CANON = false, int ESRC = kEArg, bool STAGED = false,
+template <int EXACT, int H, bool EQ, bool CANON = false, int ESRC = kEArg, bool STAGED = false,
           typename Store>
 __device__ __forceinline__ bool project_links(const ProjConfig &cfg, const double (&k)[3],
                                               const double (&u)[3], const double (&v)[3],
@@ -152,8 +152,9 @@ __device__ __forceinline__ bool project_links(const ProjConfig &cfg, const doubl
             }
             if constexpr (EXACT) {
                 norm = sqrt(norm);
+                const double y_norm = rcp_nr2(norm);  // one reciprocal for the three quotients
 #pragma unroll
-                for (int c = 0; c < 3; ++c) n[c] = n[c] / norm;
+                for (int c = 0; c < 3; ++c) n[c] = div_rcp(n[c], norm, y_norm);
             } else {  // one reciprocal square root instead of a root and three divisions
                 const double inv = ESRC == kELdsFold ? rsqrt_pos1(norm) : rsqrt_pos(norm);
 #pragma unroll
@@ -186,7 +187,7 @@ __device__ __forceinline__ bool project_links(const ProjConfig &cfg, const doubl
 // Every unit of every channel at time t, summed per channel in index order into acc. Ls[r *
 // ls_stride] is the light travel time of table row r at t; row r of the y window starts at
 // ywin + r * cap. Returns true if a stencil fell outside the window (its channel gets NaN).
-template <bool EXACT, int H>
+template <int EXACT, int H>
 __device__ __forceinline__ bool tdi_units(const TdiConfig &cfg, double t, double t0_offset,
                                           const double *Ls, int ls_stride, const double *ywin,
                                           int cap, int win_lo, int win_len, const LagrangeView &lg,
@@ -282,6 +283,17 @@ inline hipError_t set_lds_limit(Kernel k, size_t bytes)
 {
     if (bytes <= 64 * 1024) return hipSuccess;
     return hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+// f(std::integral_constant<int, form>): the kernels are compiled per stencil form.
+template <typename F>
+inline hipError_t by_form(int form, F &&f)
+{
+    switch (form) {
+    case kFast: return f(std::integral_constant<int, kFast>{});
+    case kExact: return f(std::integral_constant<int, kExact>{});
+    default: return f(std::integral_constant<int, kExact2>{});
+    }
 }
 
 // Persistent batch grid: grid_per_cu workgroups per CU (enough to fill every CU a few times

@@ -1,0 +1,58 @@
+// flr_quotient.hpp -- the exact stencils' quotients in two operations each.
+//
+// Written for host and device: the host build (the bit-for-bit test against a / b) defines
+// FLR_HOST_DEVICE empty and FLR_RCP_SEED as an approximate reciprocal.
+#pragma once
+
+#ifndef FLR_HOST_DEVICE
+#define FLR_HOST_DEVICE __host__ __device__
+#endif
+#ifndef FLR_RCP_SEED
+#define FLR_RCP_SEED(x) __builtin_amdgcn_rcp(x)
+#endif
+
+namespace flr {
+
+// The smallest sample position from which div_recip is proven for half point count h.
+constexpr int exact2_min_position(int h) { return h <= 16 ? 256 : 512; }
+
+// The reciprocal of b as an unevaluated sum: 1/b = y + l up to ~2^-103 of itself.
+struct Recip {
+    double y, l;
+};
+
+// a / b, correctly rounded, as y a + l a rounded once, from b's two-part reciprocal. Why the bits
+// are those of a / b for the stencils' denominators, b = j + e or j + 1 - e, at most h (u = 2^-53): at a
+// position cf >= 2^c (in samples) the fraction e is a multiple of ulp(cf) >= 2^(c-52); so are j + e and
+// j + (1 - e), which are exact, and b = B 2^(c-52) with B <= h 2^(52-c). The quotient of such a b and a
+// 53-bit a is never a midpoint M of two doubles (M < 2^54 odd), and is at least 1 / (B M) >
+// 2^(c-106) / h of itself away from each. recip_pair's y is off by at most e1 = 3 u (the roundings of
+// F G, of its reciprocal and of the product by the other factor), 1 - b y = e1 comes out exactly, and
+// l = e1 y leaves e1^2 = 9 u^2 and its own rounding, 3 u^2; the product l a adds 3 u^2. Together
+// 15 u^2 = 15 2^-106, below that distance when h <= 2^c / 15: c = 8 for h <= 16, 9 up to
+// kMaxHalf (exact2_min_position). Two operations per quotient instead of div_rcp's three, and one
+// v_rcp_f64 (4 issue slots) per tap pair instead of two: 58 issue slots instead of 72 per tap pair of
+// six units with one fraction, 30 instead of 36 of a complex stencil, 23 instead of 27 of one unit.
+// The exact forms are bound by these FP64 operations: 1-yr FP64 drop-in (3,153,600 samples) 1.125 ->
+// 0.961 ms with equal arms, 2.002 -> 1.769 ms with unequal ones, order 31 with a custom table
+// (262,145 samples) 0.135 -> 0.119 ms (interleaved A/B on one box).
+FLR_HOST_DEVICE inline double div_recip(double a, const Recip &r)
+{
+    return __builtin_fma(a, r.y, a * r.l);
+}
+
+// The two denominators of a tap pair, F = j + e and G = j + (1 - e): one hardware reciprocal of
+// their product (relative error below 2^-22), refined to third order, gives both.
+FLR_HOST_DEVICE inline void recip_pair(double F, double G, Recip &rF, Recip &rG)
+{
+    const double p = F * G;
+    double r = FLR_RCP_SEED(p);
+    const double e = __builtin_fma(-p, r, 1.0);
+    r = __builtin_fma(r, __builtin_fma(e, e, e), r);
+    rF.y = G * r;
+    rG.y = F * r;
+    rF.l = __builtin_fma(-F, rF.y, 1.0) * rF.y;
+    rG.l = __builtin_fma(-G, rG.y, 1.0) * rG.y;
+}
+
+}  // namespace flr

@@ -127,7 +127,7 @@ constexpr int done_prefix(int nx, int m)
 // reciprocals (exact form) or Lagrange weights (fast form). Per unit the tap sum runs over j
 // in the reference's order, and units are added to their channel sum in index order.
 // Returns false if a stencil fell outside the window (the affected outputs are NaN).
-template <int NX, bool EXACT>
+template <int NX, int EXACT>
 __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offset, double fs,
                                               const double *ywin, const int (&rowoff)[6],
                                               int win_lo, int win_len, const LagrangeView &lg,
@@ -170,16 +170,12 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
         for (int j = 1; j < H; ++j) {
             const double E = lg.E[j - 1];
             if constexpr (EXACT) {
-                const double F = j + e;
-                const double G = j + (1 - e);
-                const double yF = rcp_nr2(F);
-                const double yG = rcp_nr2(G);
+                const PairDiv<EXACT> q(j + e, j + (1 - e));
 #pragma unroll
                 for (int c = 0; c < 3; ++c)
 #pragma unroll
                     for (int k = 0; k < 2; ++k)
-                        S[c][k] += E * (div_rcp(xr[c][k][H + j], F, yF) +
-                                        div_rcp(xr[c][k][H - 1 - j], G, yG));
+                        S[c][k] += E * q.sum(xr[c][k][H + j], xr[c][k][H - 1 - j]);
             } else {
                 const double qu = (double)j + e;
                 const double qd = (double)(j + 1) - e;
@@ -250,7 +246,7 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
 // chain order -- the generic tdi_units' operation sequence unit by unit, hence bitwise equal to
 // it -- and every unit's stencil is addressed from its lowest tap. Units are added to their
 // channel in index order. Returns false if a stencil fell outside the window.
-template <int NX, bool EXACT>
+template <int NX, int EXACT>
 __device__ __forceinline__ bool tdi_stock_unequal(double t, const double (&L)[6], double t0_offset,
                                                   double fs, const double *ywin,
                                                   const int (&rowoff)[6], int win_lo, int win_len,
