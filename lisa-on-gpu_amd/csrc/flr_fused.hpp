@@ -18,8 +18,8 @@ namespace flr {
 //
 // TDI modes: kModeGeneric -- any table, unit by unit (tdi_units); kModeStock -- stock table,
 // unequal arms, compile-time chains (tdi_stock_unequal); kModeGroups -- stock table
-// with equal arms, shared delays per chain length (tdi_equal_arm, exact or fast); kModeLinear --
-// the same, fast, with each group's units merged into one stencil per output (tdi_linear; the
+// with equal arms, shared delays per chain length (tdi_equal_arm, exact); kModeLinear --
+// the fast form, with each group's units merged into one stencil per output (tdi_linear; the
 // window columns are replaced by the combined series right after projection).
 constexpr int kModeGeneric = 0;
 constexpr int kModeGroups = 1;

@@ -124,8 +124,8 @@ constexpr int done_prefix(int nx, int m)
 // Equal-arm TDI for one sample: all six light travel times are bitwise equal, so every chain
 // of m links yields the same delay t - L - ... - L; each distinct delay is split once and the
 // units of that chain length (2 per channel) share one fraction, i.e. one set of per-tap
-// reciprocals (exact form) or Lagrange weights (fast form). Per unit the tap sum runs over j
-// in the reference's order, and units are added to their channel sum in index order.
+// reciprocals. Per unit the tap sum runs over j in the reference's order, and units are added to
+// their channel sum in index order (exact forms; the fast form is tdi_linear).
 // Returns false if a stencil fell outside the window (the affected outputs are NaN).
 template <int NX, int EXACT>
 __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offset, double fs,
@@ -133,6 +133,7 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
                                               int win_lo, int win_len, const LagrangeView &lg,
                                               double y_deps, double (&acc)[3])
 {
+    static_assert(EXACT != kFast, "the fast form merges the units of a chain length (tdi_linear)");
     constexpr int H = 13;
     constexpr int NG = stock::max_len(NX) + 1;
     bool ok = true;
@@ -162,35 +163,18 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
             });
         });
         double S[3][2] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
-        double P = 1.0;
         // j fully unrolled: every tap address is the unit's base plus an immediate offset (the
         // up/down pair of a unit loads with one ds_read2_b64); the memory barrier and the pins
         // at the end of each j keep its loads and arithmetic together.
 #pragma unroll
         for (int j = 1; j < H; ++j) {
             const double E = lg.E[j - 1];
-            if constexpr (EXACT) {
-                const PairDiv<EXACT> q(j + e, j + (1 - e));
+            const PairDiv<EXACT> q(j + e, j + (1 - e));
 #pragma unroll
-                for (int c = 0; c < 3; ++c)
+            for (int c = 0; c < 3; ++c)
 #pragma unroll
-                    for (int k = 0; k < 2; ++k)
-                        S[c][k] += E * q.sum(xr[c][k][H + j], xr[c][k][H - 1 - j]);
-            } else {
-                const double qu = (double)j + e;
-                const double qd = (double)(j + 1) - e;
-                const double Q = (double)(j * (j + 1)) + e * (1.0 - e);
-                const double EP = E * P;
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-#pragma unroll
-                    for (int k = 0; k < 2; ++k) {
-                        const double num = __builtin_fma(xr[c][k][H + j], qd, xr[c][k][H - 1 - j] * qu);
-                        S[c][k] = __builtin_fma(S[c][k], Q, num * EP);
-                    }
-                P = P * Q;
-                pin(P);
-            }
+                for (int k = 0; k < 2; ++k)
+                    S[c][k] += E * q.sum(xr[c][k][H + j], xr[c][k][H - 1 - j]);
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 pin(S[c][0]);
@@ -198,29 +182,16 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
             }
             __asm__ volatile("" ::: "memory");
         }
-        double A, B, C, D, invP = 0.0;
-        if constexpr (EXACT) {
-            A = lagrange_A_exact(lg, e, y_deps);
-            B = 1.0 - e;
-            C = e;
-            D = e * (1.0 - e);
-        } else {
-            A = lagrange_A_fast(lg, e);
-            B = 1.0 - e;
-            C = e;
-            D = e * B;
-            invP = 1.0 / P;
-        }
+        const double A = lagrange_A_exact(lg, e, y_deps);
+        const double B = 1.0 - e;
+        const double C = e;
+        const double D = e * (1.0 - e);
         static_for<3>([&](auto c) {
             int k = 0;
             static_for<NX>([&](auto x) {
                 if constexpr (stock::kX[x].len == m) {
                     const double *p = xr[c][k] + (H - 1);  // p[0] = x[d], p[1] = x[d+1]
-                    double val;
-                    if constexpr (EXACT)
-                        val = A * (B * p[1] + C * p[0] + D * S[c][k]);
-                    else
-                        val = A * __builtin_fma(D, S[c][k] * invP, __builtin_fma(B, p[1], C * p[0]));
+                    double val = A * (B * p[1] + C * p[0] + D * S[c][k]);
                     val *= (double)stock::kX[x].sign;
                     v[c][x] = gbad ? __builtin_nan("") : val;
                     pin(v[c][x]);
@@ -286,6 +257,16 @@ constexpr double kInvSqrt2 = 0.70710678118654752440084436210484903928;
 constexpr double kInvSqrt6 = 0.40824829046386301636621401245098189866;
 constexpr double kInvSqrt3 = 0.57735026918962576450914878050195745565;
 
+// The combined series of the six links y (canonical order): k[0][c] = y13 - y12, k[1][c] = y31 - y21,
+// cyclically shifted for channel c.
+__device__ __forceinline__ void combine_links(const double (&y)[6], double (&k)[2][3])
+{
+    static_for<3>([&](auto c) {
+        k[0][c] = y[stock::canon(stock::cyc(13, c))] - y[stock::canon(stock::cyc(12, c))];
+        k[1][c] = y[stock::canon(stock::cyc(31, c))] - y[stock::canon(stock::cyc(21, c))];
+    });
+}
+
 // Column of the combined series (in place of the six y rows, same stride `cap`): row
 // 2*o + kind holds output o's combination of kind `kind` -- X, Y, Z themselves, or A, E, T
 // formed from them when aet is set. yc points at the column; rm maps canonical links to rows
@@ -297,10 +278,7 @@ __device__ __forceinline__ void linear_series(double *yc, int cap, const RowMap 
 #pragma unroll
     for (int k = 0; k < 6; ++k) y[k] = yc[(CANON ? k : rm.row[k]) * cap];
     double kd[2][3];
-    static_for<3>([&](auto c) {
-        kd[0][c] = y[stock::canon(stock::cyc(13, c))] - y[stock::canon(stock::cyc(12, c))];
-        kd[1][c] = y[stock::canon(stock::cyc(31, c))] - y[stock::canon(stock::cyc(21, c))];
-    });
+    combine_links(y, kd);
 #pragma unroll
     for (int kind = 0; kind < 2; ++kind) {
         const double X = kd[kind][0], Y = kd[kind][1], Z = kd[kind][2];
