@@ -537,7 +537,7 @@ __device__ __forceinline__ bool lti_matches(double t, int i, double L, double t0
 // position error (at most kLtiTol, tested per unit on the tile's two ends and middle), the
 // second-order term (|sigma| (b - a) / 2 <= kUtvDrift keeps it
 // below 1e-9 of the interpolated value) and a change of the A table's slope inside the tile's
-// range of e (tolerated up to kUtvKnot past a node of the table). A tile that fails any test
+// range of e (tolerated up to an error of kUtvKnot times that change). A tile that fails any test
 // takes the per-sample stencils instead.
 constexpr double kUtvDrift = 1e-4;
 constexpr double kUtvKnot = 3e-8;
@@ -673,25 +673,45 @@ __device__ __forceinline__ void utv_unit(UtvShared &sh, int u, int chain, int a,
     const double sigma = b > a ? (pos[2] - pos[0]) / (double)(b - a) : 0.0;
     // (1) the line through the middle position with the chord's slope is off the positions at
     // a and b by dev, and off any position in between by at most 3 dev (the positions are
-    // piecewise linear in i between the orbit nodes)
-    const double dev = fabs(pos[0] + sigma * (double)(m - a) - pos[1]);
+    // piecewise linear in i between the orbit nodes); the model takes the line half way between it
+    // and the chord, whose mean error over the tile is about zero: the rms error of a kink anywhere in
+    // the tile drops to 0.75 of the line's through the middle (null channel T against
+    // extended-precision delays, kinks of 1.5e-12 s/s: 9.9e-8 -> 7.6e-8 at the 512-sample window)
+    const double off_chord = pos[0] + sigma * (double)(m - a) - pos[1];
+    const double dev = fabs(off_chord);
     bool ok = 3.0 * dev <= kLtiTol;
+    e_m -= 0.5 * off_chord;
     // (2) drift across the tile
     const double drift = fabs(sigma) * (double)max(m - a, b - m);
     ok = ok && drift <= kUtvDrift;
-    // (3) e over the tile, [e_m - drift, e_m + drift], within the A-table segment of e_m
-    const double s_m = e_m * lg.inv_deps;
+    // (3) e over the tile, [e_m - drift, e_m + drift], within the A-table segment of e_m, or past one of
+    // its nodes by `over`: then A's chord over that range, moved half way to A(e_m), is off A by at most
+    // (3/4 - over / (2 drift)) over <= 0.28 drift times the change of slope at the node. (At the ends of
+    // [0, 1] the stencil itself moves by a sample: there `over` counts in full.) On the cartwheel no
+    // tile of 1024 samples fails any more; before, about 1 in 150 did, and one tile's per-sample
+    // path takes ~100 us (2nd generation, dt = 5 s, 1024-sample window: 262,144 samples 161 -> 77 us,
+    // 2,000,000 375 -> 297 us)
+    const double s_m = e_m * lg.inv_deps, s_d = drift * lg.inv_deps;
     const int ind = min(max((int)s_m, 0), lg.num_A - 2);
-    const double over = fmax(fmax((double)ind - (s_m - drift * lg.inv_deps),
-                                  (s_m + drift * lg.inv_deps) - (double)(ind + 1)),
+    const double over = fmax(fmax((double)ind - (s_m - s_d), (s_m + s_d) - (double)(ind + 1)),
                              0.0) / lg.inv_deps;
-    ok = ok && over <= kUtvKnot;
+    const double2 as = lg.Aslope[ind];  // A as lagrange_A_fast interpolates it, and its slope
+    double A_m = __builtin_fma(as.y, s_m - (double)ind, as.x), dA_m = as.y * lg.inv_deps;
+    if (over > 0.0) {
+        if (s_m - s_d < 0.0 || s_m + s_d > (double)(lg.num_A - 1)) {
+            ok = ok && over <= kUtvKnot;
+        } else {
+            const double lo = lagrange_A_fast(lg, e_m - drift), hi = lagrange_A_fast(lg, e_m + drift);
+            ok = ok && over * (0.75 - over / (2.0 * drift)) <= kUtvKnot;
+            A_m = 0.5 * A_m + 0.25 * (lo + hi);
+            dA_m = (hi - lo) / (2.0 * drift);
+        }
+    }
     sh.off[u] = (double)off_m;
     sh.e[u] = e_m;
     sh.sigma[u] = sigma;
-    const double2 as = lg.Aslope[ind];  // A as lagrange_A_fast interpolates it, and its slope
-    sh.A[u] = __builtin_fma(as.y, s_m - (double)ind, as.x);
-    sh.dA[u] = as.y * lg.inv_deps;
+    sh.A[u] = A_m;
+    sh.dA[u] = dA_m;
     atomicMin(&sh.kmin, off_m - (H - 1));
     atomicMax(&sh.kmax, off_m + H);
     if (!ok) sh.ok = 0;
