@@ -166,6 +166,8 @@ struct flr_batch {
     int fused_tiles = 0;
     int capacity = 0;             // fused: sources the tables hold
     int tile_passes = kFusedPasses;  // fused: the tile's window is tile_passes * kBlock samples
+    bool auto_shape = true;          // ... chosen by auto_passes until flr_batch_set_launch sets it
+    uint64_t shape_version = ~0ull;  // response version auto_passes chose it for
     int tile_len = 0;                // fused: output samples per tile (make_fused_config)
     int grid_per_cu = 32;            // persistent workgroups per CU (the autotuner's usual pick)
     FusedSource *h_fused = nullptr;  // pinned staging of the source table and tile prefix
@@ -447,6 +449,14 @@ bool orbit_stage_fits(const flr_orbits *o, int win_cap, double dt)
 // ~ the tile's range of e over the table spacing) -- is below one half. Otherwise the per-sample
 // kernel runs, which is faster than the filter form's per-sample path on its block-interleaved
 // rows. Only the speed depends on this choice.
+double utv_crossings(const flr_orbits *o, int nx, int tile, double dt, double fs, double deps)
+{
+    const int M = nx == 8 ? 3 : 7;  // longest chain
+    const double drift = M * o->max_rate * dt * fs * 0.5 * tile;
+    const double p = std::min(1.0, 2.0 * drift / deps);  // per unit
+    return 1.0 - std::pow(1.0 - p, 3.0 * nx);
+}
+
 bool utv_suitable(const flr_orbits *o, int nx, int tile, double dt, double fs, double deps)
 {
     const int M = nx == 8 ? 3 : 7;  // longest chain
@@ -457,9 +467,21 @@ bool utv_suitable(const flr_orbits *o, int nx, int tile, double dt, double fs, d
     if (drift > kUtvDrift) return false;
     const double kink = M * o->max_kink * per_sample;    // change of that drift at a node
     if (3.0 * kink * tile / 4.0 > kLtiTol) return false;
-    const double p = std::min(1.0, 2.0 * drift / deps);  // per unit
-    const double fail = 1.0 - std::pow(1.0 - p, 3.0 * nx);
-    return fail < 0.5;
+    return utv_crossings(o, nx, tile, dt, fs, deps) < 0.5;
+}
+
+// Whether 1024-sample windows suit these orbits: few tiles cross a node of the A table (the
+// per-sample path of one long tile takes as long as six others), and the kinks of the arms at the
+// orbit nodes move no unit's position by more than 6e-10 samples off a tile of `tile` samples' model (a kink in mid-tile, every unit at the worst case). The
+// null channel T shows such deviations first: at the 1024-sample window on the cartwheel (5.6e-10) T of
+// a 2 mHz source is 3.6e-8 from the TDI with extended-precision delays, of which the float32 outputs
+// are 2.4e-8 (2.6e-8 at the 512-sample window), where FP64 delays, the reference's, are 5.1e-7 away;
+// kinks of 1.5e-12 s/s would take it to 2.2e-7 (7.6e-8 at 512).
+bool utv_long_tiles(const flr_orbits *o, int nx, int tile, double dt, double fs, double deps)
+{
+    const int M = nx == 8 ? 3 : 7;
+    return utv_crossings(o, nx, tile, dt, fs, deps) < 0.1 &&
+           M * o->max_kink * dt * fs * tile / 4.0 <= 6e-10;
 }
 
 bool lti_source_uniform(const flr_orbits *o, const FusedSource &f, double dt, double fs, int nx,
@@ -522,6 +544,80 @@ int make_fused_config(const flr_response *r, double dt, double fs, int flags, in
     if (fused_lds_bytes(pc, tc, generic, lti, passes, utv) > kMaxLds)
         return fail(FLR_ERR_UNSUPPORTED, "fused delay windows exceed LDS (sampling too fine)");
     return FLR_OK;
+}
+
+// Window of a fused launch nobody chose a shape for, in units of kBlock samples: 1, 2 or 4 for the
+// mixed matrix-core forms, kFusedPasses otherwise. src: the sources; uniform: every one clears the
+// composite-filter test as a whole.
+//
+// Equal arms: a launch takes about 8 us plus, per tile that the busiest CU works through, 4.4, 8.75
+// or 16.3 us for the 256-, 512- and 1024-sample windows (MI355X; within 5% from 8,192 to 3,153,600
+// samples, both generations, dt 5 and 10 s). So the window with the least rounds times cost is
+// taken: long tiles recompute less halo and share one barrier among more work, short ones spread a
+// small launch over the CUs. 131,072 samples: 21.7 (256) against 26.7 us (512); 1-yr source: 219
+// (1024) against 243 us; 64 sources, 1.06e8 samples: 6.53 against 7.20 ms. The results do not depend
+// on the choice.
+// Unequal arms: the per-tile filters make a tile's fixed cost larger, and their results depend on
+// the tile's length (within the float32 rounding), so the choice must not depend on a batch's size:
+// 1024 wherever the filters fit their taps, the orbits suit long tiles (utv_long_tiles) and two
+// workgroups share a CU's LDS. 8 sources, 4.3e6 samples: 578 against 876 us; 131,072: 48.7 against
+// 63.8; below 65,536 samples the two are equal within 4%.
+int auto_passes(const flr_response *r, double dt, double fs, int flags, const FusedSource *src,
+                int num_sources, bool uniform)
+{
+    if (!(flags & FLR_FLAG_MIXED) || r->order != 25 || r->stock_gen == 0) return kFusedPasses;
+    const int zero_edges = (flags & FLR_FLAG_ZERO_EDGES) ? 1 : 0;
+    const int nx = r->stock_gen == 1 ? 8 : 16;
+    ProjConfig pc;
+    TdiConfig tc;
+    StockTdi stock;
+    if (!r->orbits->equal_arm) {
+        const int chain = (int)std::ceil(r->max_chain * r->orbits->max_ltt * fs);
+        return chain + r->order + 3 <= kFir &&
+                       make_fused_config(r, dt, fs, flags, 4, pc, tc, stock) == FLR_OK &&
+                       2 * fused_lds_bytes(pc, tc, false, false, 4, true) + 2 * kFusedStaticLds <= kMaxLds &&
+                       utv_suitable(r->orbits, nx, tc.tile, dt, fs, r->deps) &&
+                       utv_long_tiles(r->orbits, nx, tc.tile, dt, fs, r->deps)
+                   ? 4
+                   : kFusedPasses;
+    }
+    if (!uniform) return kFusedPasses;
+    const double cost[3] = {4.4, 8.75, 16.3};
+    const int cus = compute_units();
+    int best = kFusedPasses;
+    double least = 0.0;
+    for (int k = 2; k >= 0; --k) {  // the longer window where two cost the same
+        const int passes = 1 << k;
+        if (make_fused_config(r, dt, fs, flags, passes, pc, tc, stock) != FLR_OK) continue;
+        if (k == 2 && 2 * fused_lds_bytes(pc, tc, false, true, 4) + 2 * kFusedStaticLds > kMaxLds) continue;
+        int64_t tiles = 0;
+        for (int s = 0; s < num_sources; ++s)
+            tiles += tiles_for(src[s].num_pts, src[s].tdi_start, zero_edges, tc.tile);
+        const double c = cost[k] * (double)((tiles + cus - 1) / cus);
+        if (least == 0.0 || c < least) {
+            least = c;
+            best = passes;
+        }
+    }
+    return best;
+}
+
+// Whether every source clears the composite-filter test as a whole (lti_source_uniform) at the
+// TDI halos of the mixed kernels, which no window changes.
+bool sources_uniform(const flr_response *r, double dt, double fs, int flags, const FusedSource *src,
+                     int num_sources)
+{
+    ProjConfig pc;
+    TdiConfig tc;
+    StockTdi stock;
+    if (!(flags & FLR_FLAG_MIXED) || r->order != 25 || r->stock_gen == 0 || !r->orbits->equal_arm ||
+        make_fused_config(r, dt, fs, flags, kFusedPasses, pc, tc, stock) != FLR_OK)
+        return false;
+    for (int s = 0; s < num_sources; ++s)
+        if (!lti_source_uniform(r->orbits, src[s], dt, fs, r->stock_gen == 1 ? 8 : 16, tc.halo_lo,
+                                tc.halo_hi))
+            return false;
+    return true;
 }
 
 int projection_impl(flr_response *r, double *y_gw, const double *input_in, int num_delays,
@@ -1154,24 +1250,30 @@ int flr_fused_bind(flr_batch *b, const flr_source *sources, int num_sources, con
     DeviceGuard g(b->r->device);
     const int flags = b->flags;
     const int zero_edges = (flags & FLR_FLAG_ZERO_EDGES) ? 1 : 0;
-    // the tile the response's current tables give (they may have changed since the reserve)
-    ProjConfig pc;
-    TdiConfig tc;
-    StockTdi stock;
-    int cst = make_fused_config(b->r, b->dt, b->fs, flags, b->tile_passes, pc, tc, stock);
-    if (cst) return cst;
     std::vector<FusedSource> fs(num_sources);
     std::vector<int> ft(num_sources + 1, 0);
     int64_t samples = 0;
+    int cst;
     for (int s = 0; s < num_sources; ++s) {
         if ((cst = fused_source_record(sources[s], s, flags, h_all, out_all, fs[s]))) return cst;
         samples += sources[s].num_pts;
     }
+    // the tile the response's current tables give (they may have changed since the reserve)
+    const bool uniform = sources_uniform(b->r, b->dt, b->fs, flags, fs.data(), num_sources);
+    const int passes = b->auto_shape ? auto_passes(b->r, b->dt, b->fs, flags, fs.data(), num_sources,
+                                                   uniform)
+                                     : b->tile_passes;
+    ProjConfig pc;
+    TdiConfig tc;
+    StockTdi stock;
+    if ((cst = make_fused_config(b->r, b->dt, b->fs, flags, passes, pc, tc, stock))) return cst;
     if ((cst = fused_tile_prefix(fs.data(), num_sources, zero_edges, tc.tile, ft.data()))) return cst;
     hipStream_t st = (hipStream_t)stream;
     FLR_HIP(hipEventSynchronize(b->uploaded));  // the staging buffers are free again
     // a run still in flight (possibly on another stream) reads the tables about to be replaced
     if (b->ran_recorded) FLR_HIP(hipStreamWaitEvent(st, b->ran, 0));
+    b->tile_passes = passes;
+    b->shape_version = b->r->version;
     b->tile_len = tc.tile;
     // A source's composite filters depend on its first time and first TDI sample (and on the
     // response's tables, tracked by lti_version), not on its sky position or input: when these
@@ -1194,7 +1296,9 @@ int flr_fused_bind(flr_batch *b, const flr_source *sources, int num_sources, con
     b->fused_tiles = ft[num_sources];
     b->out_base = out_all;
     if (!same_refs) b->lti_version = ~0ull;  // new sources: their filters are built now
-    b->uniform_version = ~0ull;               // and the tile-test proof is redone at the run
+    b->lti_uniform = uniform;                 // the tile-test proof for these sources
+    b->uniform_version = b->r->version;
+    b->uniform_tile = tc.tile;
     const int fst = lti_refresh(b, st);
     // recorded after the filters too: flr_fused_create waits on it before returning
     FLR_HIP(hipEventRecord(b->uploaded, st));
@@ -1237,6 +1341,12 @@ int fused_launch(flr_batch *b, hipStream_t s, const void *data, double *sums)
     StockTdi stock;
     int st;
     if (b->num_sources < 1) return fail(FLR_ERR_INVALID_ARGUMENT, "no sources bound to the batch");
+    if (b->auto_shape && b->shape_version != r->version) {  // the tables changed since the bind
+        b->tile_passes = auto_passes(r, b->dt, b->fs, b->flags, b->h_fused, b->num_sources,
+                                     sources_uniform(r, b->dt, b->fs, b->flags, b->h_fused,
+                                                     b->num_sources));
+        b->shape_version = r->version;
+    }
     if ((st = make_fused_config(r, b->dt, b->fs, b->flags, b->tile_passes, pc, tc, stock)))
         return st;
     bool cap = false;
@@ -1270,11 +1380,7 @@ int fused_launch(flr_batch *b, hipStream_t s, const void *data, double *sums)
         if (b->uniform_version != r->version || b->uniform_tile != tc.tile) {
             // the staging copy holds the bound sources (its upload may still be in flight:
             // reading it on the host is fine)
-            bool all = true;
-            for (int q = 0; q < b->num_sources && all; ++q)
-                all = lti_source_uniform(r->orbits, b->h_fused[q], b->dt, b->fs,
-                                         stock.generation == 1 ? 8 : 16, tc.halo_lo, tc.halo_hi);
-            b->lti_uniform = all;
+            b->lti_uniform = sources_uniform(r, b->dt, b->fs, b->flags, b->h_fused, b->num_sources);
             b->uniform_version = r->version;
             b->uniform_tile = tc.tile;
         }
@@ -1378,7 +1484,16 @@ int flr_batch_set_launch(flr_batch *b, int tile_samples, int grid_per_cu)
         FLR_HIP(hipEventSynchronize(b->uploaded));
         b->tile_passes = passes;
     }
+    if (tile_samples != 0) b->auto_shape = false;
     if (grid_per_cu != 0) b->grid_per_cu = grid_per_cu;
+    return FLR_OK;
+}
+
+int flr_batch_launch(const flr_batch *b, int *tile_samples, int *grid_per_cu)
+{
+    if (!b) return fail(FLR_ERR_INVALID_ARGUMENT, "batch is NULL");
+    if (tile_samples) *tile_samples = b->fused ? b->tile_passes * kBlock : kBlock;
+    if (grid_per_cu) *grid_per_cu = b->grid_per_cu;
     return FLR_OK;
 }
 
@@ -1557,18 +1672,22 @@ int flr_fused_run_static(flr_response *r, const flr_source *sources, int num_sou
     }
     DeviceGuard g(r->device);
     hipStream_t s = (hipStream_t)stream;
+    // validate every source before anything is enqueued
+    int st;
+    std::vector<FusedSource> recs(num_sources);
+    for (int q = 0; q < num_sources; ++q)
+        if ((st = fused_source_record(sources[q], q, flags, h_all, out_all, recs[q]))) return st;
+    const bool uniform = sources_uniform(r, dt, sampling_frequency, flags, recs.data(), num_sources);
+    if (tile_samples == 0)
+        passes = auto_passes(r, dt, sampling_frequency, flags, recs.data(), num_sources, uniform);
     ProjConfig pc;
     TdiConfig tc;
     StockTdi stock;
-    int st = make_fused_config(r, dt, sampling_frequency, flags, passes, pc, tc, stock);
-    if (st) return st;
-    // validate every source before anything is enqueued
+    if ((st = make_fused_config(r, dt, sampling_frequency, flags, passes, pc, tc, stock))) return st;
     const int zero_edges = (flags & FLR_FLAG_ZERO_EDGES) ? 1 : 0;
     int64_t tiles = 0;
     int min_start = INT32_MAX;
-    for (int q = 0; q < num_sources; ++q) {
-        FusedSource f;
-        if ((st = fused_source_record(sources[q], q, flags, h_all, out_all, f))) return st;
+    for (const FusedSource &f : recs) {
         min_start = std::min(min_start, f.tdi_start);
         tiles += tiles_for(f.num_pts, f.tdi_start, zero_edges, tc.tile);
         if (tiles > INT32_MAX) return fail(FLR_ERR_UNSUPPORTED, "batch has too many tiles");
@@ -1585,8 +1704,7 @@ int flr_fused_run_static(flr_response *r, const flr_source *sources, int num_sou
         chunk.first = first;
         chunk.count = std::min(kStageChunk, num_sources - first);
         for (int k = 0; k < chunk.count; ++k) {
-            (void)fused_source_record(sources[first + k], first + k, flags, h_all, out_all,
-                                      chunk.src[k]);
+            chunk.src[k] = recs[first + k];
             prefix += tiles_for(chunk.src[k].num_pts, chunk.src[k].tdi_start, zero_edges, tc.tile);
             chunk.tile_end[k] = prefix;
         }
@@ -1598,16 +1716,7 @@ int flr_fused_run_static(flr_response *r, const flr_source *sources, int num_sou
     const OrbitView orb = r->orbits->view();
     if (mixed) {
         tc.lti_fir = d_lti;
-        if (stock.generation != 0 && stock.equal_arm && r->order == 25) {
-            bool all = true;
-            for (int q = 0; q < num_sources && all; ++q) {
-                FusedSource f;
-                (void)fused_source_record(sources[q], q, flags, h_all, out_all, f);
-                all = lti_source_uniform(r->orbits, f, dt, sampling_frequency,
-                                         stock.generation == 1 ? 8 : 16, tc.halo_lo, tc.halo_hi);
-            }
-            tc.lti_uniform = all ? 1 : 0;
-        }
+        tc.lti_uniform = uniform ? 1 : 0;
         if (stock.generation != 0 && !stock.equal_arm && r->order == 25)
             tc.utv = utv_suitable(r->orbits, stock.generation == 1 ? 8 : 16, tc.tile, dt,
                                   sampling_frequency, r->deps) ? 1 : 0;

@@ -188,6 +188,13 @@ struct FusedSource {
     double k[3], u[3], v[3];
 };
 
+// Static LDS of a mixed matrix-core kernel at most: the E and orbit-node copies, the unit model of
+// the unequal-arm form, the inner-product slots.
+constexpr size_t kFusedStaticLds = 6656;
+
+// CUs of the current device (looked up once).
+int compute_units();
+
 // Launchers (flr_kernels.hip).
 hipError_t launch_projection(const ProjConfig &cfg, const ProjSource &src, const OrbitView &orb,
                              const LagrangeView &lg, bool exact, bool equal_arm,

@@ -298,17 +298,22 @@ __global__ void clear_kernel(int *word)
 
 // ------------------------------------------------------------------ launchers
 
+int compute_units()
+{
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+            n <= 0)
+            n = 256;
+        return n;
+    }();
+    return cus;
+}
+
 int batch_grid(int total_tiles, int grid_per_cu)
 {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            cus <= 0)
-            cus = 256;
-    }
-    const int grid = cus * (grid_per_cu > 0 ? grid_per_cu : 16);
+    const int grid = compute_units() * (grid_per_cu > 0 ? grid_per_cu : 16);
     return total_tiles < grid ? total_tiles : grid;
 }
 

@@ -380,7 +380,9 @@ class BatchPlan:
         self._h = h
         self.num_sources = n
         self.samples = int(lib().flr_batch_samples(h))
-        self.launch_shape = (512 if br.fused else 256, 32)  # (tile window samples, WGs per CU)
+        tile, grid = ctypes.c_int(), ctypes.c_int()
+        check(lib().flr_batch_launch(h, ctypes.byref(tile), ctypes.byref(grid)))
+        self.launch_shape = (tile.value, grid.value)  # (tile window samples, WGs per CU)
 
     def _records(self, lams, betas, t0s=None, scales=None):
         """flr_source records of the plan's sources (packed offsets, the lengths of the plan)."""
