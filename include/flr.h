@@ -281,6 +281,10 @@ typedef struct {
  * source are left untouched. */
 int flr_gb_generate(const flr_gb_source *sources, int num_sources, int64_t total_samples,
                     double dt, int format, void *out, void *stream);
+/* The same for one source, whose record is in HOST memory: it travels as a kernel argument, so
+ * there is no table to upload. */
+int flr_gb_generate_one(const flr_gb_source *source, int64_t total_samples, double dt, int format,
+                        void *out, void *stream);
 
 /* ------------------------------------------------------------------ packed series
  * No counterpart in the reference. Statistics of the sources of a packed series, and its

@@ -1512,6 +1512,21 @@ int flr_gb_generate(const flr_gb_source *sources, int num_sources, int64_t total
     return FLR_OK;
 }
 
+int flr_gb_generate_one(const flr_gb_source *source, int64_t total_samples, double dt, int format,
+                        void *out, void *stream)
+{
+    if (!source) return fail(FLR_ERR_INVALID_ARGUMENT, "no sources");
+    if (!out || total_samples < 1) return fail(FLR_ERR_INVALID_ARGUMENT, "empty output");
+    if (!(dt > 0.0)) return fail(FLR_ERR_INVALID_ARGUMENT, "dt must be > 0");
+    if (source->offset < 0 || source->num_pts < 0)
+        return fail(FLR_ERR_INVALID_ARGUMENT, "bad source offset or size");
+    if (format != FLR_GB_COMPLEX128 && format != FLR_GB_COMPLEX64 && format != FLR_GB_Q31)
+        return fail(FLR_ERR_INVALID_ARGUMENT, "unknown waveform format");
+    hipError_t e = launch_gb_one(*source, total_samples, dt, format, out, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "waveform launch");
+    return FLR_OK;
+}
+
 namespace {
 
 int series_args(const void *h, int num_sources, const int64_t *offsets, int64_t max_len)

@@ -254,6 +254,8 @@ size_t fused_lds_bytes(const ProjConfig &pc, const TdiConfig &tc, bool generic, 
 hipError_t launch_inner_reduce(const double *part, const int *tile_start, int num_sources,
                                double *sums, hipStream_t stream);
 // Galactic-binary generator (flr_waveform.hip).
+hipError_t launch_gb_one(const flr_gb_source &source, int64_t total, double dt, int format,
+                         void *out, hipStream_t stream);
 hipError_t launch_gb(const flr_gb_source *sources, int num_sources, int64_t total, double dt,
                      int format, void *out, hipStream_t stream);
 // Statistics and 8-byte formats of a packed series (flr_pack.hip); series_chunks(max_len): the

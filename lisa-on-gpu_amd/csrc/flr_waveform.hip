@@ -95,6 +95,34 @@ __global__ __launch_bounds__(kBlock) void gb_kernel(const flr_gb_source *__restr
     }
 }
 
+// One source, its record in the kernel's arguments (scalar registers): no table to upload before the
+// launch and no lookup of a sample's source. The call that generates one waveform is bound by the
+// host and the stream, not by this kernel (4 us for 8,192 samples, 15 for a year's 3,153,600): the
+// table's blocking upload made every call wait for the stream (GBWave of 8,192 samples 48 us on the
+// host, 8 without it).
+__global__ __launch_bounds__(kBlock) void gb_one_kernel(flr_gb_source s, int64_t total, double dt,
+                                                        int format, void *__restrict__ out)
+{
+    const int64_t k0 = (int64_t)blockIdx.x * (kBlock * kGbPerThread);
+#pragma unroll 1
+    for (int r = 0; r < kGbPerThread; ++r) {
+        const int64_t k = k0 + (int64_t)r * kBlock + threadIdx.x;
+        if (k >= s.num_pts || s.offset + k >= total) return;
+        gb_write(s, k, s.offset + k, dt, format, out);
+    }
+}
+
+hipError_t launch_gb_one(const flr_gb_source &source, int64_t total, double dt, int format,
+                         void *out, hipStream_t stream)
+{
+    const int64_t per_block = (int64_t)kBlock * kGbPerThread;
+    const int64_t blocks = ((int64_t)source.num_pts + per_block - 1) / per_block;
+    if (blocks <= 0) return hipSuccess;
+    hipLaunchKernelGGL(gb_one_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, stream, source,
+                       total, dt, format, out);
+    return hipGetLastError();
+}
+
 hipError_t launch_gb(const flr_gb_source *sources, int num_sources, int64_t total, double dt,
                      int format, void *out, hipStream_t stream)
 {

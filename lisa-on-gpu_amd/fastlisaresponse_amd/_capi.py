@@ -62,6 +62,7 @@ SIGNATURES = {
     "flr_batch_destroy": (None, [_vp]),
     "flr_fused_run_static": (_ci, [_vp, _vp, _ci, _vp, _vp, _cd, _cd, _ci, _ci, _ci, _vp]),
     "flr_gb_generate": (_ci, [_vp, _ci, ctypes.c_int64, _cd, _ci, _vp, _vp]),
+    "flr_gb_generate_one": (_ci, [_vp, ctypes.c_int64, _cd, _ci, _vp, _vp]),
     "flr_series_work": (ctypes.c_int64, [_ci, ctypes.c_int64]),
     "flr_series_stats": (_ci, [_vp, _ci, _vp, _ci, ctypes.c_int64, _vp, ctypes.c_int64, _vp, _vp]),
     "flr_series_pack": (_ci, [_vp, _vp, _ci, ctypes.c_int64, _vp, _ci, _vp, _vp]),

@@ -9,7 +9,7 @@ parameters alone (MCMC walkers, catalogues, served requests).
 """
 from __future__ import annotations
 
-import ctypes
+import struct
 from typing import Optional, Sequence, Tuple
 
 import numpy as np
@@ -17,6 +17,7 @@ import torch
 
 from . import _capi
 from ._capi import check, lib
+from .backend import current_stream
 
 YRSID_SI = 31558149.763545603
 
@@ -28,6 +29,7 @@ GB_SOURCE_DTYPE = np.dtype([
     ("phi0", np.float64), ("t0", np.float64), ("scale", np.float64),
 ])
 assert GB_SOURCE_DTYPE.itemsize == 96
+_GB_RECORD = struct.Struct("<qii10d")  # the same record
 
 FORMATS = {"complex128": _capi.FLR_GB_COMPLEX128, "complex64": _capi.FLR_GB_COMPLEX64,
            "q31": _capi.FLR_GB_Q31}
@@ -75,8 +77,9 @@ def generate_gb(params, lengths: Sequence[int], dt: float, fmt: str = "complex12
                 offsets: Optional[Sequence[int]] = None):
     """Waveforms of the sources (rows of params: A, f0, fdot, iota, phi0, psi) in `fmt`, packed
     back to back (or at `offsets` in `out`, other samples untouched); returns (tensor, scales).
-    `out`, if given, must have the format's dtype. The records are uploaded and the generator
-    enqueued on `stream` (default: the current one)."""
+    `out`, if given, must have the format's dtype. The generator is enqueued on `stream` (default:
+    the current one) without waiting for it: one source's record travels as a kernel argument,
+    several from pinned memory."""
     if fmt not in FORMATS:
         raise ValueError(f"fmt must be one of {sorted(FORMATS)}")
     rec, scales = gb_table(params, lengths, t0s, fmt, offsets)
@@ -97,11 +100,30 @@ def generate_gb(params, lengths: Sequence[int], dt: float, fmt: str = "complex12
     with torch.cuda.stream(stream):  # table allocated, filled and read in this stream's order
         if out is None:
             out = torch.empty(numel, dtype=dtype, device=device)
-        table = torch.from_numpy(rec.view(np.uint8).copy()).to(out.device, non_blocking=False)
-        check(lib().flr_gb_generate(ctypes.c_void_p(table.data_ptr()), len(rec), total, float(dt),
-                                    FORMATS[fmt], ctypes.c_void_p(out.data_ptr()),
-                                    ctypes.c_void_p(stream.cuda_stream)))
+        if len(rec) == 1:
+            check(lib().flr_gb_generate_one(rec.ctypes.data, total, float(dt), FORMATS[fmt],
+                                            out.data_ptr(), stream.cuda_stream))
+        else:
+            table = torch.empty(rec.nbytes, dtype=torch.uint8, pin_memory=True)
+            table.numpy()[:] = rec.view(np.uint8)
+            table = table.to(out.device, non_blocking=True)
+            check(lib().flr_gb_generate(table.data_ptr(), len(rec), total, float(dt), FORMATS[fmt],
+                                        out.data_ptr(), stream.cuda_stream))
     return out, scales
+
+
+def gb_record(A, f0, fdot, iota, phi0, psi, n: int) -> bytes:
+    """The record of one source of n samples from time 0, from plain numbers and in gb_table's
+    arithmetic (~20 us less on the host than a table of one row)."""
+    ci = float(np.cos(iota))
+    return _GB_RECORD.pack(0, n, 0, A, f0, fdot, 11.0 / 3.0 * (fdot * fdot) / f0, ci,
+                           float(np.cos(2.0 * psi)), float(np.sin(2.0 * psi)), phi0, 0.0,
+                           A * (1.0 + ci * ci))
+
+
+def num_samples(T: float, dt: float) -> int:
+    """len(np.arange(0, T yr, dt)), as arange rounds it."""
+    return max(0, int(np.ceil((T * YRSID_SI - 0.0) / dt)))
 
 
 class GBWave:
@@ -110,6 +132,12 @@ class GBWave:
     dt)."""
 
     def __call__(self, A, f, fdot, iota, phi0, psi, T=1.0, dt=10.0):
-        n = len(np.arange(0.0, T * YRSID_SI, dt))
+        n = num_samples(T, dt)
+        if n > 0 and f and all(isinstance(x, (int, float)) for x in (A, f, fdot, iota, phi0, psi)):
+            rec = gb_record(A, f, fdot, iota, phi0, psi, n)
+            h = torch.empty(n, dtype=torch.complex128, device="cuda")
+            check(lib().flr_gb_generate_one(rec, n, float(dt), _capi.FLR_GB_COMPLEX128,
+                                            h.data_ptr(), current_stream()))
+            return h
         h, _ = generate_gb(np.array([[A, f, fdot, iota, phi0, psi]]), [n], dt)
         return h
