@@ -29,7 +29,8 @@ def device() -> torch.device:
 
 
 def current_stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """The raw handle of torch's current stream (without building a Stream object, ~7 us)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 _NP_OF = {torch.float64: np.float64, torch.complex128: np.complex128, torch.int32: np.int32}
@@ -63,7 +64,10 @@ def to_device(x, dtype: torch.dtype, name: str, n: int | None = None) -> torch.T
 
 
 def to_host(x, np_dtype, name: str, n: int | None = None) -> np.ndarray:
-    """Contiguous numpy copy of a small configuration array."""
+    """Contiguous numpy array of a small configuration array."""
+    if type(x) is np.ndarray and x.dtype == np_dtype and x.ndim == 1 and x.flags.c_contiguous and (
+            n is None or x.size == n):
+        return x
     if isinstance(x, torch.Tensor):
         x = x.detach().cpu().numpy()
     arr = np.ascontiguousarray(np.asarray(x), dtype=np_dtype).reshape(-1)

@@ -35,6 +35,9 @@ from .backend import current_stream
 from .response import pyResponseTDI
 from .tables import buffer_indices, sky_basis
 
+# flr_source of include/flr.h
+_SOURCE_DTYPE = np.dtype(_capi.FlrSource)
+
 PRECISIONS = ("fp64", "mixed", "mixed-q31", "mixed-c128")
 
 C_SI = 299792458.0
@@ -266,6 +269,17 @@ def pack_q31(h: torch.Tensor, lengths: Sequence[int]):
     return out, scales
 
 
+def _host_values(x) -> np.ndarray:
+    """Per-source numbers (a list, array or tensor) as a host array."""
+    if isinstance(x, torch.Tensor):
+        return x.detach().cpu().numpy()
+    if isinstance(x, np.ndarray):
+        return x
+    if any(isinstance(v, torch.Tensor) for v in x):
+        return np.array([float(v) for v in x])
+    return np.asarray(x)
+
+
 class BatchedResponse:
     """Response configuration shared by a batch: sampling, order, TDI, orbits, channels.
 
@@ -370,11 +384,13 @@ class BatchPlan:
             flags |= _capi.FLR_FLAG_C128
         h = ctypes.c_void_p()
         if br.fused:
-            check(lib().flr_fused_create(br.model.cpp_response._h, srcs, n, h_all.data_ptr(),
+            check(lib().flr_fused_create(br.model.cpp_response._h, srcs.ctypes.data, n,
+                                         h_all.data_ptr(),
                                          self.out_all.data_ptr(), br.dt, br.sampling_frequency,
                                          flags, ctypes.byref(h)))
         else:
-            check(lib().flr_batch_create(br.model.cpp_response._h, srcs, n, h_all.data_ptr(),
+            check(lib().flr_batch_create(br.model.cpp_response._h, srcs.ctypes.data, n,
+                                         h_all.data_ptr(),
                                          self.y_all.data_ptr(), self.out_all.data_ptr(), br.dt,
                                          br.sampling_frequency, flags, ctypes.byref(h)))
         self._h = h
@@ -390,19 +406,16 @@ class BatchPlan:
         if (len(lams) != n or len(betas) != n or (t0s is not None and len(t0s) != n)
                 or (scales is not None and len(scales) != n)):
             raise ValueError("lams, betas (and t0s, scales) must have one entry per source")
-        srcs = (_capi.FlrSource * n)()
-        for s in range(n):
-            k, u, v = sky_basis(lams[s], betas[s])
-            q = srcs[s]
-            q.offset = int(self.offsets[s])
-            q.num_pts = int(self.lengths[s])
-            q.projections_start_ind = self.br.projections_start_ind
-            q.tdi_start_ind = self.br.tdi_start_ind
-            q.t0 = 0.0 if t0s is None else float(t0s[s])
-            q.scale = 1.0 if scales is None else float(scales[s])
-            for c in range(3):
-                q.k[c], q.u[c], q.v[c] = k[c], u[c], v[c]
-        return srcs
+        rec = np.zeros(n, dtype=_SOURCE_DTYPE)
+        rec["offset"], rec["num_pts"] = self.offsets, self.lengths
+        rec["projections_start_ind"] = self.br.projections_start_ind
+        rec["tdi_start_ind"] = self.br.tdi_start_ind
+        rec["t0"] = 0.0 if t0s is None else _host_values(t0s)
+        rec["scale"] = 1.0 if scales is None else _host_values(scales)
+        k, u, v = sky_basis(_host_values(lams), _host_values(betas))
+        for c in range(3):
+            rec["k"][:, c], rec["u"][:, c], rec["v"][:, c] = k[c], u[c], v[c]
+        return rec
 
     def rebind(self, lams, betas, t0s=None, scales=None, h_all: Optional[torch.Tensor] = None,
                stream: Optional[int] = None) -> None:
@@ -425,7 +438,7 @@ class BatchPlan:
                                                action=self.br.storage_check)
             self.h_all = h_all
         srcs = self._records(lams, betas, t0s, scales)
-        check(lib().flr_fused_bind(self._h, srcs, len(self.lengths), self.h_all.data_ptr(),
+        check(lib().flr_fused_bind(self._h, srcs.ctypes.data, len(self.lengths), self.h_all.data_ptr(),
                                    self.out_all.data_ptr(),
                                    current_stream() if stream is None else stream))
 

@@ -291,7 +291,7 @@ class pyResponseTDI:
 
     def _data_time_check(self, t0: float, n: int, input_in):
         t_last = t0 + (n - 1) * self.dt
-        if t_last > self.response_orbits.t.max():
+        if t_last > self.response_orbits.t[-1]:  # an increasing grid
             warnings.warn("Input waveform is longer than available orbital information. "
                           "Trimming to fit orbital information.")
             t_data = t0 + np.arange(n) * self.dt

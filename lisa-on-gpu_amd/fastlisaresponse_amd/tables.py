@@ -126,10 +126,11 @@ def buffer_indices(sampling_frequency: float, order: int, t_buffer: float, x_bas
 
 
 def sky_basis(lam: float, beta: float):
-    """(k, u, v): propagation direction and polarisation basis for ecliptic (lam, beta)."""
+    """(k, u, v): propagation direction and polarisation basis for ecliptic (lam, beta), numbers or
+    arrays of one length (then [3, sources])."""
     cb, sb = np.cos(beta), np.sin(beta)
     cl, sl = np.cos(lam), np.sin(lam)
     k = np.array([-cb * cl, -cb * sl, -sb])
-    u = np.array([sl, -cl, 0.0])
+    u = np.array([sl, -cl, np.zeros_like(sl)])
     v = np.array([-sb * cl, -sb * sl, cb])
     return k, u, v

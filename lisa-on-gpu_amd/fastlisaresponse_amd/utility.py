@@ -108,18 +108,25 @@ def overlap_from_sums(sums, dsums, N: int) -> torch.Tensor:
     return (dh / torch.sqrt(dd * hh)).mean(-1)
 
 
+def _variances(noise_var, device) -> torch.Tensor:
+    """sigma^2 per channel on the device; a number is filled in there (its transfer would wait for
+    the stream)."""
+    if isinstance(noise_var, (int, float)):
+        return torch.full((3,), float(noise_var), dtype=torch.float64, device=device)
+    w = torch.as_tensor(noise_var, dtype=torch.float64, device=device).reshape(-1)
+    return w.expand(3) if w.numel() == 1 else w
+
+
 def inner_from_sums(sums, noise_var=1.0) -> torch.Tensor:
     """White-noise inner products (d|h) = sum_c sum_i d h / sigma_c^2 and (h|h) per source
     ([sources, 2]); noise_var: sigma^2, a scalar or one value per channel."""
-    w = torch.as_tensor(noise_var, dtype=torch.float64, device=sums.device).reshape(-1)
-    w = w.expand(3) if w.numel() == 1 else w
+    w = _variances(noise_var, sums.device)
     return torch.stack([(sums[..., 0] / w).sum(-1), (sums[..., 1] / w).sum(-1)], dim=-1)
 
 
 def log_likelihood_from_sums(sums, dsums, noise_var=1.0) -> torch.Tensor:
     """Gaussian white-noise log-likelihood -1/2 sum_c sum_i (d - h)^2 / sigma_c^2 per source
     (up to the normalisation constant), from the fused sums and data_sums."""
-    w = torch.as_tensor(noise_var, dtype=torch.float64, device=sums.device).reshape(-1)
-    w = w.expand(3) if w.numel() == 1 else w
+    w = _variances(noise_var, sums.device)
     chi2 = (dsums[..., 0] - 2.0 * sums[..., 0] + sums[..., 1]) / w
     return -0.5 * chi2.sum(-1)
