@@ -199,6 +199,14 @@ int compute_units();
 hipError_t launch_projection(const ProjConfig &cfg, const ProjSource &src, const OrbitView &orb,
                              const LagrangeView &lg, bool exact, bool equal_arm,
                              hipStream_t stream);
+// The same for short series, a sample's work split over waves (flr_split.hip): false if the series is
+// longer than these kernels are used for, otherwise launched, with its status in err.
+bool launch_projection_split(const ProjConfig &cfg, const ProjSource &src, const OrbitView &orb,
+                             const LagrangeView &lg, int form, bool equal_arm, hipStream_t stream,
+                             hipError_t &err);
+bool launch_tdi_split(const TdiConfig &cfg, const TdiSource &src, const OrbitView &orb,
+                      const LagrangeView &lg, int form, const StockTdi &stock, hipStream_t stream,
+                      hipError_t &err);
 hipError_t launch_projection_batch(const ProjConfig &cfg, const Batch<ProjSource> &batch,
                                    const OrbitView &orb, const LagrangeView &lg, bool exact,
                                    bool equal_arm, int grid_per_cu, hipStream_t stream);

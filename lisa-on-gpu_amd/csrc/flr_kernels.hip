@@ -327,7 +327,10 @@ hipError_t launch_projection(const ProjConfig &cfg, const ProjSource &src, const
 {
     const int nb = tiles_for(src.num_delays, src.start, cfg.zero_edges);
     const size_t shm = proj_lds(cfg);
-    return by_form(stencil_form(exact, (int64_t)src.start - cfg.halo_lo, lg.h), [&](auto form) {
+    const int form = stencil_form(exact, (int64_t)src.start - cfg.halo_lo, lg.h);
+    hipError_t err;
+    if (launch_projection_split(cfg, src, orb, lg, form, equal_arm, stream, err)) return err;
+    return by_form(form, [&](auto form) {
         constexpr int F = decltype(form)::value;
         if (lg.h == 13 && equal_arm)
             return launch(projection_kernel<F, 13, true>, nb, shm, stream, cfg, src, orb, lg);
@@ -364,7 +367,10 @@ hipError_t launch_tdi(const TdiConfig &cfg, const TdiSource &src, const OrbitVie
 {
     const int nb = tiles_for(src.num_delays, src.start, cfg.zero_edges);
     const RowMap &rm = st.rows;
-    return by_form(stencil_form(exact, (int64_t)src.start - cfg.halo_lo, lg.h), [&](auto form) {
+    const int form = stencil_form(exact, (int64_t)src.start - cfg.halo_lo, lg.h);
+    hipError_t err;
+    if (launch_tdi_split(cfg, src, orb, lg, form, st, stream, err)) return err;
+    return by_form(form, [&](auto form) {
         constexpr int F = decltype(form)::value;
         if (use_stock(st, lg)) {
             const size_t shm = tdi_lds(cfg, true);

@@ -10,24 +10,91 @@
 
 namespace flr {
 
-// Sample range of tile `tile` of a source: lanes i in [i0, i0 + kBlock), computed samples
+// Sample range of tile `tile` of a source: lanes i in [i0, i0 + len), computed samples
 // [lo_valid, hi_valid), and the tile's first/last computed sample.
 struct TileRange {
     int i0, lo_valid, hi_valid, first, last;
 };
 
-__device__ __forceinline__ TileRange tile_range(int tile, int num_delays, int start, int zero_edges)
+__device__ __forceinline__ TileRange tile_range(int tile, int num_delays, int start, int zero_edges,
+                                                int len = kBlock)
 {
     TileRange r;
-    r.i0 = (zero_edges ? 0 : start) + tile * kBlock;
+    r.i0 = (zero_edges ? 0 : start) + tile * len;
     r.lo_valid = start;
     r.hi_valid = num_delays - start;
     r.first = max(r.i0, r.lo_valid);
-    r.last = min(r.i0 + kBlock, r.hi_valid) - 1;
+    r.last = min(r.i0 + len, r.hi_valid) - 1;
     return r;
 }
 
 // ------------------------------------------------------------------ projection
+
+// Projection of one link from its receiver's and emitter's positions (xr, xe) and interpolated
+// signals (hr, he); NaN if a stencil fell outside its window (bad). Operation order of the exact
+// forms: LISAResponse.cu:565-668.
+template <int EXACT, int ESRC>
+__device__ __forceinline__ double link_value(const double (&k)[3], const double (&u)[3],
+                                             const double (&v)[3], const double (&xr)[3],
+                                             const double (&xe)[3], double2 hr, double2 he, bool bad)
+{
+    double n[3];
+    double norm = 0.0;
+    if constexpr (EXACT) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            double nt = xr[c] - xe[c];
+            n[c] = nt;
+            norm += nt * nt;
+        }
+        norm = sqrt(norm);
+        const double y_norm = rcp_nr2(norm);  // one reciprocal for the three quotients
+#pragma unroll
+        for (int c = 0; c < 3; ++c) n[c] = div_rcp(n[c], norm, y_norm);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) n[c] = xr[c] - xe[c];
+        norm = dot3_form<false>(n, n);
+        // one reciprocal square root instead of a root and three divisions
+        const double inv = ESRC == kELdsFold ? rsqrt_pos1(norm) : rsqrt_pos(norm);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) n[c] = n[c] * inv;
+    }
+    const double un = dot3_form<EXACT>(u, n);
+    const double vn = dot3_form<EXACT>(v, n);
+    const double xi_p =
+        EXACT ? 0.5 * ((un * un) - (vn * vn)) : 0.5 * __builtin_fma(un, un, -(vn * vn));
+    const double xi_c = un * vn;
+    const double kn = dot3_form<EXACT>(k, n);
+    double out = __builtin_nan("");
+    if (!bad) {
+        const double pre = EXACT ? 1. / (1. - kn)
+                           : ESRC == kELdsFold ? rcp_nr1(1. - kn) : rcp_nr2(1. - kn);
+        const double large = EXACT ? (he.x - hr.x) * xi_p + (he.y - hr.y) * xi_c
+                                   : __builtin_fma(he.x - hr.x, xi_p, (he.y - hr.y) * xi_c);
+        out = pre * large;
+    }
+    return out;
+}
+
+// One complex stencil at window offset l and fraction e; the fast form with a compile-time order reads
+// every tap at a constant offset from the lowest one.
+template <int EXACT, int H, int ESRC>
+__device__ __forceinline__ double2 window_stencil(const double2 *hwin, int l, double e,
+                                                  const LagrangeView &lg, double y_deps,
+                                                  const double *E_lds)
+{
+    if constexpr (!EXACT && H > 0) {
+        int lo = l - (H - 1);
+        pin(lo);  // an opaque base: the taps are not re-addressed from another register
+        if constexpr (ESRC == kELdsFold)
+            return stencil_fold_c_lo<H>(hwin + lo, e, lg, E_lds);
+        else
+            return stencil_fast_c_lo<H, ESRC>(hwin + lo, e, lg, E_lds);
+    } else {
+        return stencil_c<EXACT, H>(hwin + l, e, lg, y_deps);
+    }
+}
 
 // Projections of all six links at time t from the staged h window (hwin[0] = sample win_lo):
 // per receiving spacecraft its stencil (shared by its two links), then each link's emitter
@@ -59,19 +126,8 @@ __device__ __forceinline__ bool project_links(const ProjConfig &cfg, const doubl
     };
     const OrbitNode nr = node(t);
     bool bad = false;
-    // one complex stencil at window offset l (sample d = win_lo + l) and fraction e; the fast
-    // form with a compile-time order reads every tap at a constant offset from the lowest one
     auto cstencil = [&](int l, double e) -> double2 {
-        if constexpr (!EXACT && H > 0) {
-            int lo = l - (H - 1);
-            pin(lo);  // an opaque base: the taps are not re-addressed from another register
-            if constexpr (ESRC == kELdsFold)
-                return stencil_fold_c_lo<H>(hwin + lo, e, lg, E_lds);
-            else
-                return stencil_fast_c_lo<H, ESRC>(hwin + lo, e, lg, E_lds);
-        } else {
-            return stencil_c<EXACT, H>(hwin + l, e, lg, y_deps);
-        }
+        return window_stencil<EXACT, H, ESRC>(hwin, l, e, lg, y_deps, E_lds);
     };
     // EQ (all six light travel times bitwise equal): the emission time t - L, the emitter's
     // position and so the emitter stencil depend on the emitting spacecraft only -- 3 emitter
@@ -116,7 +172,7 @@ __device__ __forceinline__ bool project_links(const ProjConfig &cfg, const doubl
         static_for<2>([&](auto q) {
             constexpr int se = (s + 1 + q) % 3;  // the emitters of receiver s
             const int row = CANON ? stock::canon(10 * (s + 1) + se + 1) : cfg.link_row[s][se];
-            double xe[3], n[3];
+            double xe[3];
             double2 he = make_double2(0.0, 0.0);
             bool bq;
             if constexpr (EQ) {
@@ -137,44 +193,7 @@ __device__ __forceinline__ bool project_links(const ProjConfig &cfg, const doubl
                 bq = br || miss || (le - (h - 1) < 0) || (le + h >= win_len);
                 if (!bq) he = cstencil(le, e_em);
             }
-            double norm = 0.0;
-            if constexpr (EXACT) {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    double nt = xr[c] - xe[c];
-                    n[c] = nt;
-                    norm += nt * nt;
-                }
-            } else {
-#pragma unroll
-                for (int c = 0; c < 3; ++c) n[c] = xr[c] - xe[c];
-                norm = dot3_form<false>(n, n);
-            }
-            if constexpr (EXACT) {
-                norm = sqrt(norm);
-                const double y_norm = rcp_nr2(norm);  // one reciprocal for the three quotients
-#pragma unroll
-                for (int c = 0; c < 3; ++c) n[c] = div_rcp(n[c], norm, y_norm);
-            } else {  // one reciprocal square root instead of a root and three divisions
-                const double inv = ESRC == kELdsFold ? rsqrt_pos1(norm) : rsqrt_pos(norm);
-#pragma unroll
-                for (int c = 0; c < 3; ++c) n[c] = n[c] * inv;
-            }
-            const double un = dot3_form<EXACT>(u, n);
-            const double vn = dot3_form<EXACT>(v, n);
-            const double xi_p = EXACT ? 0.5 * ((un * un) - (vn * vn))
-                                      : 0.5 * __builtin_fma(un, un, -(vn * vn));
-            const double xi_c = un * vn;
-            const double kn = dot3_form<EXACT>(k, n);
-            double out = __builtin_nan("");
-            if (!bq) {
-                const double pre = EXACT ? 1. / (1. - kn)
-                                   : ESRC == kELdsFold ? rcp_nr1(1. - kn) : rcp_nr2(1. - kn);
-                const double large =
-                    EXACT ? (he.x - hr.x) * xi_p + (he.y - hr.y) * xi_c
-                          : __builtin_fma(he.x - hr.x, xi_p, (he.y - hr.y) * xi_c);
-                out = pre * large;
-            }
+            const double out = link_value<EXACT, ESRC>(k, u, v, xr, xe, hr, he, bq);
             bad |= bq;
             store(row, out);
         });

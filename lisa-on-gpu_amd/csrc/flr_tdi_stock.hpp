@@ -294,64 +294,79 @@ __device__ __forceinline__ void linear_series(double *yc, int cap, const RowMap 
     }
 }
 
+// One chain length of the equal-arm stock TDI from the combined series (fast stencils): at delay Dm
+// one set of stencil weights and one stencil per output, times sgn, into val (NaN, and false, if a
+// stencil fell outside the window). The taps are read through cols(o, kind, c0) -> a pointer p with
+// p[k] = window column c0 + k of output o's series of that kind (k = 0 .. 2H-1).
+template <bool CE, typename Kind, typename Cols>
+__device__ __forceinline__ bool linear_group(double Dm, Kind kind, double sgn, double t0_offset,
+                                             double fs, int win_lo, int win_len,
+                                             const LagrangeView &lg, Cols cols, double (&val)[3])
+{
+    constexpr int H = 13;
+    int d;
+    double e;
+    split_delay(Dm, t0_offset, fs, d, e);
+    const bool gbad = (d - win_lo - (H - 1) < 0) || (d - win_lo + H >= win_len);
+    if (gbad) d = win_lo + H - 1;  // in-window stand-in; the result is discarded
+    const int c0 = d - win_lo - (H - 1);  // lowest tap
+    using Taps = decltype(cols(0, kind, c0));
+    const Taps xr[3] = {cols(0, kind, c0), cols(1, kind, c0), cols(2, kind, c0)};
+    double S[3] = {0.0, 0.0, 0.0};
+    double P = 1.0;
+    const double D = e * (1.0 - e);
+#pragma unroll
+    for (int j = 1; j < H; ++j) {
+        const double Q = (double)(j * (j + 1)) + D;
+        const double EP = lagrange_E<CE>(lg, j - 1) * P;
+        const double eEP = e * EP;
+        // the pair's weights times E_{j-1} P_{j-1}, shared by the three outputs
+        const double wu = __builtin_fma((double)(j + 1), EP, -eEP);
+        const double wd = __builtin_fma((double)j, EP, eEP);
+#pragma unroll
+        for (int o = 0; o < 3; ++o) {
+            const Taps &x = xr[o];
+            const double num = __builtin_fma(x[H + j], wu, x[H - 1 - j] * wd);
+            S[o] = j == 1 ? num : __builtin_fma(S[o], Q, num);  // S_1 = n_1
+            pin(S[o]);
+        }
+        P = P * Q;
+        pin(P);
+        __asm__ volatile("" ::: "memory");
+    }
+    const double A = lagrange_A_fast(lg, e);
+    const double B = 1.0 - e;
+    const double invP = 1.0 / P;
+#pragma unroll
+    for (int o = 0; o < 3; ++o) {
+        const Taps &x = xr[o];  // x[H - 1] = sample d, x[H] = d + 1
+        const double v = A * __builtin_fma(D, S[o] * invP, __builtin_fma(B, x[H], e * x[H - 1]));
+        val[o] = gbad ? __builtin_nan("") : sgn * v;
+    }
+    return !gbad;
+}
+
 // Equal-arm stock TDI from the combined series (fast stencils): per chain length m one delay
-// t - m*L, one set of stencil weights and one stencil per output -- 3 stencils per group
-// instead of 6 units. Equal to the unit-by-unit sum up to rounding. Returns false if a stencil
-// fell outside the window (the outputs are NaN). The taps are read through
-// cols(o, kind, c0) -> a pointer p with p[k] = window column c0 + k of output o's series of
-// that kind (k = 0 .. 2H-1).
+// t - m*L and one stencil per output (linear_group) -- 3 stencils per group instead of 6 units.
+// Equal to the unit-by-unit sum up to rounding. Returns false if a stencil fell outside the window
+// (the outputs are NaN).
 template <int NX, bool CE = false, typename Cols>
 __device__ __forceinline__ bool tdi_linear_cols(double t, double L, double t0_offset, double fs,
                                                 int win_lo, int win_len, const LagrangeView &lg,
                                                 Cols cols, double (&acc)[3])
 {
-    constexpr int H = 13;
     constexpr int NG = stock::max_len(NX) + 1;
     bool ok = true;
     double Dm = t;
     static_for<NG>([&](auto m) {
         if constexpr (m > 0) Dm -= L;
-        int d;
-        double e;
-        split_delay(Dm, t0_offset, fs, d, e);
-        const bool gbad = (d - win_lo - (H - 1) < 0) || (d - win_lo + H >= win_len);
-        ok = ok && !gbad;
-        if (gbad) d = win_lo + H - 1;  // in-window stand-in; the result is discarded
-        constexpr int kind = stock::group_kind(m);
-        const int c0 = d - win_lo - (H - 1);  // lowest tap
-        using Taps = decltype(cols(0, kind, c0));
-        const Taps xr[3] = {cols(0, kind, c0), cols(1, kind, c0), cols(2, kind, c0)};
-        double S[3] = {0.0, 0.0, 0.0};
-        double P = 1.0;
-        const double D = e * (1.0 - e);
-#pragma unroll
-        for (int j = 1; j < H; ++j) {
-            const double Q = (double)(j * (j + 1)) + D;
-            const double EP = lagrange_E<CE>(lg, j - 1) * P;
-            const double eEP = e * EP;
-            // the pair's weights times E_{j-1} P_{j-1}, shared by the three outputs
-            const double wu = __builtin_fma((double)(j + 1), EP, -eEP);
-            const double wd = __builtin_fma((double)j, EP, eEP);
-#pragma unroll
-            for (int o = 0; o < 3; ++o) {
-                const Taps &x = xr[o];
-                const double num = __builtin_fma(x[H + j], wu, x[H - 1 - j] * wd);
-                S[o] = j == 1 ? num : __builtin_fma(S[o], Q, num);  // S_1 = n_1
-                pin(S[o]);
-            }
-            P = P * Q;
-            pin(P);
-            __asm__ volatile("" ::: "memory");
-        }
-        const double A = lagrange_A_fast(lg, e);
-        const double B = 1.0 - e;
-        const double invP = 1.0 / P;
-        constexpr double sgn = (double)stock::group_sign(m);
+        double val[3];
+        ok = linear_group<CE>(Dm, std::integral_constant<int, stock::group_kind(m)>{},
+                              (double)stock::group_sign(m), t0_offset, fs, win_lo, win_len, lg, cols,
+                              val) && ok;
 #pragma unroll
         for (int o = 0; o < 3; ++o) {
-            const Taps &x = xr[o];  // x[H - 1] = sample d, x[H] = d + 1
-            const double val = A * __builtin_fma(D, S[o] * invP, __builtin_fma(B, x[H], e * x[H - 1]));
-            acc[o] += gbad ? __builtin_nan("") : sgn * val;
+            acc[o] += val[o];
             pin(acc[o]);
         }
     });

@@ -19,7 +19,7 @@ LIB_PATH = os.path.join(LIB_DIR, "libflr_hip.so")
 
 SOURCES = ["flr_kernels.hip", "flr_fused_fp64.hip", "flr_fused_mixed.hip", "flr_fused_q31.hip",
            "flr_fused_c128.hip",
-           "flr_waveform.hip", "flr_pack.hip", "flr_capi.hip"]
+           "flr_waveform.hip", "flr_pack.hip", "flr_split.hip", "flr_capi.hip"]
 HEADERS = ["flr_internal.hpp", "flr_device.hpp", "flr_tdi_stock.hpp", "flr_paths.hpp", "flr_quotient.hpp",
            "flr_fused.hpp"]
 BUILD_DIR = os.path.join(LIB_DIR, "obj")
