@@ -62,15 +62,41 @@ struct PairDiv {
         return div_rcp(up, F, yF) + div_rcp(down, G, yG);
     }
 };
-template <>
-struct PairDiv<kExact2> {
+struct PairRecip {
     Recip rF, rG;
-    __device__ __forceinline__ PairDiv(double F, double G) { recip_pair(F, G, rF, rG); }
     __device__ __forceinline__ double sum(double up, double down) const
     {
         return div_recip(up, rF) + div_recip(down, rG);
     }
 };
+template <>
+struct PairDiv<kExact2> : PairRecip {
+    __device__ __forceinline__ PairDiv(double F, double G) { recip_pair(F, G, rF, rG); }
+};
+template <>
+struct PairDiv<kExact4> : PairRecip {
+    __device__ __forceinline__ PairDiv(double F, double G) { recip_pair(F, G, rF, rG); }
+};
+
+// f(j, q) for the tap pairs j = 1 .. H-1 in order, q their quotients at fraction e (exact forms;
+// kExact4: two pairs per hardware reciprocal).
+template <int FORM, int H, typename F>
+__device__ __forceinline__ void for_tap_pairs(double e, F &&f)
+{
+    if constexpr (FORM == kExact4) {
+        static_assert(H % 2 == 1, "an even number of tap pairs");
+#pragma unroll
+        for (int j = 1; j < H; j += 2) {
+            PairRecip a, b;
+            recip_quad(j + e, j + (1 - e), (j + 1) + e, (j + 1) + (1 - e), a.rF, a.rG, b.rF, b.rG);
+            f(j, a);
+            f(j + 1, b);
+        }
+    } else {
+#pragma unroll
+        for (int j = 1; j < H; ++j) f(j, PairDiv<FORM>(j + e, j + (1 - e)));
+    }
+}
 
 // ------------------------------------------------------------------ orbit interpolation
 // Uniform-grid linear interpolation of the orbit tables (the lisatools Orbits methods called
@@ -313,14 +339,19 @@ __device__ __forceinline__ double stencil_exact(const double *x, double e, const
     double C = e;
     double D = e * (1.0 - e);
     double sum = 0.0;
+    if constexpr (FORM == kExact4) {
+        for_tap_pairs<FORM, H>(
+            e, [&](int j, const auto &q) { sum += lg.E[j - 1] * q.sum(x[1 + j], x[-j]); });
+    } else {
 #pragma unroll kUnroll
-    for (int j = 1; j < h; j += 1) {
-        double E = lg.E[j - 1];
-        double F = j + e;
-        double G = j + (1 - e);
-        double up = x[1 + j];
-        double down = x[-j];
-        sum += E * PairDiv<FORM>(F, G).sum(up, down);
+        for (int j = 1; j < h; j += 1) {
+            double E = lg.E[j - 1];
+            double F = j + e;
+            double G = j + (1 - e);
+            double up = x[1 + j];
+            double down = x[-j];
+            sum += E * PairDiv<FORM>(F, G).sum(up, down);
+        }
     }
     return A * (B * x[1] + C * x[0] + D * sum);
 }

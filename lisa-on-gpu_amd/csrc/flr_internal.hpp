@@ -24,17 +24,21 @@ constexpr int kOrbitStride = 2 * kOrbitVals;
 // Stencil forms (flr_device.hpp). kFast: no per-tap divisions. kExact: the reference's operation
 // sequence, each quotient in three operations from its denominator's reciprocal. kExact2: the same
 // quotients, bit for bit, in two (div_recip) -- for stencils at sample positions of at least
-// exact2_min_position(h).
+// exact2_min_position(h). kExact4: kExact2 with the real stencils' reciprocals four at a time, from
+// exact4_min_position(h) on (the stock TDI tables and the fused FP64 kernels).
 constexpr int kFast = 0;
 constexpr int kExact = 1;
 constexpr int kExact2 = 2;
+constexpr int kExact4 = 3;
 
 // The form of a launch whose staged windows start at sample `lowest` or later: every stencil that
 // passes its window test sits at least h - 1 samples above its window's start.
-inline int stencil_form(bool exact, int64_t lowest, int h)
+// best: the form where it is proven, kExact2 or kExact4.
+inline int stencil_form(bool exact, int64_t lowest, int h, int best = kExact2)
 {
     if (!exact) return kFast;
-    return lowest + h - 1 >= exact2_min_position(h) ? kExact2 : kExact;
+    const int least = best == kExact4 ? exact4_min_position(h) : exact2_min_position(h);
+    return lowest + h - 1 >= least ? best : kExact;
 }
 
 // Device error word bits.

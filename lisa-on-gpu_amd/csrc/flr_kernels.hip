@@ -367,20 +367,24 @@ hipError_t launch_tdi(const TdiConfig &cfg, const TdiSource &src, const OrbitVie
 {
     const int nb = tiles_for(src.num_delays, src.start, cfg.zero_edges);
     const RowMap &rm = st.rows;
-    const int form = stencil_form(exact, (int64_t)src.start - cfg.halo_lo, lg.h);
+    const int64_t lowest = (int64_t)src.start - cfg.halo_lo;
     hipError_t err;
-    if (launch_tdi_split(cfg, src, orb, lg, form, st, stream, err)) return err;
-    return by_form(form, [&](auto form) {
-        constexpr int F = decltype(form)::value;
-        if (use_stock(st, lg)) {
-            const size_t shm = tdi_lds(cfg, true);
+    if (launch_tdi_split(cfg, src, orb, lg, stencil_form(exact, lowest, lg.h), st, stream, err))
+        return err;
+    if (use_stock(st, lg)) {
+        const size_t shm = tdi_lds(cfg, true);
+        return by_form<kExact4>(stencil_form(exact, lowest, lg.h, kExact4), [&](auto form) {
+            constexpr int F = decltype(form)::value;
 #define FLR_STOCK(NX, EQ) \
     launch(tdi_stock_kernel<NX, F, EQ>, nb, shm, stream, cfg, src, orb, lg, rm)
             if (st.equal_arm) return st.generation == 1 ? FLR_STOCK(8, true) : FLR_STOCK(16, true);
             return st.generation == 1 ? FLR_STOCK(8, false) : FLR_STOCK(16, false);
 #undef FLR_STOCK
-        }
-        const size_t shm = tdi_lds(cfg, false);
+        });
+    }
+    const size_t shm = tdi_lds(cfg, false);
+    return by_form(stencil_form(exact, lowest, lg.h), [&](auto form) {
+        constexpr int F = decltype(form)::value;
         if (lg.h == 13) return launch(tdi_kernel<F, 13>, nb, shm, stream, cfg, src, orb, lg);
         return launch(tdi_kernel<F, 0>, nb, shm, stream, cfg, src, orb, lg);
     });
@@ -392,17 +396,21 @@ hipError_t launch_tdi_batch(const TdiConfig &cfg, const Batch<TdiSource> &b, con
 {
     const int nb = batch_grid(b.total_tiles, grid_per_cu);
     const RowMap &rm = st.rows;
-    return by_form(stencil_form(exact, (int64_t)b.min_start - cfg.halo_lo, lg.h), [&](auto form) {
-        constexpr int F = decltype(form)::value;
-        if (use_stock(st, lg)) {
-            const size_t shm = tdi_lds(cfg, true);
+    const int64_t lowest = (int64_t)b.min_start - cfg.halo_lo;
+    if (use_stock(st, lg)) {
+        const size_t shm = tdi_lds(cfg, true);
+        return by_form<kExact4>(stencil_form(exact, lowest, lg.h, kExact4), [&](auto form) {
+            constexpr int F = decltype(form)::value;
 #define FLR_STOCK(NX, EQ) \
     launch(tdi_stock_batch_kernel<NX, F, EQ>, nb, shm, stream, cfg, b, orb, lg, rm)
             if (st.equal_arm) return st.generation == 1 ? FLR_STOCK(8, true) : FLR_STOCK(16, true);
             return st.generation == 1 ? FLR_STOCK(8, false) : FLR_STOCK(16, false);
 #undef FLR_STOCK
-        }
-        const size_t shm = tdi_lds(cfg, false);
+        });
+    }
+    const size_t shm = tdi_lds(cfg, false);
+    return by_form(stencil_form(exact, lowest, lg.h), [&](auto form) {
+        constexpr int F = decltype(form)::value;
         if (lg.h == 13) return launch(tdi_batch_kernel<F, 13>, nb, shm, stream, cfg, b, orb, lg);
         return launch(tdi_batch_kernel<F, 0>, nb, shm, stream, cfg, b, orb, lg);
     });

@@ -166,10 +166,8 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
         // j fully unrolled: every tap address is the unit's base plus an immediate offset (the
         // up/down pair of a unit loads with one ds_read2_b64); the memory barrier and the pins
         // at the end of each j keep its loads and arithmetic together.
-#pragma unroll
-        for (int j = 1; j < H; ++j) {
+        for_tap_pairs<EXACT, H>(e, [&](int j, const auto &q) {
             const double E = lg.E[j - 1];
-            const PairDiv<EXACT> q(j + e, j + (1 - e));
 #pragma unroll
             for (int c = 0; c < 3; ++c)
 #pragma unroll
@@ -181,7 +179,7 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
                 pin(S[c][1]);
             }
             __asm__ volatile("" ::: "memory");
-        }
+        });
         const double A = lagrange_A_exact(lg, e, y_deps);
         const double B = 1.0 - e;
         const double C = e;
@@ -226,8 +224,68 @@ __device__ __forceinline__ bool tdi_stock_unequal(double t, const double (&L)[6]
 {
     constexpr int H = 13;
     bool ok = true;
+    // Exact forms: the six undelayed units (terms 0 and 4 of every channel) share one fraction, so
+    // their tap pairs share their reciprocals, as a group of tdi_equal_arm; term 4 waits for its turn.
+    double undelayed[3] = {0.0, 0.0, 0.0};
+    if constexpr (EXACT) {
+        static_assert(stock::kX[0].len == 0 && stock::kX[4].len == 0, "the undelayed terms");
+        int d;
+        double e;
+        split_delay(t, t0_offset, fs, d, e);
+        const bool bad = (d - win_lo - (H - 1) < 0) || (d - win_lo + H >= win_len);
+        ok = ok && !bad;
+        const double *xr[3][2];
+        static_for<3>([&](auto c) {
+            static_for<2>([&](auto k) {
+                int off = rowoff[stock::base_of(c, 4 * k)] + (bad ? win_lo + H - 1 : d) - (H - 1);
+                pin(off);
+                xr[c][k] = ywin + off;
+            });
+        });
+        double S[3][2] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
+        for_tap_pairs<EXACT, H>(e, [&](int j, const auto &q) {
+            const double E = lg.E[j - 1];
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    S[c][k] += E * q.sum(xr[c][k][H + j], xr[c][k][H - 1 - j]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                pin(S[c][0]);
+                pin(S[c][1]);
+            }
+            __asm__ volatile("" ::: "memory");
+        });
+        const double A = lagrange_A_exact(lg, e, y_deps);
+        const double B = 1.0 - e;
+        const double C = e;
+        const double D = e * (1.0 - e);
+        static_for<3>([&](auto c) {
+            static_for<2>([&](auto k) {
+                const double *p = xr[c][k] + (H - 1);
+                double val = A * (B * p[1] + C * p[0] + D * S[c][k]);
+                val = bad ? __builtin_nan("") : val;
+                val *= (double)stock::kX[4 * k].sign;
+                if constexpr (k == 0) {
+                    acc[c] += val;
+                    pin(acc[c]);
+                } else {
+                    undelayed[c] = val;
+                    pin(undelayed[c]);
+                }
+            });
+        });
+        __asm__ volatile("" ::: "memory");
+    }
     static_for<3>([&](auto c) {
         static_for<NX>([&](auto x) {
+            if constexpr (EXACT != kFast && x == 0) return;
+            if constexpr (EXACT != kFast && x == 4) {
+                acc[c] += undelayed[c];
+                pin(acc[c]);
+                return;
+            }
             // a fresh copy of t per unit: its delay arithmetic cannot be hoisted above the
             // previous unit (which would keep every unit's split live at once)
             double delay = t;

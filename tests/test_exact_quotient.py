@@ -24,6 +24,23 @@ static thread_local double seed_error;
 #define FLR_RCP_SEED(x) ((1.0 / (x)) * (1.0 + seed_error))
 #include "flr_quotient.hpp"
 extern "C" int min_position(int h) { return flr::exact2_min_position(h); }
+extern "C" int min_position4(int h) { return flr::exact4_min_position(h); }
+// the same through recip_quad, each pair beside the one n/2 further on
+extern "C" long check4(const double *a, const double *F, const double *G, const double *err, long n)
+{
+    long wrong = 0;
+    for (long i = 0; i + n / 2 < n; ++i) {
+        seed_error = err[i];
+        const long k = i + n / 2;
+        flr::Recip f1, g1, f2, g2;
+        flr::recip_quad(F[i], G[i], F[k], G[k], f1, g1, f2, g2);
+        wrong += flr::div_recip(a[i], f1) != a[i] / F[i];
+        wrong += flr::div_recip(a[i], g1) != a[i] / G[i];
+        wrong += flr::div_recip(a[k], f2) != a[k] / F[k];
+        wrong += flr::div_recip(a[k], g2) != a[k] / G[k];
+    }
+    return wrong;
+}
 // wrong[0]: quotients of div_recip that differ from a / b; wrong[1]: those of y a alone
 extern "C" void check(const double *a, const double *F, const double *G, const double *err, long n,
                       long *wrong)
@@ -62,6 +79,13 @@ def _check(lib, a, F, G, err):
     return wrong[0], wrong[1]
 
 
+def _check4(lib, a, F, G, err):
+    a, F, G, err = (np.ascontiguousarray(x, dtype=np.float64) for x in (a, F, G, err))
+    lib.check4.restype = ctypes.c_long
+    return lib.check4(*(ctypes.c_void_p(x.ctypes.data) for x in (a, F, G, err)),
+                      ctypes.c_long(len(a)))
+
+
 def _denominators(rng, h, pos, n):
     """j + e, j + (1 - e) for j = 1 .. h-1 and e a multiple of ulp(pos) = 2^(log2(pos) - 52)."""
     bits = 52 - (pos.bit_length() - 1)
@@ -82,13 +106,18 @@ def test_random_numerators(lib, h):
     two_ops, one_op = _check(lib, a, F, G, err)
     assert two_ops == 0
     assert one_op > n // 20  # the test can tell
+    if h <= 14:  # the form of four at a time, from its own least position
+        F, G, _ = _denominators(rng, h, lib.min_position4(h), n)
+        assert _check4(lib, a, F, G, err) == 0
+    else:
+        assert lib.min_position4(h) > 1 << 29  # never used
 
 
-@pytest.mark.parametrize("h", [13, 16, 20])
-def test_hardest_numerators(lib, h):
+@pytest.mark.parametrize("h,four", [(13, False), (16, False), (20, False), (13, True)])
+def test_hardest_numerators(lib, h, four):
     rng = np.random.default_rng(100 + h)
     n = 20_000
-    F, _, bits = _denominators(rng, h, lib.min_position(h), n)
+    F, _, bits = _denominators(rng, h, (lib.min_position4 if four else lib.min_position)(h), n)
     a, Fk, Gk = [], [], []
     for f in F:
         B = int(f * 2.0 ** bits)
@@ -113,5 +142,8 @@ def test_hardest_numerators(lib, h):
             Gk.append(2.0 * np.floor(f) + 1.0 - f)
     assert len(a) > 2000
     err = rng.uniform(-1, 1, len(a)) * 2.0 ** -22
+    if four:
+        assert _check4(lib, np.array(a), np.array(Fk), np.array(Gk), err) == 0
+        return
     two_ops, _ = _check(lib, np.array(a), np.array(Fk), np.array(Gk), err)
     assert two_ops == 0

@@ -46,17 +46,22 @@ def test_projection_either_side_of_the_limit(gpu, orbits, oracle_orbits, oracle_
 @pytest.mark.parametrize("order,tdi", [(25, "1st generation"), (25, "2nd generation"), (25, CUSTOM),
                                        (31, "1st generation"), (35, CUSTOM)])
 @pytest.mark.parametrize("side", [-1, 0])
-def test_tdi_either_side_of_the_limit(gpu, orbits, oracle_orbits, oracle_mod, order, tdi, side):
+@pytest.mark.parametrize("limit,n", [(None, 1601), (512, 2501), (512, 170_001)])
+def test_tdi_either_side_of_the_limit(gpu, orbits, oracle_orbits, oracle_mod, order, tdi, side, limit,
+                                      n):
     import torch
     from fastlisaresponse_amd import _capi
     ow, rw, (A, deps, E), tabs = _setup(gpu, orbits, order=order, tdi=tdi)
-    n, dt, h, t0 = 1601, 10.0, (order + 1) // 2, 0.0
+    dt, h, t0 = 10.0, (order + 1) // 2, 0.0
+    limit = limit or _limit(h)
     chain = {"1st generation": 3, "2nd generation": 7}.get(tdi, 2) if isinstance(tdi, str) else 2
     halo_lo = math.ceil(chain * ow.extent()[1] / dt) + h + 4
-    T = _limit(h) + halo_lo - (h - 1) + side
+    # the stock tables at order 25 also change form at 512 (four reciprocals at a time); long enough
+    # a series for the one-lane kernels
+    T = limit + halo_lo - (h - 1) + side
     y = np.random.default_rng(order + side).standard_normal((6, n))
     exp = oracle_mod.get_tdi_delays(oracle_orbits, y, t0 + np.arange(n) * dt, _oracle_tables(tabs),
-                                    order, 1 / dt, A, deps, E, T, 4)
+                                    order, 1 / dt, A, deps, E, T, 16)
     out = torch.zeros(3 * n, dtype=torch.float64, device="cuda")
     rw.tdi(out, torch.as_tensor(y.reshape(-1), device="cuda"), n, t0, dt, 1 / dt, T,
            _capi.FLR_FLAG_OVERWRITE | _capi.FLR_FLAG_ZERO_EDGES | _capi.FLR_FLAG_EXACT)
