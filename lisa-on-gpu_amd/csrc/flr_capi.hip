@@ -351,7 +351,6 @@ int set_tdi_impl(flr_response *r, const int32_t *unit_starts, const int32_t *uni
     return FLR_OK;
 }
 
-constexpr size_t kMaxLds = 160 * 1024;
 
 // Launch configuration shared by all sources of a projection launch: receiver/emitter rows,
 // and halos sized from the orbit extent (max |x|/c and max light travel time).

@@ -559,11 +559,8 @@ __device__ __forceinline__ void fused_tile(const ProjConfig &pc, const TdiConfig
         } else {
             const double L = orbit_val(orbit_node<EXACT>(orb, t), rm.row[0]);
             if constexpr (MODE == kModeGroups) {
-                int rowoff[6];
-#pragma unroll
-                for (int k = 0; k < 6; ++k) rowoff[k] = rm.row[k] * cap - yw_lo;
-                bad |= !tdi_equal_arm<NX, EXACT>(t, L, t0_offset, tc.fs, ywin, rowoff, yw_lo,
-                                                 yw_len, lg, y_deps, acc);
+                bad |= !tdi_equal_arm_rows<NX, EXACT>(t, L, t0_offset, tc.fs, ywin, cap, rm, yw_lo,
+                                                      yw_len, lg, y_deps, acc);
             } else {
                 bad |= !tdi_linear<NX, true>(t, L, t0_offset, tc.fs, ywin, cap, yw_lo, yw_len, lg,
                                              acc);

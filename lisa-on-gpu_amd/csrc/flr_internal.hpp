@@ -192,6 +192,9 @@ struct FusedSource {
     double k[3], u[3], v[3];
 };
 
+// LDS a workgroup may take.
+constexpr size_t kMaxLds = 160 * 1024;
+
 // Static LDS of a mixed matrix-core kernel at most: the E and orbit-node copies, the unit model of
 // the unequal-arm form, the inner-product slots.
 constexpr size_t kFusedStaticLds = 6656;

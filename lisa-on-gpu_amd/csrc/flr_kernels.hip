@@ -85,10 +85,15 @@ __device__ __forceinline__ void tdi_store(const TdiConfig &cfg, const TdiSource 
     }
 }
 
-// Zero the tile's edge samples if asked, check and stage the y window -- the six rows, or (LINEAR)
-// the combined series of the equal-arm fast form in their place (rm: canonical links to rows).
+// What the y window in LDS holds: the six rows (read by tdi_units, tdi_stock_unequal or, kEqualRows,
+// tdi_equal_arm_rows), the six paired rows of tdi_equal_arm_pairs or the combined series of
+// tdi_linear_packed.
+enum WindowLayout { kRows, kEqualRows, kPairs, kPacked };
+
+// Zero the tile's edge samples if asked, check and stage the y window (rm: canonical links to rows, for
+// kPairs and kPacked).
 // Returns false when the tile has nothing (more) to do; every lane returns the same value.
-template <bool LINEAR = false>
+template <WindowLayout LAYOUT = kRows>
 __device__ __forceinline__ bool tdi_stage(const TdiConfig &cfg, const TdiSource &src,
                                           const TileRange &tr, int i, bool valid, double *ywin,
                                           int &win_lo, int &win_len,
@@ -109,18 +114,18 @@ __device__ __forceinline__ bool tdi_stage(const TdiConfig &cfg, const TdiSource 
         }
         return false;
     }
-    if constexpr (LINEAR) {
+    if constexpr (LAYOUT == kPairs || LAYOUT == kPacked) {
         const double *from = src.y + win_lo;
+        double2 *pairs = reinterpret_cast<double2 *>(ywin);
+        double *z = ywin + 4 * cfg.win_cap;  // kPacked, after the two rows of double2
         for (int jj = threadIdx.x; jj < win_len; jj += kBlock) {
-            double y[kNLinks], k[2][3];
+            double y[kNLinks];
 #pragma unroll
             for (int l = 0; l < kNLinks; ++l) y[l] = from[(size_t)rm->row[l] * src.num_inputs + jj];
-            combine_links(y, k);
-#pragma unroll
-            for (int o = 0; o < 3; ++o) {
-                ywin[(2 * o) * cfg.win_cap + jj] = k[0][o];
-                ywin[(2 * o + 1) * cfg.win_cap + jj] = k[1][o];
-            }
+            if constexpr (LAYOUT == kPairs)
+                store_link_pairs(pairs + jj, cfg.win_cap, y);
+            else
+                store_packed_series(pairs + jj, z + jj, cfg.win_cap, y);
         }
         return true;
     }
@@ -176,10 +181,14 @@ __device__ __forceinline__ void tdi_tile(const TdiConfig &cfg, const TdiSource &
 // (fast form) are shared by the units of that length -- 8 groups instead of 48 units for 2nd
 // generation, with bit-identical results. The fast form goes further: by linearity the two units of
 // each chain length and channel become one stencil of a combined series (tdi_linear), formed while
-// the window is staged -- 24 stencils instead of 48, half the LDS reads. FP64-bound: its TDI launch over
-// 1,000,003 samples takes 96 us instead of 183 (MI355X, 2nd generation).
+// the window is staged -- 24 stencils instead of 48, half the LDS reads: 1,000,003 samples, 2nd
+// generation, 183 -> 96 us (MI355X).
+// Bound by the FP64 pipes and, beside them, LDS reads (a ds_read2_b64 returns 125 bytes per clock and
+// CU, a ds_read_b128 239), so the taps that are read together lie together: the two links of a channel
+// (exact forms, paired rows: each link twice, 28 KB a tile at dt = 10 s), or X and Y (fast form). The same
+// bits; 1,048,577 samples, 2nd generation: exact 225.6 -> 213.9 us, fast 96.2 -> 84.4 us.
 
-template <int NX, int EXACT, bool EQ>
+template <int NX, int EXACT, WindowLayout LAYOUT>
 __device__ __forceinline__ void tdi_stock_tile(const TdiConfig &cfg, const TdiSource &src,
                                                int tile, const OrbitView &orb,
                                                const LagrangeView &lg, const RowMap &rm,
@@ -189,8 +198,7 @@ __device__ __forceinline__ void tdi_stock_tile(const TdiConfig &cfg, const TdiSo
     const int i = tr.i0 + (int)threadIdx.x;
     const bool valid = (i >= tr.lo_valid) && (i < tr.hi_valid);
     int win_lo = 0, win_len = 0;
-    constexpr bool kLinear = EQ && !EXACT;
-    if (!tdi_stage<kLinear>(cfg, src, tr, i, valid, ywin, win_lo, win_len, &rm)) return;
+    if (!tdi_stage<LAYOUT>(cfg, src, tr, i, valid, ywin, win_lo, win_len, &rm)) return;
 
     const int ic = valid ? i : tr.first;
     const double t = src.t_arr ? src.t_arr[ic] : src.t0 + (double)ic * cfg.dt;
@@ -199,9 +207,6 @@ __device__ __forceinline__ void tdi_stock_tile(const TdiConfig &cfg, const TdiSo
     double L[6];
 #pragma unroll
     for (int k = 0; k < 6; ++k) L[k] = orbit_val(nd, rm.row[k]);
-    int rowoff[6];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) rowoff[k] = rm.row[k] * cfg.win_cap - win_lo;
     __syncthreads();
     if (!valid) return;
     const double y_deps = EXACT ? rcp_nr2(lg.deps) : 0.0;
@@ -211,14 +216,23 @@ __device__ __forceinline__ void tdi_stock_tile(const TdiConfig &cfg, const TdiSo
     for (int c = 0; c < 3; ++c)
         acc[c] = cfg.overwrite ? 0.0 : src.out[(size_t)c * src.num_delays + i];
     bool ok;
-    if constexpr (kLinear)
-        ok = tdi_linear<NX>(t, L[0], t0_offset, cfg.fs, ywin, cfg.win_cap, win_lo, win_len, lg, acc);
-    else if constexpr (EQ)
-        ok = tdi_equal_arm<NX, EXACT>(t, L[0], t0_offset, cfg.fs, ywin, rowoff, win_lo, win_len, lg,
-                                      y_deps, acc);
-    else
+    const double2 *pairs = reinterpret_cast<const double2 *>(ywin);
+    if constexpr (LAYOUT == kPacked) {
+        ok = tdi_linear_packed<NX>(t, L[0], t0_offset, cfg.fs, pairs, cfg.win_cap, win_lo, win_len, lg,
+                                   acc);
+    } else if constexpr (LAYOUT == kEqualRows) {
+        ok = tdi_equal_arm_rows<NX, EXACT>(t, L[0], t0_offset, cfg.fs, ywin, cfg.win_cap, rm, win_lo,
+                                           win_len, lg, y_deps, acc);
+    } else if constexpr (LAYOUT == kPairs) {
+        ok = tdi_equal_arm_pairs<NX, EXACT>(t, L[0], t0_offset, cfg.fs, pairs, cfg.win_cap, win_lo,
+                                            win_len, lg, y_deps, acc);
+    } else {
+        int rowoff[6];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) rowoff[k] = rm.row[k] * cfg.win_cap - win_lo;
         ok = tdi_stock_unequal<NX, EXACT>(t, L, t0_offset, cfg.fs, ywin, rowoff, win_lo, win_len,
                                           lg, y_deps, acc);
+    }
     if (!ok) atomicOr(cfg.err, kErrWindow);
     tdi_store(cfg, src, i, acc);
 }
@@ -258,23 +272,23 @@ __global__ __launch_bounds__(kBlock) void tdi_batch_kernel(TdiConfig cfg, Batch<
     FLR_BATCH_LOOP(batch, (tdi_tile<EXACT, H>(cfg, src, tile, orb, lg, smem)));
 }
 
-template <int NX, int EXACT, bool EQ>
+template <int NX, int EXACT, WindowLayout LAYOUT>
 __global__ __launch_bounds__(kBlock) void tdi_stock_kernel(TdiConfig cfg, TdiSource src,
                                                                OrbitView orb, LagrangeView lg,
                                                                RowMap rm)
 {
-    extern __shared__ double smem[];
-    tdi_stock_tile<NX, EXACT, EQ>(cfg, src, blockIdx.x, orb, lg, rm, smem);
+    extern __shared__ __align__(16) double smem[];
+    tdi_stock_tile<NX, EXACT, LAYOUT>(cfg, src, blockIdx.x, orb, lg, rm, smem);
 }
 
-template <int NX, int EXACT, bool EQ>
+template <int NX, int EXACT, WindowLayout LAYOUT>
 __global__ __launch_bounds__(kBlock) void tdi_stock_batch_kernel(TdiConfig cfg,
                                                                      Batch<TdiSource> batch,
                                                                      OrbitView orb,
                                                                      LagrangeView lg, RowMap rm)
 {
-    extern __shared__ double smem[];
-    FLR_BATCH_LOOP(batch, (tdi_stock_tile<NX, EXACT, EQ>(cfg, src, tile, orb, lg, rm, smem)));
+    extern __shared__ __align__(16) double smem[];
+    FLR_BATCH_LOOP(batch, (tdi_stock_tile<NX, EXACT, LAYOUT>(cfg, src, tile, orb, lg, rm, smem)));
 }
 
 // ------------------------------------------------------------------ small kernels
@@ -362,6 +376,27 @@ static size_t tdi_lds(const TdiConfig &cfg, bool stock)
     return ((size_t)kNLinks * cfg.win_cap + (stock ? 0 : (size_t)kNLinks * kBlock)) * sizeof(double);
 }
 
+// The stock tables' kernel: f(form, layout, LDS bytes). Equal arms in the exact forms read paired rows
+// while the window fits (windows of up to 1706 samples; the limit of rows is 3157). Paired rows are the
+// better at every window that fits, if only one workgroup does: 500,000 samples, 2nd generation,
+// dt = 2 s (352 samples) 123.7 -> 115.6 us, dt = 0.2 s (616 samples) 111.2 -> 105.0 us.
+template <typename F>
+static hipError_t by_stock_layout(const TdiConfig &cfg, bool exact, int64_t lowest,
+                                  const LagrangeView &lg, bool equal_arm, F &&f)
+{
+    const size_t rows = tdi_lds(cfg, true), pairs = 2 * rows;
+    using std::integral_constant;
+    if (equal_arm && exact && pairs > kMaxLds)
+        return f(integral_constant<int, kExact>{}, integral_constant<WindowLayout, kEqualRows>{}, rows);
+    return by_form<kExact4>(stencil_form(exact, lowest, lg.h, kExact4), [&](auto form) {
+        constexpr int F_ = decltype(form)::value;
+        if (equal_arm)
+            return f(form, integral_constant<WindowLayout, F_ == kFast ? kPacked : kPairs>{},
+                     F_ == kFast ? rows : pairs);
+        return f(form, integral_constant<WindowLayout, kRows>{}, rows);
+    });
+}
+
 hipError_t launch_tdi(const TdiConfig &cfg, const TdiSource &src, const OrbitView &orb,
                       const LagrangeView &lg, bool exact, const StockTdi &st, hipStream_t stream)
 {
@@ -372,14 +407,12 @@ hipError_t launch_tdi(const TdiConfig &cfg, const TdiSource &src, const OrbitVie
     if (launch_tdi_split(cfg, src, orb, lg, stencil_form(exact, lowest, lg.h), st, stream, err))
         return err;
     if (use_stock(st, lg)) {
-        const size_t shm = tdi_lds(cfg, true);
-        return by_form<kExact4>(stencil_form(exact, lowest, lg.h, kExact4), [&](auto form) {
+        return by_stock_layout(cfg, exact, lowest, lg, st.equal_arm, [&](auto form, auto layout, size_t shm) {
             constexpr int F = decltype(form)::value;
-#define FLR_STOCK(NX, EQ) \
-    launch(tdi_stock_kernel<NX, F, EQ>, nb, shm, stream, cfg, src, orb, lg, rm)
-            if (st.equal_arm) return st.generation == 1 ? FLR_STOCK(8, true) : FLR_STOCK(16, true);
-            return st.generation == 1 ? FLR_STOCK(8, false) : FLR_STOCK(16, false);
-#undef FLR_STOCK
+            constexpr WindowLayout W = decltype(layout)::value;
+            return st.generation == 1
+                       ? launch(tdi_stock_kernel<8, F, W>, nb, shm, stream, cfg, src, orb, lg, rm)
+                       : launch(tdi_stock_kernel<16, F, W>, nb, shm, stream, cfg, src, orb, lg, rm);
         });
     }
     const size_t shm = tdi_lds(cfg, false);
@@ -398,14 +431,12 @@ hipError_t launch_tdi_batch(const TdiConfig &cfg, const Batch<TdiSource> &b, con
     const RowMap &rm = st.rows;
     const int64_t lowest = (int64_t)b.min_start - cfg.halo_lo;
     if (use_stock(st, lg)) {
-        const size_t shm = tdi_lds(cfg, true);
-        return by_form<kExact4>(stencil_form(exact, lowest, lg.h, kExact4), [&](auto form) {
+        return by_stock_layout(cfg, exact, lowest, lg, st.equal_arm, [&](auto form, auto layout, size_t shm) {
             constexpr int F = decltype(form)::value;
-#define FLR_STOCK(NX, EQ) \
-    launch(tdi_stock_batch_kernel<NX, F, EQ>, nb, shm, stream, cfg, b, orb, lg, rm)
-            if (st.equal_arm) return st.generation == 1 ? FLR_STOCK(8, true) : FLR_STOCK(16, true);
-            return st.generation == 1 ? FLR_STOCK(8, false) : FLR_STOCK(16, false);
-#undef FLR_STOCK
+            constexpr WindowLayout W = decltype(layout)::value;
+            return st.generation == 1
+                       ? launch(tdi_stock_batch_kernel<8, F, W>, nb, shm, stream, cfg, b, orb, lg, rm)
+                       : launch(tdi_stock_batch_kernel<16, F, W>, nb, shm, stream, cfg, b, orb, lg, rm);
         });
     }
     const size_t shm = tdi_lds(cfg, false);

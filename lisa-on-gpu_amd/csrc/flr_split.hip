@@ -282,12 +282,7 @@ __global__ __launch_bounds__(kSplit *(stock::max_len(NX) + 1)) void tdi_split_eq
         double val[3];
         bad = !linear_group<false>(Dm, kind, (kNegative >> m) & 1 ? -1.0 : 1.0, st.t0_offset, cfg.fs,
                                    st.win_lo, st.win_len, lg,
-                                   [&](int o, int kd, int c0) {
-                                       int off = (2 * o + kd) * cap + c0;
-                                       pin(off);
-                                       return ywin + off;
-                                   },
-                                   val);
+                                   [&](int kd, int c0) { return row_taps(ywin, cap, kd, c0); }, val);
 #pragma unroll
         for (int o = 0; o < 3; ++o) vals[(o * kVals + m) * kSplit + lane] = val[o];
     }

@@ -85,6 +85,13 @@ constexpr int group_sign(int m)
 {
     return pair_sign(m, 13, 12) != 0 ? pair_sign(m, 13, 12) : pair_sign(m, 31, 21);
 }
+// The two units of chain length m and one channel: slot 0 of links 13 (m even) and 31 (odd), slot 1
+// of 12 and 21, cyclically shifted for Y and Z.
+constexpr int slot_of(int x) { return kX[x].link == 13 || kX[x].link == 31 ? 0 : 1; }
+constexpr int slot_row(int c, int kind, int slot)
+{
+    return canon(cyc(kind == 0 ? (slot == 0 ? 13 : 12) : (slot == 0 ? 31 : 21), c));
+}
 static_assert(group_sign(0) != 0 && group_sign(1) != 0 && group_sign(2) != 0 &&
                   group_sign(3) != 0 && group_sign(4) != 0 && group_sign(5) != 0 &&
                   group_sign(6) != 0 && group_sign(7) != 0,
@@ -126,12 +133,13 @@ constexpr int done_prefix(int nx, int m)
 // units of that chain length (2 per channel) share one fraction, i.e. one set of per-tap
 // reciprocals. Per unit the tap sum runs over j in the reference's order, and units are added to
 // their channel sum in index order (exact forms; the fast form is tdi_linear).
-// Returns false if a stencil fell outside the window (the affected outputs are NaN).
-template <int NX, int EXACT>
+// Returns false if a stencil fell outside the window (the affected outputs are NaN). The taps are
+// read through cols(c, kind, c0) -> a p with p[k] = window column c0 + k of channel c's two links of
+// that kind (slot 0 in .x, 1 in .y).
+template <int NX, int EXACT, typename Cols>
 __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offset, double fs,
-                                              const double *ywin, const int (&rowoff)[6],
                                               int win_lo, int win_len, const LagrangeView &lg,
-                                              double y_deps, double (&acc)[3])
+                                              double y_deps, Cols cols, double (&acc)[3])
 {
     static_assert(EXACT != kFast, "the fast form merges the units of a chain length (tdi_linear)");
     constexpr int H = 13;
@@ -148,31 +156,25 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
         ok = ok && !gbad;
         if (gbad) d = win_lo + H - 1;  // in-window stand-in; the result is discarded
 
-        // the units of this group: (c, x) with len(x) == m, two per channel
-        const double *xr[3][2];
-        static_for<3>([&](auto c) {
-            int k = 0;
-            static_for<NX>([&](auto x) {
-                // based at the lowest tap x[d - (H-1)], so every tap is a non-negative immediate
-                // offset; the pinned index keeps the compiler from choosing another base
-                if constexpr (stock::kX[x].len == m) {
-                    int off = rowoff[stock::base_of(c, x)] + d - (H - 1);
-                    pin(off);
-                    xr[c][k++] = ywin + off;
-                }
-            });
-        });
+        // the units of this group: two per channel, from the lowest tap x[d - (H-1)] on
+        using kind = std::integral_constant<int, stock::group_kind(m)>;
+        using Taps = decltype(cols(std::integral_constant<int, 0>{}, kind{}, 0));
+        const int c0 = d - win_lo - (H - 1);
+        const Taps xr[3] = {cols(std::integral_constant<int, 0>{}, kind{}, c0),
+                            cols(std::integral_constant<int, 1>{}, kind{}, c0),
+                            cols(std::integral_constant<int, 2>{}, kind{}, c0)};
         double S[3][2] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
-        // j fully unrolled: every tap address is the unit's base plus an immediate offset (the
-        // up/down pair of a unit loads with one ds_read2_b64); the memory barrier and the pins
-        // at the end of each j keep its loads and arithmetic together.
+        // j fully unrolled: every tap address is the channel's base plus an immediate offset;
+        // the memory barrier and the pins at the end of each j keep its loads and arithmetic
+        // together.
         for_tap_pairs<EXACT, H>(e, [&](int j, const auto &q) {
             const double E = lg.E[j - 1];
 #pragma unroll
-            for (int c = 0; c < 3; ++c)
-#pragma unroll
-                for (int k = 0; k < 2; ++k)
-                    S[c][k] += E * q.sum(xr[c][k][H + j], xr[c][k][H - 1 - j]);
+            for (int c = 0; c < 3; ++c) {
+                const double2 up = xr[c][H + j], dn = xr[c][H - 1 - j];
+                S[c][0] += E * q.sum(up.x, dn.x);
+                S[c][1] += E * q.sum(up.y, dn.y);
+            }
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 pin(S[c][0]);
@@ -185,15 +187,14 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
         const double C = e;
         const double D = e * (1.0 - e);
         static_for<3>([&](auto c) {
-            int k = 0;
+            const double2 x0 = xr[c][H - 1], x1 = xr[c][H];  // samples d and d + 1
             static_for<NX>([&](auto x) {
                 if constexpr (stock::kX[x].len == m) {
-                    const double *p = xr[c][k] + (H - 1);  // p[0] = x[d], p[1] = x[d+1]
-                    double val = A * (B * p[1] + C * p[0] + D * S[c][k]);
+                    constexpr int k = stock::slot_of(x);
+                    double val = A * (B * (k ? x1.y : x1.x) + C * (k ? x0.y : x0.x) + D * S[c][k]);
                     val *= (double)stock::kX[x].sign;
                     v[c][x] = gbad ? __builtin_nan("") : val;
                     pin(v[c][x]);
-                    ++k;
                 }
             });
         });
@@ -208,6 +209,57 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
         });
     });
     return ok;
+}
+
+// Column k of two rows of doubles, as one value.
+struct RowPair {
+    const double *p0, *p1;
+    __device__ __forceinline__ double2 operator[](int k) const { return {p0[k], p1[k]}; }
+};
+
+// tdi_equal_arm on contiguous rows of pitch cap, link k (canonical order) in row row[k]. The pinned
+// index keeps the compiler from choosing another base.
+template <int NX, int EXACT>
+__device__ __forceinline__ bool tdi_equal_arm_rows(double t, double L, double t0_offset, double fs,
+                                                   const double *ywin, int cap, const RowMap &rm,
+                                                   int win_lo, int win_len, const LagrangeView &lg,
+                                                   double y_deps, double (&acc)[3])
+{
+    return tdi_equal_arm<NX, EXACT>(t, L, t0_offset, fs, win_lo, win_len, lg, y_deps,
+                                    [&](auto c, auto kind, int c0) {
+                                        int o0 = rm.row[stock::slot_row(c, kind, 0)] * cap + c0;
+                                        int o1 = rm.row[stock::slot_row(c, kind, 1)] * cap + c0;
+                                        pin(o0);
+                                        pin(o1);
+                                        return RowPair{ywin + o0, ywin + o1};
+                                    },
+                                    acc);
+}
+
+// The six paired rows of tdi_equal_arm_pairs: row 2 c + kind holds {slot 0, slot 1} of the six links y.
+__device__ __forceinline__ void store_link_pairs(double2 *col, int cap, const double (&y)[6])
+{
+    static_for<3>([&](auto c) {
+        static_for<2>([&](auto kind) {
+            col[(2 * c + kind) * cap] = {y[stock::slot_row(c, kind, 0)], y[stock::slot_row(c, kind, 1)]};
+        });
+    });
+}
+
+// tdi_equal_arm on paired rows: one ds_read_b128 per tap and channel.
+template <int NX, int EXACT>
+__device__ __forceinline__ bool tdi_equal_arm_pairs(double t, double L, double t0_offset, double fs,
+                                                    const double2 *pairs, int cap, int win_lo,
+                                                    int win_len, const LagrangeView &lg,
+                                                    double y_deps, double (&acc)[3])
+{
+    return tdi_equal_arm<NX, EXACT>(t, L, t0_offset, fs, win_lo, win_len, lg, y_deps,
+                                    [&](auto c, auto kind, int c0) {
+                                        int off = (2 * c + kind) * cap + c0;
+                                        pin(off);
+                                        return pairs + off;
+                                    },
+                                    acc);
 }
 
 // Stock TDI for one sample with arbitrary (unequal) light travel times L[k] (canonical link
@@ -352,10 +404,15 @@ __device__ __forceinline__ void linear_series(double *yc, int cap, const RowMap 
     }
 }
 
+// One window column of the three outputs' combined series.
+struct Tap3 {
+    double v[3];
+};
+
 // One chain length of the equal-arm stock TDI from the combined series (fast stencils): at delay Dm
 // one set of stencil weights and one stencil per output, times sgn, into val (NaN, and false, if a
-// stencil fell outside the window). The taps are read through cols(o, kind, c0) -> a pointer p with
-// p[k] = window column c0 + k of output o's series of that kind (k = 0 .. 2H-1).
+// stencil fell outside the window). The taps are read through cols(kind, c0) -> a p with p(k) = window
+// column c0 + k of the three outputs' series of that kind (k = 0 .. 2H-1).
 template <bool CE, typename Kind, typename Cols>
 __device__ __forceinline__ bool linear_group(double Dm, Kind kind, double sgn, double t0_offset,
                                              double fs, int win_lo, int win_len,
@@ -368,8 +425,7 @@ __device__ __forceinline__ bool linear_group(double Dm, Kind kind, double sgn, d
     const bool gbad = (d - win_lo - (H - 1) < 0) || (d - win_lo + H >= win_len);
     if (gbad) d = win_lo + H - 1;  // in-window stand-in; the result is discarded
     const int c0 = d - win_lo - (H - 1);  // lowest tap
-    using Taps = decltype(cols(0, kind, c0));
-    const Taps xr[3] = {cols(0, kind, c0), cols(1, kind, c0), cols(2, kind, c0)};
+    const auto taps = cols(kind, c0);
     double S[3] = {0.0, 0.0, 0.0};
     double P = 1.0;
     const double D = e * (1.0 - e);
@@ -381,10 +437,10 @@ __device__ __forceinline__ bool linear_group(double Dm, Kind kind, double sgn, d
         // the pair's weights times E_{j-1} P_{j-1}, shared by the three outputs
         const double wu = __builtin_fma((double)(j + 1), EP, -eEP);
         const double wd = __builtin_fma((double)j, EP, eEP);
+        const Tap3 up = taps(H + j), dn = taps(H - 1 - j);
 #pragma unroll
         for (int o = 0; o < 3; ++o) {
-            const Taps &x = xr[o];
-            const double num = __builtin_fma(x[H + j], wu, x[H - 1 - j] * wd);
+            const double num = __builtin_fma(up.v[o], wu, dn.v[o] * wd);
             S[o] = j == 1 ? num : __builtin_fma(S[o], Q, num);  // S_1 = n_1
             pin(S[o]);
         }
@@ -395,10 +451,11 @@ __device__ __forceinline__ bool linear_group(double Dm, Kind kind, double sgn, d
     const double A = lagrange_A_fast(lg, e);
     const double B = 1.0 - e;
     const double invP = 1.0 / P;
+    const Tap3 x0 = taps(H - 1), x1 = taps(H);  // samples d and d + 1
 #pragma unroll
     for (int o = 0; o < 3; ++o) {
-        const Taps &x = xr[o];  // x[H - 1] = sample d, x[H] = d + 1
-        const double v = A * __builtin_fma(D, S[o] * invP, __builtin_fma(B, x[H], e * x[H - 1]));
+        const double v =
+            A * __builtin_fma(D, S[o] * invP, __builtin_fma(B, x1.v[o], e * x0.v[o]));
         val[o] = gbad ? __builtin_nan("") : sgn * v;
     }
     return !gbad;
@@ -431,18 +488,65 @@ __device__ __forceinline__ bool tdi_linear_cols(double t, double L, double t0_of
     return ok;
 }
 
-// Contiguous rows of pitch cap: every tap at a non-negative immediate offset from one pinned
-// base address per output.
+// Contiguous rows of pitch cap (row 2 o + kind): every tap at a non-negative immediate offset from
+// one pinned base address per output.
+struct RowTaps {
+    const double *p[3];
+    __device__ __forceinline__ Tap3 operator()(int k) const { return {{p[0][k], p[1][k], p[2][k]}}; }
+};
+__device__ __forceinline__ RowTaps row_taps(const double *ywin, int cap, int kind, int c0)
+{
+    int o[3] = {kind * cap + c0, (2 + kind) * cap + c0, (4 + kind) * cap + c0};
+    pin(o[0]);
+    pin(o[1]);
+    pin(o[2]);
+    return {{ywin + o[0], ywin + o[1], ywin + o[2]}};
+}
+
 template <int NX, bool CE = false>
 __device__ __forceinline__ bool tdi_linear(double t, double L, double t0_offset, double fs,
                                            const double *ywin, int cap, int win_lo, int win_len,
                                            const LagrangeView &lg, double (&acc)[3])
 {
     return tdi_linear_cols<NX, CE>(t, L, t0_offset, fs, win_lo, win_len, lg,
-                               [&](int o, int kind, int c0) {
-                                   int off = (2 * o + kind) * cap + c0;
+                               [&](int kind, int c0) { return row_taps(ywin, cap, kind, c0); }, acc);
+}
+
+// The combined series as the unfused kernel holds them: {X, Y} of kinds 0 and 1 in two rows of double2,
+// then Z of each in rows of doubles (all of pitch cap).
+struct PackedTaps {
+    const double2 *xy;
+    const double *z;
+    __device__ __forceinline__ Tap3 operator()(int k) const
+    {
+        const double2 a = xy[k];
+        return {{a.x, a.y, z[k]}};
+    }
+};
+
+__device__ __forceinline__ void store_packed_series(double2 *xy, double *z, int cap,
+                                                    const double (&y)[6])
+{
+    double k[2][3];
+    combine_links(y, k);
+#pragma unroll
+    for (int kind = 0; kind < 2; ++kind) {
+        xy[kind * cap] = {k[kind][0], k[kind][1]};
+        z[kind * cap] = k[kind][2];
+    }
+}
+
+template <int NX>
+__device__ __forceinline__ bool tdi_linear_packed(double t, double L, double t0_offset, double fs,
+                                                  const double2 *xy, int cap, int win_lo, int win_len,
+                                                  const LagrangeView &lg, double (&acc)[3])
+{
+    const double *z = reinterpret_cast<const double *>(xy + 2 * cap);
+    return tdi_linear_cols<NX>(t, L, t0_offset, fs, win_lo, win_len, lg,
+                               [&](int kind, int c0) {
+                                   int off = kind * cap + c0;
                                    pin(off);
-                                   return ywin + off;
+                                   return PackedTaps{xy + off, z + off};
                                },
                                acc);
 }
@@ -473,12 +577,18 @@ __device__ __forceinline__ void blk_zero(double *ywin, int pitch, int R, int len
     }
 }
 
-// Block-interleaved window column c0 + k of a row, read through operator[].
+// Block-interleaved window column c0 + k of a row, read through operator[] (BlockTaps3: of the three
+// outputs' rows of one kind).
 struct BlockTaps {
     const double *row;
     int R;
     int c0;
     __device__ __forceinline__ double operator[](int k) const { return row[blk_col(c0 + k, R)]; }
+};
+
+struct BlockTaps3 {
+    BlockTaps o[3];
+    __device__ __forceinline__ Tap3 operator()(int k) const { return {{o[0][k], o[1][k], o[2][k]}}; }
 };
 
 // tdi_linear on block-interleaved rows (the per-sample fallback of the matrix-core path).
@@ -489,8 +599,11 @@ __device__ __forceinline__ bool tdi_linear_padded(double t, double L, double t0_
                                                   double (&acc)[3])
 {
     return tdi_linear_cols<NX, CE>(t, L, t0_offset, fs, win_lo, win_len, lg,
-                               [&](int o, int kind, int c0) {
-                                   return BlockTaps{ywin + (2 * o + kind) * pitch, R, c0};
+                               [&](int kind, int c0) {
+                                   const double *row = ywin + kind * pitch;
+                                   return BlockTaps3{{{row, R, c0},
+                                                      {row + 2 * pitch, R, c0},
+                                                      {row + 4 * pitch, R, c0}}};
                                },
                                acc);
 }

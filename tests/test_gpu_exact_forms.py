@@ -67,3 +67,24 @@ def test_tdi_either_side_of_the_limit(gpu, orbits, oracle_orbits, oracle_mod, or
            _capi.FLR_FLAG_OVERWRITE | _capi.FLR_FLAG_ZERO_EDGES | _capi.FLR_FLAG_EXACT)
     rw.check_errors()
     np.testing.assert_array_equal(out.cpu().numpy().reshape(3, n), exp)
+
+
+@pytest.mark.parametrize("tdi", ["1st generation", "2nd generation"])
+@pytest.mark.parametrize("over", [0, 1])
+def test_tdi_either_side_of_the_paired_window(gpu, orbits, oracle_orbits, oracle_mod, tdi, over):
+    """Equal arms read paired rows of links while 1706 window samples fit, single rows past that."""
+    import torch
+    from fastlisaresponse_amd import _capi
+    order, n, T = 25, 6000, 2000
+    ow, rw, (A, deps, E), tabs = _setup(gpu, orbits, order=order, tdi=tdi)
+    reach = (3 if tdi == "1st generation" else 7) * ow.extent()[1]
+    dt = reach / (1706 - 256 - 2 * 17 + over - 0.5)
+    assert 256 + 2 * 17 + math.ceil(reach / dt) == 1706 + over
+    y = np.random.default_rng(over).standard_normal((6, n))
+    exp = oracle_mod.get_tdi_delays(oracle_orbits, y, np.arange(n) * dt, _oracle_tables(tabs), order,
+                                    1 / dt, A, deps, E, T, 16)
+    out = torch.zeros(3 * n, dtype=torch.float64, device="cuda")
+    rw.tdi(out, torch.as_tensor(y.reshape(-1), device="cuda"), n, 0.0, dt, 1 / dt, T,
+           _capi.FLR_FLAG_OVERWRITE | _capi.FLR_FLAG_ZERO_EDGES | _capi.FLR_FLAG_EXACT)
+    rw.check_errors()
+    np.testing.assert_array_equal(out.cpu().numpy().reshape(3, n), exp)
