@@ -333,6 +333,19 @@ int batch_grid(int total_tiles, int grid_per_cu)
 
 static size_t proj_lds(const ProjConfig &cfg) { return (size_t)cfg.win_cap * sizeof(double2); }
 
+// f(form, H): the kernels are compiled for order 25 (H = 13, with the four-reciprocal form), and for any
+// (H = 0).
+template <typename F>
+static hipError_t by_order(bool exact, int64_t lowest, const LagrangeView &lg, F &&f)
+{
+    if (lg.h == 13)
+        return by_form<kExact4>(stencil_form(exact, lowest, lg.h, kExact4), [&](auto form) {
+            return f(form, std::integral_constant<int, 13>{});
+        });
+    return by_form(stencil_form(exact, lowest, lg.h),
+                   [&](auto form) { return f(form, std::integral_constant<int, 0>{}); });
+}
+
 // equal_arm: all six light travel time columns of the orbit table are bitwise equal (the
 // emitter stencils are then shared per emitting spacecraft; order 25 only).
 hipError_t launch_projection(const ProjConfig &cfg, const ProjSource &src, const OrbitView &orb,
@@ -341,16 +354,16 @@ hipError_t launch_projection(const ProjConfig &cfg, const ProjSource &src, const
 {
     const int nb = tiles_for(src.num_delays, src.start, cfg.zero_edges);
     const size_t shm = proj_lds(cfg);
-    const int form = stencil_form(exact, (int64_t)src.start - cfg.halo_lo, lg.h);
+    const int64_t lowest = (int64_t)src.start - cfg.halo_lo;
     hipError_t err;
-    if (launch_projection_split(cfg, src, orb, lg, form, equal_arm, stream, err)) return err;
-    return by_form(form, [&](auto form) {
-        constexpr int F = decltype(form)::value;
-        if (lg.h == 13 && equal_arm)
-            return launch(projection_kernel<F, 13, true>, nb, shm, stream, cfg, src, orb, lg);
-        if (lg.h == 13)
-            return launch(projection_kernel<F, 13, false>, nb, shm, stream, cfg, src, orb, lg);
-        return launch(projection_kernel<F, 0, false>, nb, shm, stream, cfg, src, orb, lg);
+    if (launch_projection_split(cfg, src, orb, lg, stencil_form(exact, lowest, lg.h), equal_arm, stream,
+                                err))
+        return err;
+    return by_order(exact, lowest, lg, [&](auto form, auto h) {
+        constexpr int F = decltype(form)::value, H = decltype(h)::value;
+        if (H == 13 && equal_arm)
+            return launch(projection_kernel<F, H, H == 13>, nb, shm, stream, cfg, src, orb, lg);
+        return launch(projection_kernel<F, H, false>, nb, shm, stream, cfg, src, orb, lg);
     });
 }
 
@@ -360,13 +373,11 @@ hipError_t launch_projection_batch(const ProjConfig &cfg, const Batch<ProjSource
 {
     const int nb = batch_grid(b.total_tiles, grid_per_cu);
     const size_t shm = proj_lds(cfg);
-    return by_form(stencil_form(exact, (int64_t)b.min_start - cfg.halo_lo, lg.h), [&](auto form) {
-        constexpr int F = decltype(form)::value;
-        if (lg.h == 13 && equal_arm)
-            return launch(projection_batch_kernel<F, 13, true>, nb, shm, stream, cfg, b, orb, lg);
-        if (lg.h == 13)
-            return launch(projection_batch_kernel<F, 13, false>, nb, shm, stream, cfg, b, orb, lg);
-        return launch(projection_batch_kernel<F, 0, false>, nb, shm, stream, cfg, b, orb, lg);
+    return by_order(exact, (int64_t)b.min_start - cfg.halo_lo, lg, [&](auto form, auto h) {
+        constexpr int F = decltype(form)::value, H = decltype(h)::value;
+        if (H == 13 && equal_arm)
+            return launch(projection_batch_kernel<F, H, H == 13>, nb, shm, stream, cfg, b, orb, lg);
+        return launch(projection_batch_kernel<F, H, false>, nb, shm, stream, cfg, b, orb, lg);
     });
 }
 
@@ -416,10 +427,9 @@ hipError_t launch_tdi(const TdiConfig &cfg, const TdiSource &src, const OrbitVie
         });
     }
     const size_t shm = tdi_lds(cfg, false);
-    return by_form(stencil_form(exact, lowest, lg.h), [&](auto form) {
-        constexpr int F = decltype(form)::value;
-        if (lg.h == 13) return launch(tdi_kernel<F, 13>, nb, shm, stream, cfg, src, orb, lg);
-        return launch(tdi_kernel<F, 0>, nb, shm, stream, cfg, src, orb, lg);
+    return by_order(exact, lowest, lg, [&](auto form, auto h) {
+        constexpr int F = decltype(form)::value, H = decltype(h)::value;
+        return launch(tdi_kernel<F, H>, nb, shm, stream, cfg, src, orb, lg);
     });
 }
 
@@ -440,10 +450,9 @@ hipError_t launch_tdi_batch(const TdiConfig &cfg, const Batch<TdiSource> &b, con
         });
     }
     const size_t shm = tdi_lds(cfg, false);
-    return by_form(stencil_form(exact, lowest, lg.h), [&](auto form) {
-        constexpr int F = decltype(form)::value;
-        if (lg.h == 13) return launch(tdi_batch_kernel<F, 13>, nb, shm, stream, cfg, b, orb, lg);
-        return launch(tdi_batch_kernel<F, 0>, nb, shm, stream, cfg, b, orb, lg);
+    return by_order(exact, lowest, lg, [&](auto form, auto h) {
+        constexpr int F = decltype(form)::value, H = decltype(h)::value;
+        return launch(tdi_batch_kernel<F, H>, nb, shm, stream, cfg, b, orb, lg);
     });
 }
 

@@ -41,6 +41,16 @@ FLR_HOST_DEVICE inline double div_recip(double a, const Recip &r)
     return __builtin_fma(a, r.y, a * r.l);
 }
 
+// The same quotient from y alone: with y off by at most e1, q = y a by at most e1 + u, the residual
+// a - b q comes out exactly (a multiple of ulp(b) ulp(q) below 8 b of them) and the last operation rounds
+// a / b off by e1 (e1 + u): 12 u^2 with recip_pair's e1 = 3 u, 30 u^2 with recip_quad's 5 u, less than
+// div_recip's from the same y.
+FLR_HOST_DEVICE inline double div_recip_y(double a, double b, const Recip &r)
+{
+    const double q = a * r.y;
+    return __builtin_fma(__builtin_fma(-b, q, a), r.y, q);
+}
+
 // The two denominators of a tap pair, F = j + e and G = j + (1 - e): one hardware reciprocal of
 // their product (relative error below 2^-22), refined to third order, gives both.
 FLR_HOST_DEVICE inline void recip_pair(double F, double G, Recip &rF, Recip &rG)

@@ -38,10 +38,14 @@ extern "C" long check4(const double *a, const double *F, const double *G, const 
         wrong += flr::div_recip(a[i], g1) != a[i] / G[i];
         wrong += flr::div_recip(a[k], f2) != a[k] / F[k];
         wrong += flr::div_recip(a[k], g2) != a[k] / G[k];
+        wrong += flr::div_recip_y(a[i], F[i], f1) != a[i] / F[i];
+        wrong += flr::div_recip_y(a[i], G[i], g1) != a[i] / G[i];
+        wrong += flr::div_recip_y(a[k], F[k], f2) != a[k] / F[k];
+        wrong += flr::div_recip_y(a[k], G[k], g2) != a[k] / G[k];
     }
     return wrong;
 }
-// wrong[0]: quotients of div_recip that differ from a / b; wrong[1]: those of y a alone
+// wrong[0]: quotients of div_recip and div_recip_y that differ from a / b; wrong[1]: those of y a alone
 extern "C" void check(const double *a, const double *F, const double *G, const double *err, long n,
                       long *wrong)
 {
@@ -52,6 +56,8 @@ extern "C" void check(const double *a, const double *F, const double *G, const d
         flr::recip_pair(F[i], G[i], rF, rG);
         wrong[0] += flr::div_recip(a[i], rF) != a[i] / F[i];
         wrong[0] += flr::div_recip(a[i], rG) != a[i] / G[i];
+        wrong[0] += flr::div_recip_y(a[i], F[i], rF) != a[i] / F[i];
+        wrong[0] += flr::div_recip_y(a[i], G[i], rG) != a[i] / G[i];
         wrong[1] += a[i] * rF.y != a[i] / F[i];
     }
 }

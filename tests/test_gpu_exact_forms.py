@@ -22,20 +22,24 @@ def _limit(h):
 
 @pytest.mark.parametrize("order", [15, 25, 31, 35])
 @pytest.mark.parametrize("side", [-1, 0])
-def test_projection_either_side_of_the_limit(gpu, orbits, oracle_orbits, oracle_mod, order, side):
+@pytest.mark.parametrize("limit,n", [(None, 2001), (512, 100_001)])
+def test_projection_either_side_of_the_limit(gpu, orbits, oracle_orbits, oracle_mod, order, side, limit,
+                                             n):
     import torch
     from fastlisaresponse_amd import _capi
     from fastlisaresponse_amd.tables import sky_basis
     ow, rw, (A, deps, E), _ = _setup(gpu, orbits, order=order)
-    n, dt, h, t0 = 2001, 10.0, (order + 1) // 2, 1.1e6
+    dt, h, t0 = 10.0, (order + 1) // 2, 1.1e6
     radius, ltt = ow.extent()
     halo_lo = math.ceil((ltt + radius * C_INV) / dt) + h + 4
-    P = _limit(h) + halo_lo - (h - 1) + side
+    # order 25 also changes form at 512 (four reciprocals at a time) in the one-lane kernels, which take
+    # the longer series
+    P = (limit or _limit(h)) + halo_lo - (h - 1) + side
     rng = np.random.default_rng(order + side)
     hh = rng.standard_normal(n) + 1j * rng.standard_normal(n)
     k, u, v = sky_basis(2.2, -0.6)
     exp = oracle_mod.get_response(oracle_orbits, hh, t0 + np.arange(n) * dt, k, u, v, order, 1 / dt,
-                                  A, deps, E, P, 4)
+                                  A, deps, E, P, 16)
     y = torch.zeros(6 * n, dtype=torch.float64, device="cuda")
     rw.projection(y, torch.as_tensor(hh, device="cuda"), n, t0, dt, 1 / dt, k, u, v, P,
                   _capi.FLR_FLAG_ZERO_EDGES | _capi.FLR_FLAG_EXACT)
@@ -56,8 +60,10 @@ def test_tdi_either_side_of_the_limit(gpu, orbits, oracle_orbits, oracle_mod, or
     limit = limit or _limit(h)
     chain = {"1st generation": 3, "2nd generation": 7}.get(tdi, 2) if isinstance(tdi, str) else 2
     halo_lo = math.ceil(chain * ow.extent()[1] / dt) + h + 4
-    # the stock tables at order 25 also change form at 512 (four reciprocals at a time); long enough
-    # a series for the one-lane kernels
+    # order 25 also changes form at 512 (four reciprocals at a time) in the one-lane kernels, which take
+    # the longest series (any other table: past half a million samples)
+    if order == 25 and tdi is CUSTOM and n > 100_000:
+        n = 530_001
     T = limit + halo_lo - (h - 1) + side
     y = np.random.default_rng(order + side).standard_normal((6, n))
     exp = oracle_mod.get_tdi_delays(oracle_orbits, y, t0 + np.arange(n) * dt, _oracle_tables(tabs),
