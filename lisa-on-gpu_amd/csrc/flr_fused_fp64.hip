@@ -11,7 +11,7 @@ hipError_t launch_fused_fp64(const ProjConfig &pc, const TdiConfig &tc,
 {
     // the projection's windows reach lowest: the TDI window's start less the projection's halo
     const int64_t lowest = (int64_t)b.min_start - tc.halo_lo - pc.halo_lo;
-    return by_form<kExact4>(stencil_form(exact, lowest, lg.h, kExact4), [&](auto form) {
+    return by_form(stencil_form(exact, lowest, lg.h), [&](auto form) {
         return launch_fused_variant<decltype(form)::value, double2, double, 2>(
             pc, tc, b, orb, lg, st, grid_per_cu, stream);
     });

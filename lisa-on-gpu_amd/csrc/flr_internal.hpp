@@ -25,7 +25,7 @@ constexpr int kOrbitStride = 2 * kOrbitVals;
 // sequence, each quotient in three operations from its denominator's reciprocal. kExact2: the same
 // quotients, bit for bit, in two (div_recip) -- for stencils at sample positions of at least
 // exact2_min_position(h). kExact4: kExact2 with the reciprocals four at a time, from
-// exact4_min_position(h) on (the one-lane and fused kernels of order 25).
+// exact4_min_position(h) on.
 constexpr int kFast = 0;
 constexpr int kExact = 1;
 constexpr int kExact2 = 2;
@@ -33,11 +33,10 @@ constexpr int kExact4 = 3;
 
 // The form of a launch whose staged windows start at sample `lowest` or later: every stencil that
 // passes its window test sits at least h - 1 samples above its window's start.
-// best: the best form the kernel has, kExact2 or kExact4.
-inline int stencil_form(bool exact, int64_t lowest, int h, int best = kExact2)
+inline int stencil_form(bool exact, int64_t lowest, int h)
 {
     if (!exact) return kFast;
-    if (best == kExact4 && lowest + h - 1 >= exact4_min_position(h)) return kExact4;
+    if (lowest + h - 1 >= exact4_min_position(h)) return kExact4;
     return lowest + h - 1 >= exact2_min_position(h) ? kExact2 : kExact;
 }
 

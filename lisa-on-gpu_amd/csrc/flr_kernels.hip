@@ -333,17 +333,14 @@ int batch_grid(int total_tiles, int grid_per_cu)
 
 static size_t proj_lds(const ProjConfig &cfg) { return (size_t)cfg.win_cap * sizeof(double2); }
 
-// f(form, H): the kernels are compiled for order 25 (H = 13, with the four-reciprocal form), and for any
-// (H = 0).
+// f(form, H): the kernels are compiled for order 25 (H = 13) and for any (H = 0).
 template <typename F>
 static hipError_t by_order(bool exact, int64_t lowest, const LagrangeView &lg, F &&f)
 {
-    if (lg.h == 13)
-        return by_form<kExact4>(stencil_form(exact, lowest, lg.h, kExact4), [&](auto form) {
-            return f(form, std::integral_constant<int, 13>{});
-        });
-    return by_form(stencil_form(exact, lowest, lg.h),
-                   [&](auto form) { return f(form, std::integral_constant<int, 0>{}); });
+    return by_form(stencil_form(exact, lowest, lg.h), [&](auto form) {
+        if (lg.h == 13) return f(form, std::integral_constant<int, 13>{});
+        return f(form, std::integral_constant<int, 0>{});
+    });
 }
 
 // equal_arm: all six light travel time columns of the orbit table are bitwise equal (the
@@ -399,7 +396,7 @@ static hipError_t by_stock_layout(const TdiConfig &cfg, bool exact, int64_t lowe
     using std::integral_constant;
     if (equal_arm && exact && pairs > kMaxLds)
         return f(integral_constant<int, kExact>{}, integral_constant<WindowLayout, kEqualRows>{}, rows);
-    return by_form<kExact4>(stencil_form(exact, lowest, lg.h, kExact4), [&](auto form) {
+    return by_form(stencil_form(exact, lowest, lg.h), [&](auto form) {
         constexpr int F_ = decltype(form)::value;
         if (equal_arm)
             return f(form, integral_constant<WindowLayout, F_ == kFast ? kPacked : kPairs>{},

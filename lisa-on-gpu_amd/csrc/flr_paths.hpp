@@ -304,16 +304,15 @@ inline hipError_t set_lds_limit(Kernel k, size_t bytes)
     return hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-// f(std::integral_constant<int, form>): the kernels are compiled per stencil form, up to BEST
-// (stencil_form's best).
-template <int BEST = kExact2, typename F>
+// f(std::integral_constant<int, form>): the kernels are compiled per stencil form.
+template <typename F>
 inline hipError_t by_form(int form, F &&f)
 {
     switch (form) {
     case kFast: return f(std::integral_constant<int, kFast>{});
     case kExact: return f(std::integral_constant<int, kExact>{});
     case kExact2: return f(std::integral_constant<int, kExact2>{});
-    default: return f(std::integral_constant<int, BEST>{});
+    default: return f(std::integral_constant<int, kExact4>{});
     }
 }
 

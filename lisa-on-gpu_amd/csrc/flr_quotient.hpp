@@ -68,11 +68,12 @@ FLR_HOST_DEVICE inline void recip_pair(double F, double G, Recip &rF, Recip &rG)
 // Two tap pairs at once: one hardware reciprocal of p1 p2 for all four denominators (14 issue slots
 // per pair, with the two sums j + e and j + (1 - e), instead of 16). Their y is off by up to e1 = 5 u
 // (p1, p1 p2, its reciprocal, the product by p2, the product by the other factor; p2's rounding cancels),
-// so a quotient by div_recip is a / b up to 25 u^2 + 5 u^2 + 5 u^2 = 35 u^2: below the least distance from a
-// midpoint, 2^c u^2 / h, for h <= 14 from position 2^9 on (exact4_min_position). With the six undelayed
+// so a quotient by div_recip is a / b up to 25 u^2 + 5 u^2 + 5 u^2 = 35 u^2, by div_recip_y up to 30 u^2: below
+// the least distance from a midpoint, 2^c u^2 / h, from position 2^9 on for h <= 14 and h <= 17, from 2^10
+// on for h <= 29 and h <= 34 (exact4_min_position; kernels for any order use div_recip_y). With the six undelayed
 // units of unequal arms sharing theirs, 13,744 instead of 15,791 issue slots per sample of unequal-arm
 // TDI: 1,048,577 samples, 2nd generation, 453 -> 410 us (equal arms 225 -> 221).
-constexpr int exact4_min_position(int h) { return h <= 14 ? 512 : 1 << 30; }
+constexpr int exact4_min_position(int h) { return h <= 17 ? 512 : 1024; }
 
 FLR_HOST_DEVICE inline void recip_quad(double F1, double G1, double F2, double G2, Recip &rF1,
                                        Recip &rG1, Recip &rF2, Recip &rG2)

@@ -372,7 +372,8 @@ constexpr size_t kSplitLds = 64 * 1024;  // wider windows (fine sampling) keep t
 //   unequal-arm stock TDI: exact 163,841 samples 99.3 -> 91.6, 196,608 104.2 -> 108.8; fast 98,304
 //     39.6 -> 36.1, 131,072 (1st generation) 22.6 -> 24.8
 //   any other table: 262,145 samples 77.2 -> 71.1, 524,289 138 -> 131, 1,048,577 239 -> 241 (its
-//     one-lane form loops over units and taps one load at a time)
+//     one-lane form loops over units and taps one load at a time); since then both take their reciprocals
+//     four at a time, 262,145 69.9 -> 62.5 and 1,048,577 232.6 -> 217.1
 constexpr int kSplitProj = 384;
 constexpr int kSplitEqual = 640;
 constexpr int kSplitStock = 640;
@@ -398,9 +399,13 @@ bool launch_projection_split(const ProjConfig &cfg, const ProjSource &src, const
                      stream, cfg, src, orb, lg)                                                   \
      : lg.h == 13 ? launch_tpb(projection_split_kernel<F, 13, false>, nb,                         \
                                kSplit * split_tasks(false), shm, stream, cfg, src, orb, lg)       \
-                  : launch_tpb(projection_split_kernel<F, 0, false>, nb,                          \
+                  : launch_tpb(projection_split_kernel<F == kFast ? kFast : kExact2, 0, false>, nb, \
                                kSplit * split_tasks(false), shm, stream, cfg, src, orb, lg))
-    err = form == kFast ? FLR_SPLIT(kFast) : FLR_SPLIT(kExact2);
+    // any other order keeps two reciprocals at a time: with four (74 VGPRs) two of its 9-wave groups fit
+    // a CU instead of three, and 65,537 samples at order 31 take 20.1 us instead of 18.1
+    err = form == kFast     ? FLR_SPLIT(kFast)
+          : form == kExact2 ? FLR_SPLIT(kExact2)
+                            : FLR_SPLIT(kExact4);
 #undef FLR_SPLIT
     return true;
 }
@@ -421,15 +426,17 @@ bool launch_tdi_split(const TdiConfig &cfg, const TdiSource &src, const OrbitVie
     const int nb = tiles_for(src.num_delays, src.start, cfg.zero_edges, kSplit);
     const RowMap &rm = stock.rows;
 #define FLR_SPLIT(F)                                                                             \
-    (eq ? nx == 8 ? launch_tpb(tdi_split_equal_kernel<8, F>, nb, 4 * kSplit, shm, stream, cfg,   \
-                               src, orb, lg, rm)                                                 \
-                  : launch_tpb(tdi_split_equal_kernel<16, F>, nb, 8 * kSplit, shm, stream, cfg,  \
-                               src, orb, lg, rm)                                                 \
+    (eq ? nx == 8 ? launch_tpb(tdi_split_equal_kernel<8, F == kFast ? kFast : kExact2>, nb,      \
+                               4 * kSplit, shm, stream, cfg, src, orb, lg, rm)                   \
+                  : launch_tpb(tdi_split_equal_kernel<16, F == kFast ? kFast : kExact2>, nb,     \
+                               8 * kSplit, shm, stream, cfg, src, orb, lg, rm)                   \
      : lg.h == 13 ? launch_tpb(tdi_split_units_kernel<F, 13>, nb, kSplit * kSplitWaves, shm,     \
                                stream, cfg, src, orb, lg)                                        \
                   : launch_tpb(tdi_split_units_kernel<F, 0>, nb, kSplit * kSplitWaves, shm,      \
                                stream, cfg, src, orb, lg))
-    err = form == kFast ? FLR_SPLIT(kFast) : FLR_SPLIT(kExact2);
+    err = form == kFast     ? FLR_SPLIT(kFast)
+          : form == kExact2 ? FLR_SPLIT(kExact2)
+                            : FLR_SPLIT(kExact4);
 #undef FLR_SPLIT
     return true;
 }

@@ -167,7 +167,7 @@ __device__ __forceinline__ bool tdi_equal_arm(double t, double L, double t0_offs
         // j fully unrolled: every tap address is the channel's base plus an immediate offset;
         // the memory barrier and the pins at the end of each j keep its loads and arithmetic
         // together.
-        for_tap_pairs<EXACT, H>(e, [&](int j, const auto &q) {
+        for_tap_pairs<EXACT, H>(e, H, [&](int j, const auto &q) {
             const double E = lg.E[j - 1];
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
@@ -295,7 +295,7 @@ __device__ __forceinline__ bool tdi_stock_unequal(double t, const double (&L)[6]
             });
         });
         double S[3][2] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
-        for_tap_pairs<EXACT, H>(e, [&](int j, const auto &q) {
+        for_tap_pairs<EXACT, H>(e, H, [&](int j, const auto &q) {
             const double E = lg.E[j - 1];
 #pragma unroll
             for (int c = 0; c < 3; ++c)

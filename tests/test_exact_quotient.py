@@ -25,8 +25,10 @@ static thread_local double seed_error;
 #include "flr_quotient.hpp"
 extern "C" int min_position(int h) { return flr::exact2_min_position(h); }
 extern "C" int min_position4(int h) { return flr::exact4_min_position(h); }
-// the same through recip_quad, each pair beside the one n/2 further on
-extern "C" long check4(const double *a, const double *F, const double *G, const double *err, long n)
+// the same through recip_quad, each pair beside the one n/2 further on (parts: div_recip too, which
+// order 25 takes)
+extern "C" long check4(const double *a, const double *F, const double *G, const double *err, long n,
+                       int parts)
 {
     long wrong = 0;
     for (long i = 0; i + n / 2 < n; ++i) {
@@ -34,10 +36,12 @@ extern "C" long check4(const double *a, const double *F, const double *G, const 
         const long k = i + n / 2;
         flr::Recip f1, g1, f2, g2;
         flr::recip_quad(F[i], G[i], F[k], G[k], f1, g1, f2, g2);
-        wrong += flr::div_recip(a[i], f1) != a[i] / F[i];
-        wrong += flr::div_recip(a[i], g1) != a[i] / G[i];
-        wrong += flr::div_recip(a[k], f2) != a[k] / F[k];
-        wrong += flr::div_recip(a[k], g2) != a[k] / G[k];
+        if (parts) {
+            wrong += flr::div_recip(a[i], f1) != a[i] / F[i];
+            wrong += flr::div_recip(a[i], g1) != a[i] / G[i];
+            wrong += flr::div_recip(a[k], f2) != a[k] / F[k];
+            wrong += flr::div_recip(a[k], g2) != a[k] / G[k];
+        }
         wrong += flr::div_recip_y(a[i], F[i], f1) != a[i] / F[i];
         wrong += flr::div_recip_y(a[i], G[i], g1) != a[i] / G[i];
         wrong += flr::div_recip_y(a[k], F[k], f2) != a[k] / F[k];
@@ -85,11 +89,11 @@ def _check(lib, a, F, G, err):
     return wrong[0], wrong[1]
 
 
-def _check4(lib, a, F, G, err):
+def _check4(lib, a, F, G, err, h):
     a, F, G, err = (np.ascontiguousarray(x, dtype=np.float64) for x in (a, F, G, err))
     lib.check4.restype = ctypes.c_long
     return lib.check4(*(ctypes.c_void_p(x.ctypes.data) for x in (a, F, G, err)),
-                      ctypes.c_long(len(a)))
+                      ctypes.c_long(len(a)), h <= 14)
 
 
 def _denominators(rng, h, pos, n):
@@ -112,14 +116,11 @@ def test_random_numerators(lib, h):
     two_ops, one_op = _check(lib, a, F, G, err)
     assert two_ops == 0
     assert one_op > n // 20  # the test can tell
-    if h <= 14:  # the form of four at a time, from its own least position
-        F, G, _ = _denominators(rng, h, lib.min_position4(h), n)
-        assert _check4(lib, a, F, G, err) == 0
-    else:
-        assert lib.min_position4(h) > 1 << 29  # never used
+    F, G, _ = _denominators(rng, h, lib.min_position4(h), n)  # from its own least position
+    assert _check4(lib, a, F, G, err, h) == 0
 
 
-@pytest.mark.parametrize("h,four", [(13, False), (16, False), (20, False), (13, True)])
+@pytest.mark.parametrize("h,four", [(13, False), (16, False), (20, False), (13, True), (16, True), (20, True)])
 def test_hardest_numerators(lib, h, four):
     rng = np.random.default_rng(100 + h)
     n = 20_000
@@ -149,7 +150,7 @@ def test_hardest_numerators(lib, h, four):
     assert len(a) > 2000
     err = rng.uniform(-1, 1, len(a)) * 2.0 ** -22
     if four:
-        assert _check4(lib, np.array(a), np.array(Fk), np.array(Gk), err) == 0
+        assert _check4(lib, np.array(a), np.array(Fk), np.array(Gk), err, h) == 0
         return
     two_ops, _ = _check(lib, np.array(a), np.array(Fk), np.array(Gk), err)
     assert two_ops == 0

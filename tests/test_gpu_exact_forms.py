@@ -32,8 +32,10 @@ def test_projection_either_side_of_the_limit(gpu, orbits, oracle_orbits, oracle_
     dt, h, t0 = 10.0, (order + 1) // 2, 1.1e6
     radius, ltt = ow.extent()
     halo_lo = math.ceil((ltt + radius * C_INV) / dt) + h + 4
-    # order 25 also changes form at 512 (four reciprocals at a time) in the one-lane kernels, which take
-    # the longer series
+    # the second change of form (four reciprocals at a time) in the one-lane kernels, which take the
+    # longer series
+    if limit == 512 and h > 17:
+        limit = 1024
     P = (limit or _limit(h)) + halo_lo - (h - 1) + side
     rng = np.random.default_rng(order + side)
     hh = rng.standard_normal(n) + 1j * rng.standard_normal(n)
@@ -58,11 +60,13 @@ def test_tdi_either_side_of_the_limit(gpu, orbits, oracle_orbits, oracle_mod, or
     ow, rw, (A, deps, E), tabs = _setup(gpu, orbits, order=order, tdi=tdi)
     dt, h, t0 = 10.0, (order + 1) // 2, 0.0
     limit = limit or _limit(h)
+    if n > 2000 and h > 17:
+        limit = 1024
     chain = {"1st generation": 3, "2nd generation": 7}.get(tdi, 2) if isinstance(tdi, str) else 2
     halo_lo = math.ceil(chain * ow.extent()[1] / dt) + h + 4
-    # order 25 also changes form at 512 (four reciprocals at a time) in the one-lane kernels, which take
+    # the second change of form (four reciprocals at a time) in the split and one-lane kernels, which take
     # the longest series (any other table: past half a million samples)
-    if order == 25 and tdi is CUSTOM and n > 100_000:
+    if tdi is CUSTOM and n > 100_000:
         n = 530_001
     T = limit + halo_lo - (h - 1) + side
     y = np.random.default_rng(order + side).standard_normal((6, n))
