@@ -229,16 +229,18 @@ __global__ __launch_bounds__(kBlock) void lti_filter_kernel(TdiConfig tc,
         v = (double)lref.kmin;
     else if (x == kLtiOk)
         v = lref.ok ? 1.0 : 0.0;
+    else
+        v = (double)lref.taps;
     tc.lti_fir[(size_t)s * kLtiRecord + x] = v;
 }
 
 // Composite-filter TDI of one tile on the matrix cores. Outputs are taken in blocks of 16
 // aligned to the source's first TDI sample (block q = samples T + 16q .. T + 16q + 15, so a
 // sample's arithmetic is the same whatever tile holds it); per output o and block,
-//   out[i_b + r] = sum_kind sum_{m=0}^{55} F_kind[m - r] S_{o,kind}[i_b + kmin + m],
+//   out[i_b + r] = sum_kind sum_{m=0}^{4 steps - 1} F_kind[m - r] S_{o,kind}[i_b + kmin + m],
 // which is D = A B with A[r][m] = F[m - r] (Toeplitz, the padded filters) and
 // B[m][block] = the series: one v_mfma_f64_16x16x4f64 per 4 taps of 16 blocks x 16 outputs
-// (28 per group of 16 blocks of one output). Operand layout: lane l holds A[l % 16][l / 16]
+// (2 steps = 22 .. 28, fir_steps of the filters' taps, per group of 16 blocks of one output). Operand layout: lane l holds A[l % 16][l / 16]
 // and B[l / 16][l % 16]; the result's element v is D[4v + l / 16][l % 16]. The rows are
 // block-interleaved (blk_col), so each B operand is one load at a per-lane base plus a
 // compile-time offset; edge blocks read the zeroed guard and tail slots wherever F is zero,
@@ -247,7 +249,8 @@ __global__ __launch_bounds__(kBlock) void lti_filter_kernel(TdiConfig tc,
 template <typename OT, int TPB>
 __device__ __forceinline__ void lti_mfma(const TdiConfig &tc, const FusedSource &src, int first,
                                          int last, int i0, int yw_lo, int yw_len, int kmin,
-                                         const double *ywin, int pitch, int R, const double *fpad,
+                                         int steps, const double *ywin, int pitch, int R,
+                                         const double *fpad,
                                          const unsigned char *lti_ok, bool all_ok,
                                          InnerShared *ish)
 {
@@ -275,7 +278,8 @@ __device__ __forceinline__ void lti_mfma(const TdiConfig &tc, const FusedSource 
             const double *row = ywin + (2 * o + kind) * pitch;
             const double *f = fpad + kind * kFpad + kFpadLo + kq - nb;  // f[4j] = F[4j + kq - nb]
 #pragma unroll
-            for (int j = 0; j < 14; ++j) {
+            for (int j = 0; j < kFirSteps; ++j) {
+                if (j >= kFirLeastSteps && j >= steps) break;
                 acc = __builtin_amdgcn_mfma_f64_16x16x4f64(f[4 * j], row[b[j & 3] + (j >> 2)], acc,
                                                           0, 0, 0);
                 __asm__ volatile("" ::: "memory");  // one operand pair in flight: no register growth
@@ -300,14 +304,14 @@ __device__ __forceinline__ void lti_mfma(const TdiConfig &tc, const FusedSource 
 
 // The slowly-varying-arm TDI of one tile on the matrix cores (utv_unit): per group of 16
 // blocks of 16 samples (blocks aligned to the source's first TDI sample, as lti_mfma), the
-// three channels' F0 and F1 sums over their four base links -- 24 accumulations of 14
+// three channels' F0 and F1 sums over their four base links -- 24 accumulations of `steps` (fir_steps)
 // v_mfma_f64_16x16x4f64 each, the link series' operand shared by the pair's two filters --
 // then X_c = F0 part + (i - m) F1 part, A, E, T formed from X, Y, Z in FP64, and stored.
 // filt: [2][kUtvPairs][kFpad] (F0 then F1, padded as fpad); link rows canonical at ywin +
 // k * pitch.
 template <typename OT, int TPB>
 __device__ __forceinline__ void utv_mfma(const TdiConfig &tc, const FusedSource &src, int first,
-                                         int last, int m, int yw_lo, int yw_len, int kmin,
+                                         int last, int m, int yw_lo, int yw_len, int kmin, int steps,
                                          const double *ywin, int pitch, int R, const double *filt,
                                          InnerShared *ish)
 {
@@ -331,7 +335,8 @@ __device__ __forceinline__ void utv_mfma(const TdiConfig &tc, const FusedSource 
         for (int c = 0; c < 3; ++c) a0[c] = a1[c] = d4{0.0, 0.0, 0.0, 0.0};
         const double *fl = filt + kFpadLo + kq - nb;  // fl[p * kFpad + 4j] = F0_p[4j + kq - nb]
 #pragma unroll
-        for (int j = 0; j < 14; ++j) {
+        for (int j = 0; j < kFirSteps; ++j) {
+            if (j >= kFirLeastSteps && j >= steps) break;
             const int col = b[j & 3] + (j >> 2);
             static_for<6>([&](auto l) {  // canonical link l: one operand for its two pairs
                 const double yv = ywin[l * pitch + col];
@@ -450,6 +455,7 @@ __device__ __forceinline__ void fused_tile(const ProjConfig &pc, const TdiConfig
         ost = stage_orbit_nodes(orb, src.t0 + (double)yw_lo * pc.dt, s_orb, tid, TPB);
     }
     LtiRef<NX> lref;
+    int lti_steps = 0;
     bool lti = false, tile_ok = false;
     if constexpr (kLti) {
         // the source's reference, from its filter record (lti_filter_kernel), and its filters
@@ -459,6 +465,7 @@ __device__ __forceinline__ void fused_tile(const ProjConfig &pc, const TdiConfig
         const double L_ref = fir[kLtiLref];
         lref.kmin = (int)fir[kLtiKmin];
         lti = fir[kLtiOk] != 0.0;
+        lti_steps = __builtin_amdgcn_readfirstlane(fir_steps((int)fir[kLtiTaps]));
         tile_ok = lti && lti_tile_matches<NX>(tc, src, orb, rm, lref.kmin, L_ref, first, last);
         if (lti) {
             for (int x = tid; x < 2 * kFpad; x += TPB) {
@@ -574,8 +581,8 @@ __device__ __forceinline__ void fused_tile(const ProjConfig &pc, const TdiConfig
             // lti_ok and the per-sample samples' sums written (the rows and filters were, by
             // the projection's barrier)
             if (SAMPLE_PASS || inner) __syncthreads();
-            lti_mfma<OT, TPB>(tc, src, first, last, i0, yw_lo, yw_len, lref.kmin, ywin, pitch, R,
-                              fpad, lti_ok, tile_ok, ish);
+            lti_mfma<OT, TPB>(tc, src, first, last, i0, yw_lo, yw_len, lref.kmin, lti_steps, ywin,
+                              pitch, R, fpad, lti_ok, tile_ok, ish);
         }
     }
     if (bad) atomicOr(tc.err, kErrWindow);
@@ -720,16 +727,23 @@ __device__ __forceinline__ void fused_tile_utv(const ProjConfig &pc, const TdiCo
                          sh.kmax <= tc.halo_hi;
     if (tile_ok) {
         const int nt = sh.kmax - kmin + 1;
+        // the filters' entries on consecutive lanes (12 nt of them: 6 waves' worth at dt = 10 s where the
+        // padded rows take 14), the padding on its own; with a loop over the pair's own units, 0.13 of the
+        // kernel's vector instructions less: 8 sources, 4.2e6 samples, 582 -> 539 us with fir_steps
         for (int x = tid; x < kUtvPairs * kFpad; x += TPB) {
-            const int p = x / kFpad, k = x - p * kFpad - kFpadLo;
-            double f0 = 0.0, f1 = 0.0;
-            if (k >= 0 && k < nt) utv_filter_entry<NX>(sh, lg, s_E, p, k, f0, f1);
-            filt[x] = f0;
-            filt[kUtvPairs * kFpad + x] = f1;
+            const int k = x % kFpad - kFpadLo;
+            if (k < 0 || k >= nt) filt[x] = filt[kUtvPairs * kFpad + x] = 0.0;
+        }
+        for (int x = tid; x < kUtvPairs * nt; x += TPB) {
+            const int p = x / nt, k = x - p * nt;
+            double f0, f1;
+            utv_filter_entry<NX>(sh, lg, s_E, p, k, f0, f1);
+            filt[p * kFpad + kFpadLo + k] = f0;
+            filt[(kUtvPairs + p) * kFpad + kFpadLo + k] = f1;
         }
         __syncthreads();
-        utv_mfma<float, TPB>(tc, src, first, last, m, yw_lo, yw_len, kmin, ywin, pitch, R, filt,
-                             ish);
+        utv_mfma<float, TPB>(tc, src, first, last, m, yw_lo, yw_len, kmin,
+                             __builtin_amdgcn_readfirstlane(fir_steps(nt)), ywin, pitch, R, filt, ish);
     } else {
 #pragma unroll 1
         for (int r = 0; r < PASSES; ++r) {

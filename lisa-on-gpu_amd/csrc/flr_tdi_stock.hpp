@@ -620,17 +620,35 @@ __device__ __forceinline__ bool tdi_linear_padded(double t, double L, double t0_
 constexpr int kFir = 40;
 constexpr double kLtiTol = 1e-8;
 // Per-source record of a mixed batch's composite filters (tc.lti_fir): the two filters
-// ([2][kFir]), then the reference arm length, the first tap kmin and the fit flag (1 or 0) of
-// lti_source_reference, padded to a multiple of 4 doubles.
+// ([2][kFir]), then the reference arm length, the first tap kmin, the fit flag (1 or 0) and the tap
+// count of lti_source_reference.
 constexpr int kLtiLref = 2 * kFir;
 constexpr int kLtiKmin = 2 * kFir + 1;
 constexpr int kLtiOk = 2 * kFir + 2;
+constexpr int kLtiTaps = 2 * kFir + 3;
 constexpr int kLtiRecord = 2 * kFir + 4;
 // One kind's composite filter as the matrix-core path reads it: taps -15 .. 55 (zero outside
 // 0 .. kFir-1), so that a 16-output block's Toeplitz operand F[q - r] (q in 0..55, r in 0..15)
 // is one indexed load.
 constexpr int kFpadLo = 15;
 constexpr int kFpad = 72;
+// Matrix steps of 4 taps that a block of 16 outputs takes for a filter of `taps` taps: 12 of 14 at
+// dt = 10 s (31 or 32 taps), 2nd generation. A float64 matrix instruction runs at the FP64 pipes'
+// rate and in their place (16x16x4: 64 cycles, and none of them overlaps another wave's v_fma_f64), so
+// every step left out is time: 1.06e8 samples (64 sources, mixed-c128) 6.45 -> 6.35 ms with 12 steps.
+constexpr int kFirSteps = (kFir + 15 + 3) / 4;
+constexpr int kFirLeastSteps = (26 + 15 + 3) / 4;  // one stencil has 26 taps
+__host__ __device__ constexpr int fir_steps(int taps) { return (taps + 15 + 3) >> 2; }
+constexpr bool fir_steps_cover()
+{
+    for (int taps = 26; taps <= kFir; ++taps) {
+        const int steps = fir_steps(taps), reach = taps + 15;  // output 15 reads columns 15 .. taps + 14
+        if (4 * steps < reach || 4 * (steps - 1) >= reach) return false;
+        if (steps < kFirLeastSteps || steps > kFirSteps) return false;
+    }
+    return true;
+}
+static_assert(fir_steps_cover(), "every nonzero tap of a block is in a step, and no step is empty");
 
 template <int NX>
 struct LtiRef {
@@ -638,7 +656,7 @@ struct LtiRef {
     int off[NG];       // d_m - i at the reference sample
     double e[NG];
     double delta[NG];  // d_m - i + 1 - e_m
-    int kmin;          // first tap of the composite filter, relative to i
+    int kmin, taps;    // first tap of the composite filter, relative to i, and their count
     bool ok;           // the filter fits in kFir taps
 };
 
@@ -661,7 +679,8 @@ __device__ __forceinline__ void lti_reference(double t, int i, double L, double 
         hi = max(hi, d - i);
     });
     ref.kmin = lo - (H - 1);
-    ref.ok = (hi + H) - ref.kmin + 1 <= kFir;
+    ref.taps = (hi + H) - ref.kmin + 1;
+    ref.ok = ref.taps <= kFir;
 }
 
 // Entry idx of the two composite filters: kind idx / kFir, tap kmin + idx % kFir; the groups
@@ -932,7 +951,27 @@ __device__ __forceinline__ void lagrange_weight_d(double A, double dA, const dou
     }
 }
 
-// Entry k (0 <= k < kFir) of both filters of pair p = c * kUtvLinks + q of the tile's model.
+// The X terms on base link q, four bits each in index order (first generation: the first two).
+constexpr unsigned utv_terms(int q)
+{
+    unsigned w = 0;
+    int n = 0;
+    for (int x = 0; x < 16; ++x)
+        if (utv_q(x) == q) w |= (unsigned)x << (4 * n++);
+    return w;
+}
+constexpr unsigned long long kUtvTerms01 = utv_terms(0) | (unsigned long long)utv_terms(1) << 16;
+constexpr unsigned long long kUtvTerms =
+    kUtvTerms01 | (utv_terms(2) | (unsigned long long)utv_terms(3) << 16) << 32;
+static_assert(kUtvTerms01 >> 32 == 0, "four terms a link");
+constexpr unsigned kUtvNegative = [] {
+    unsigned w = 0;
+    for (int x = 0; x < 16; ++x) w |= (stock::kX[x].sign < 0 ? 1u : 0u) << x;
+    return w;
+}();
+
+// Entry k (0 <= k < kFir) of both filters of pair p = c * kUtvLinks + q of the tile's model. Lanes of
+// any pairs share the loop over their links' terms.
 template <int NX>
 __device__ __forceinline__ void utv_filter_entry(const UtvShared &sh, const LagrangeView &lg,
                                                  const double *E_lds, int p, int k, double &f0,
@@ -942,14 +981,15 @@ __device__ __forceinline__ void utv_filter_entry(const UtvShared &sh, const Lagr
     const int c = p / kUtvLinks, q = p - c * kUtvLinks;
     f0 = 0.0;
     f1 = 0.0;
-    for (int x = 0; x < NX; ++x) {  // the pair's units in index order
-        if (utv_q(x) != q) continue;
+    const unsigned terms = (unsigned)(kUtvTerms >> (16 * q));
+    for (int n = 0; n < NX / kUtvLinks; ++n) {  // the pair's units in index order
+        const int x = (terms >> (4 * n)) & 15;
         const int u = c * NX + x;
         const int r = k + sh.kmin - (int)sh.off[u];
         if (r < -(H - 1) || r > H) continue;
         double w, dw;
         lagrange_weight_d(sh.A[u], sh.dA[u], E_lds, sh.e[u], r, w, dw);
-        const double sg = (double)stock::kX[x].sign;
+        const double sg = (kUtvNegative >> x) & 1 ? -1.0 : 1.0;
         f0 = __builtin_fma(sg, w, f0);
         f1 = __builtin_fma(-sg * sh.sigma[u], dw, f1);
     }

@@ -5,7 +5,7 @@ and those of the explicit window of that length."""
 import numpy as np
 import pytest
 
-from conftest import YRSID_SI, gb_waveform
+from conftest import YRSID_SI, check_mixed, gb_waveform, unequal_arms
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +75,37 @@ def test_unequal_arms_alone_and_in_a_batch(torch_gpu):
     plan.run()
     plan.check_errors()
     assert torch.equal(plan.out_all, got)
+
+
+@pytest.mark.parametrize("cls_name", ["EqualArmlengthOrbits", "CartwheelOrbits"])
+@pytest.mark.parametrize("tdi,dt", [("2nd generation", 15.0), ("2nd generation", 8.0),
+                                    ("2nd generation", 6.5), ("2nd generation", 4.2),
+                                    ("1st generation", 7.0)])
+def test_filters_of_every_length(torch_gpu, oracle_mod, cls_name, tdi, dt):
+    """Composite filters of 11 to 14 matrix steps against the oracle, on input as fast as order 25
+    interpolates well."""
+    import fastlisaresponse_amd.orbits as orbits_mod
+    torch = torch_gpu
+    orbits = getattr(orbits_mod, cls_name)(t_max=1.2 * YRSID_SI)
+    orbits.configure(linear_interp_setup=True)
+    oo = oracle_mod.OracleOrbits(*orbits.pycppdetector_args)
+    n, t0 = 9000, 1.0e6
+    f = 0.1 / dt
+    h = gb_waveform(n, dt, 1e-21, f, 1e-17, 0.7, 0.2, 0.4, t0=t0)
+    from fastlisaresponse_amd.batch import BatchedResponse
+    br = BatchedResponse(1.0 / dt, tdi=tdi, orbits=orbits, tdi_chan="XYZ", precision="mixed-c128",
+                         t_buffer=1000.0 * dt)
+    plan = br.plan(torch.as_tensor(h, device="cuda"), [n], [0.9], [-0.4], [t0])
+    plan.run()
+    plan.check_errors()
+    y, exp = oracle_mod.response_pipeline(oo, h, 0.9, -0.4, dt, 25, tdi, t0=t0, tdi_chan="XYZ",
+                                          x_base=orbits.x_base, nthreads=8,
+                                     t_buffer=1000.0 * dt)
+    got = torch.stack(plan.channels(0)).cpu().numpy().astype(np.float64)
+    # the outputs' float32 rounding, and positions within 1e-8 samples (times 2 pi f dt = 0.63) in each
+    # of up to 16 units of the projections' size
+    T = br.tdi_start_ind
+    units = 16 if tdi == "2nd generation" else 8
+    size = np.sqrt(np.mean(y[:, T:-T] ** 2)) / np.sqrt(np.mean(exp[:, T:-T] ** 2))
+    check_mixed(oracle_mod, oo, got, y, exp, t0, dt, tdi, "XYZ", 2.0 ** -24 + 0.63e-8 * units * size, T,
+                (), unequal_arms(orbits))
