@@ -35,7 +35,7 @@ struct Recip {
 // six units with one fraction, 30 instead of 36 of a complex stencil, 23 instead of 27 of one unit.
 // The exact forms are bound by these FP64 operations: 1-yr FP64 drop-in (3,153,600 samples) 1.125 ->
 // 0.961 ms with equal arms, 2.002 -> 1.769 ms with unequal ones, order 31 with a custom table
-// (262,145 samples) 0.135 -> 0.119 ms (interleaved A/B on one box).
+// (262,145 samples) 0.135 -> 0.119 ms (interleaved A/B).
 FLR_HOST_DEVICE inline double div_recip(double a, const Recip &r)
 {
     return __builtin_fma(a, r.y, a * r.l);

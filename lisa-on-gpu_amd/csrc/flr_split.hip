@@ -367,17 +367,18 @@ constexpr size_t kSplitLds = 64 * 1024;  // wider windows (fine sampling) keep t
 // Longest series that takes a split kernel, in samples per CU (256 CUs): where the one-lane kernel
 // fills the chip well enough to win by its smaller halo. One-lane -> split, us:
 //   projection: 98,304 samples 18.6 -> 16.3 (equal arms), 24.2 -> 23.8 (unequal); 131,072 19.7 -> 21.2
-//   equal-arm TDI: 163,841 samples 50.7 -> 44.2 (exact), 21.2 -> 20.0 (fast); 196,608 55.4 -> 53.3,
-//     21.9 -> 23.1
-//   unequal-arm stock TDI: exact 163,841 samples 99.3 -> 91.6, 196,608 104.2 -> 108.8; fast 98,304
+//   equal-arm TDI: exact 147,456 samples 45.4 -> 40.4, 163,840 46.0 -> 44.2 (131,072, where the one-lane
+//     groups come to exactly two a CU, 34.8 -> 36.9); fast 163,841 21.2 -> 20.0, 196,608 21.9 -> 23.1
+//   unequal-arm stock TDI: exact 81,920 samples 57.2 -> 46.2, 98,304 58.4 -> 54.9, 114,689 60.1 -> 63.0,
+//     131,072 64.2 -> 73.8; 1st generation 30.3 -> 29.2 and 32.5 -> 38.8 at 98,304 and 131,072; fast 98,304
 //     39.6 -> 36.1, 131,072 (1st generation) 22.6 -> 24.8
-//   any other table: 262,145 samples 77.2 -> 71.1, 524,289 138 -> 131, 1,048,577 239 -> 241 (its
-//     one-lane form loops over units and taps one load at a time); since then both take their reciprocals
-//     four at a time, 262,145 69.9 -> 62.5 and 1,048,577 232.6 -> 217.1
+//   any other table, exact, order 25: 147,456 samples 39.8 -> 32.6, 163,840 40.6 -> 37.2, 196,608
+//     43.4 -> 44.3, 524,288 100 -> 112; another order: 262,144 67.5 -> 61.8 (order 31), 524,288
+//     119 -> 117, 188 -> 181 (order 15; its one-lane form loops over taps, two pairs at a time)
 constexpr int kSplitProj = 384;
 constexpr int kSplitEqual = 640;
-constexpr int kSplitStock = 640;
-constexpr int kSplitStockFast = 384;
+constexpr int kSplitStock = 384;
+constexpr int kSplitTable25 = 640;
 constexpr int kSplitTable = 2048;
 
 static bool split_suits(int samples, int per_cu, size_t lds)
@@ -420,8 +421,8 @@ bool launch_tdi_split(const TdiConfig &cfg, const TdiSource &src, const OrbitVie
     const size_t vals = eq ? (form == kFast ? 3 * (nx == 8 ? 4 : 8) : 3 * nx) : kSplitUnits + kNLinks;
     const size_t shm = (rows + (vals + 3) * kSplit) * sizeof(double);
     const int limit = eq ? kSplitEqual
-                      : !use_stock(stock, lg) ? kSplitTable
-                      : form == kFast ? kSplitStockFast : kSplitStock;
+                      : use_stock(stock, lg) ? kSplitStock
+                      : form != kFast && lg.h == 13 ? kSplitTable25 : kSplitTable;
     if (form == kExact || !split_suits(src.num_delays, limit, shm)) return false;
     const int nb = tiles_for(src.num_delays, src.start, cfg.zero_edges, kSplit);
     const RowMap &rm = stock.rows;
