@@ -184,7 +184,9 @@ static_assert(group_kind(0) == 0 && group_kind(1) == 1 && group_kind(2) == 0 && 
 
 // Equal-arm stock TDI: wave m takes chain length m -- the six units of tdi_equal_arm's group m
 // (exact) or the three outputs of tdi_linear's (fast) -- and waves 0..2 add a channel's values in
-// index (exact) or chain-length (fast) order.
+// index (exact) or chain-length (fast) order. Exact forms: the window in paired rows, for ds_read_b128, and
+// the reciprocals four at a time where proven: 131,072 samples 37.0 -> 35.2 us (2nd generation), 19.7 ->
+// 17.9 us (1st), 8,192 samples 7.3 -> 6.7 and 6.0 -> 5.3 us, the same bits.
 template <int NX, int FORM>
 __global__ __launch_bounds__(kSplit *(stock::max_len(NX) + 1)) void tdi_split_equal_kernel(
     TdiConfig cfg, TdiSource src, OrbitView orb, LagrangeView lg, RowMap rm)
@@ -192,11 +194,12 @@ __global__ __launch_bounds__(kSplit *(stock::max_len(NX) + 1)) void tdi_split_eq
     constexpr int H = 13;
     constexpr int NG = stock::max_len(NX) + 1;
     constexpr int kVals = FORM ? NX : NG;  // per channel
-    extern __shared__ double smem[];
+    extern __shared__ __align__(16) double smem[];
     const int lane = threadIdx.x & 63, m = wave_index();
     const int cap = split_cap(cfg.win_cap);
-    double *ywin = smem;                       // [6][cap]
-    double *vals = smem + kNLinks * cap;       // [3][kVals][kSplit]
+    double *ywin = smem;                       // [6][cap], of double2 in the exact forms
+    double2 *pairs = reinterpret_cast<double2 *>(smem);
+    double *vals = smem + (FORM ? 2 : 1) * kNLinks * cap;  // [3][kVals][kSplit]
     double *sums = vals + 3 * kVals * kSplit;  // [3][kSplit]
     SplitTile st;
     if (!split_tile(cfg, src.out, 3, src.num_delays, src.num_inputs, src.start, src.t_arr, src.t0,
@@ -207,9 +210,8 @@ __global__ __launch_bounds__(kSplit *(stock::max_len(NX) + 1)) void tdi_split_eq
         double y[kNLinks];
 #pragma unroll
         for (int l = 0; l < kNLinks; ++l) y[l] = from[(size_t)rm.row[l] * src.num_inputs];
-        if constexpr (FORM) {  // canonical link order
-#pragma unroll
-            for (int l = 0; l < kNLinks; ++l) ywin[l * cap + jj] = y[l];
+        if constexpr (FORM) {
+            store_link_pairs(pairs + jj, cap, y);
         } else {
             double k[2][3];
             combine_links(y, k);
@@ -237,36 +239,30 @@ __global__ __launch_bounds__(kSplit *(stock::max_len(NX) + 1)) void tdi_split_eq
         split_delay(Dm, st.t0_offset, cfg.fs, d, e);
         bad = (d - st.win_lo - (H - 1) < 0) || (d - st.win_lo + H >= st.win_len);
         if (bad) d = st.win_lo + H - 1;  // in-window stand-in; the result is discarded
-        const bool odd = m & 1;
-        const double *xr[3][2];
+        const double2 *xr[3];  // paired rows as tdi_equal_arm_pairs, from the lowest tap on
         static_for<3>([&](auto c) {
-            static_for<2>([&](auto k) {
-                constexpr int even_row = stock::canon(stock::cyc(k == 0 ? 13 : 12, c));
-                constexpr int odd_row = stock::canon(stock::cyc(k == 0 ? 31 : 21, c));
-                int off = (odd ? odd_row : even_row) * cap + d - st.win_lo - (H - 1);
-                pin(off);
-                xr[c][k] = ywin + off;
-            });
+            int off = (2 * c + (m & 1)) * cap + d - st.win_lo - (H - 1);
+            pin(off);
+            xr[c] = pairs + off;
         });
         double S[3][2] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
-#pragma unroll
-        for (int j = 1; j < H; ++j) {
+        for_tap_pairs<FORM, H>(e, H, [&](int j, const auto &q) {
             const double E = lg.E[j - 1];
-            const PairDiv<FORM> q(j + e, j + (1 - e));
 #pragma unroll
-            for (int c = 0; c < 3; ++c)
-#pragma unroll
-                for (int k = 0; k < 2; ++k)
-                    S[c][k] += E * q.sum(xr[c][k][H + j], xr[c][k][H - 1 - j]);
-        }
+            for (int c = 0; c < 3; ++c) {
+                const double2 up = xr[c][H + j], dn = xr[c][H - 1 - j];
+                S[c][0] += E * q.sum(up.x, dn.x);
+                S[c][1] += E * q.sum(up.y, dn.y);
+            }
+        });
         const double A = lagrange_A_exact(lg, e, y_deps);
         const double B = 1.0 - e;
         const double C = e;
         const double D = e * (1.0 - e);
         static_for<3>([&](auto c) {
+            const double2 x0 = xr[c][H - 1], x1 = xr[c][H];
             static_for<2>([&](auto k) {
-                const double *p = xr[c][k] + (H - 1);
-                double val = A * (B * p[1] + C * p[0] + D * S[c][k]);
+                double val = A * (B * (k ? x1.y : x1.x) + C * (k ? x0.y : x0.x) + D * S[c][k]);
                 val *= kUnits[m].sign[k];
                 vals[(c * kVals + kUnits[m].x[k]) * kSplit + lane] = bad ? __builtin_nan("") : val;
             });
@@ -367,8 +363,8 @@ constexpr size_t kSplitLds = 64 * 1024;  // wider windows (fine sampling) keep t
 // Longest series that takes a split kernel, in samples per CU (256 CUs): where the one-lane kernel
 // fills the chip well enough to win by its smaller halo. One-lane -> split, us:
 //   projection: 98,304 samples 18.6 -> 16.3 (equal arms), 24.2 -> 23.8 (unequal); 131,072 19.7 -> 21.2
-//   equal-arm TDI: exact 147,456 samples 45.4 -> 40.4, 163,840 46.0 -> 44.2 (131,072, where the one-lane
-//     groups come to exactly two a CU, 34.8 -> 36.9); fast 163,841 21.2 -> 20.0, 196,608 21.9 -> 23.1
+//   equal-arm TDI: exact 98,304 samples 32.0 -> 25.7, 163,840 46.0 -> 43.4 (131,072, where the one-lane
+//     groups come to exactly two a CU, 34.8 -> 35.2), 1st generation 24.7 -> 22.0 at 163,840; fast 163,841 21.2 -> 20.0, 196,608 21.9 -> 23.1
 //   unequal-arm stock TDI: exact 81,920 samples 57.2 -> 46.2, 98,304 58.4 -> 54.9, 114,689 60.1 -> 63.0,
 //     131,072 64.2 -> 73.8; 1st generation 30.3 -> 29.2 and 32.5 -> 38.8 at 98,304 and 131,072; fast 98,304
 //     39.6 -> 36.1, 131,072 (1st generation) 22.6 -> 24.8
@@ -417,7 +413,7 @@ bool launch_tdi_split(const TdiConfig &cfg, const TdiSource &src, const OrbitVie
 {
     const bool eq = use_equal_arm(stock, lg);
     const int nx = stock.generation == 1 ? 8 : 16;
-    const size_t rows = (size_t)kNLinks * split_cap(cfg.win_cap);
+    const size_t rows = (size_t)(eq && form != kFast ? 2 : 1) * kNLinks * split_cap(cfg.win_cap);
     const size_t vals = eq ? (form == kFast ? 3 * (nx == 8 ? 4 : 8) : 3 * nx) : kSplitUnits + kNLinks;
     const size_t shm = (rows + (vals + 3) * kSplit) * sizeof(double);
     const int limit = eq ? kSplitEqual
@@ -427,9 +423,9 @@ bool launch_tdi_split(const TdiConfig &cfg, const TdiSource &src, const OrbitVie
     const int nb = tiles_for(src.num_delays, src.start, cfg.zero_edges, kSplit);
     const RowMap &rm = stock.rows;
 #define FLR_SPLIT(F)                                                                             \
-    (eq ? nx == 8 ? launch_tpb(tdi_split_equal_kernel<8, F == kFast ? kFast : kExact2>, nb,      \
+    (eq ? nx == 8 ? launch_tpb(tdi_split_equal_kernel<8, F>, nb,      \
                                4 * kSplit, shm, stream, cfg, src, orb, lg, rm)                   \
-                  : launch_tpb(tdi_split_equal_kernel<16, F == kFast ? kFast : kExact2>, nb,     \
+                  : launch_tpb(tdi_split_equal_kernel<16, F>, nb,     \
                                8 * kSplit, shm, stream, cfg, src, orb, lg, rm)                   \
      : lg.h == 13 ? launch_tpb(tdi_split_units_kernel<F, 13>, nb, kSplit * kSplitWaves, shm,     \
                                stream, cfg, src, orb, lg)                                        \
