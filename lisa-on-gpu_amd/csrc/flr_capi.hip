@@ -1259,9 +1259,16 @@ int flr_fused_bind(flr_batch *b, const flr_source *sources, int num_sources, con
     }
     // the tile the response's current tables give (they may have changed since the reserve)
     const bool uniform = sources_uniform(b->r, b->dt, b->fs, flags, fs.data(), num_sources);
-    const int passes = b->auto_shape ? auto_passes(b->r, b->dt, b->fs, flags, fs.data(), num_sources,
-                                                   uniform)
-                                     : b->tile_passes;
+    // The window is chosen when these lengths and start indexes are first bound (or the tables have
+    // changed since) and kept for every later bind of them, whatever the start times: a captured
+    // run or inner product holds the tile length and the tile count, and reads this bind's prefix.
+    bool choose = b->auto_shape &&
+                  (b->num_sources != num_sources || b->shape_version != b->r->version);
+    for (int s = 0; b->auto_shape && !choose && s < num_sources; ++s)
+        choose = b->h_fused[s].num_pts != fs[s].num_pts ||
+                 b->h_fused[s].tdi_start != fs[s].tdi_start;
+    const int passes = choose ? auto_passes(b->r, b->dt, b->fs, flags, fs.data(), num_sources, uniform)
+                              : b->tile_passes;
     ProjConfig pc;
     TdiConfig tc;
     StockTdi stock;
