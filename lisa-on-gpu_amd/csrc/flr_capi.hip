@@ -469,18 +469,23 @@ bool utv_suitable(const flr_orbits *o, int nx, int tile, double dt, double fs, d
     return utv_crossings(o, nx, tile, dt, fs, deps) < 0.5;
 }
 
-// Whether 1024-sample windows suit these orbits: few tiles cross a node of the A table (the
-// per-sample path of one long tile takes as long as six others), and the kinks of the arms at the
-// orbit nodes move no unit's position by more than 6e-10 samples off a tile of `tile` samples' model (a kink in mid-tile, every unit at the worst case). The
-// null channel T shows such deviations first: at the 1024-sample window on the cartwheel (5.6e-10) T of
-// a 2 mHz source is 3.6e-8 from the TDI with extended-precision delays, of which the float32 outputs
-// are 2.4e-8 (2.6e-8 at the 512-sample window), where FP64 delays, the reference's, are 5.1e-7 away;
-// kinks of 1.5e-12 s/s would take it to 2.2e-7 (7.6e-8 at 512).
+// Whether 1024-sample windows suit these orbits: few tiles cross a node of the A table (the per-sample
+// path of one long tile takes as long as six others), and a tile spans at most one orbit node, which its
+// model follows (utv_middle). Longer tiles keep the 512-sample window, whose model is one line
+// through the tile: the arms bend by as much within a tile however fine the orbit table is, and the null
+// channel T shows it (2 mHz on the cartwheel, float32 outputs included, from the TDI with
+// extended-precision delays, where FP64 delays, the reference's, are 5.1e-7 away): 3.6e-8 with a line at
+// the 1024-sample window, 2.5e-8 at 512, 2.4e-8 (the float32 rounding) with the node followed at 1024.
 bool utv_long_tiles(const flr_orbits *o, int nx, int tile, double dt, double fs, double deps)
 {
-    const int M = nx == 8 ? 3 : 7;
-    return utv_crossings(o, nx, tile, dt, fs, deps) < 0.1 &&
-           M * o->max_kink * dt * fs * tile / 4.0 <= 6e-10;
+    return utv_crossings(o, nx, tile, dt, fs, deps) < 0.1 && (double)(tile - 1) * dt <= o->dt;
+}
+
+// Whether the samples around an orbit node take a line for each side of it (kUtvTurn), every unit at the
+// worst case.
+int utv_sides(const flr_orbits *o, int nx, double dt, double fs)
+{
+    return (nx == 8 ? 3 : 7) * o->max_kink * dt * fs > kUtvTurn ? 1 : 0;
 }
 
 bool lti_source_uniform(const flr_orbits *o, const FusedSource &f, double dt, double fs, int nx,
@@ -1396,6 +1401,7 @@ int fused_launch(flr_batch *b, hipStream_t s, const void *data, double *sums)
         r->order == 25)  // inner products run in the filter form only
         tc.utv = data ? 1 : utv_suitable(r->orbits, stock.generation == 1 ? 8 : 16, tc.tile, b->dt,
                                          b->fs, r->deps) ? 1 : 0;
+    tc.utv_sides = utv_sides(r->orbits, stock.generation == 1 ? 8 : 16, b->dt, b->fs);
     if (b->flags & FLR_FLAG_MIXED) tc.orbit_stage = orbit_stage_fits(r->orbits, tc.win_cap, b->dt);
     if (data) {
         tc.inner_part = b->d_inner;
@@ -1741,6 +1747,7 @@ int flr_fused_run_static(flr_response *r, const flr_source *sources, int num_sou
         if (stock.generation != 0 && !stock.equal_arm && r->order == 25)
             tc.utv = utv_suitable(r->orbits, stock.generation == 1 ? 8 : 16, tc.tile, dt,
                                   sampling_frequency, r->deps) ? 1 : 0;
+        tc.utv_sides = utv_sides(r->orbits, stock.generation == 1 ? 8 : 16, dt, sampling_frequency);
         tc.orbit_stage = orbit_stage_fits(r->orbits, tc.win_cap, dt);
         hipError_t e = launch_lti_filters(tc, bf, orb, lg, stock, s);
         if (e != hipSuccess) return hip_fail(e, "composite filter launch");

@@ -328,12 +328,17 @@ __device__ __forceinline__ void lti_mfma(const TdiConfig &tc, const FusedSource 
 // v_mfma_f64_16x16x4f64 each, the link series' operand shared by the pair's two filters --
 // then X_c = F0 part + (i - m) F1 part, A, E, T formed from X, Y, Z in FP64, and stored.
 // filt: [2][kUtvPairs][kFpad] (F0 then F1, padded as fpad); link rows canonical at ywin +
-// k * pitch.
+// k * pitch. With kink (kUtvNodes windows) filt holds a second F1 after the first, for the samples after
+// m: the groups of either side take theirs, and the group that m lies in the F0 and F1 of the line closest
+// to its two (three more operations per pair and step in one wave of four), or, where the orbits' slopes
+// change too much for that (tc.utv_sides), is done once for each side, by two waves. 8 sources, 4.2e6 samples: 509 us
+// without the second F1, 534 with it; 609 with that group done twice (the second wave shares its SIMD's
+// matrix core with another group's).
 template <typename OT, int TPB>
 __device__ __forceinline__ void utv_mfma(const TdiConfig &tc, const FusedSource &src, int first,
-                                         int last, int m, int yw_lo, int yw_len, int kmin, int steps,
-                                         const double *ywin, int pitch, int R, const double *filt,
-                                         InnerShared *ish)
+                                         int last, int m, bool kink, int yw_lo, int yw_len, int kmin,
+                                         int steps, const double *ywin, int pitch, int R,
+                                         const double *filt, InnerShared *ish)
 {
     const bool inner = ish != nullptr;  // (inner-product kernels only)
     typedef double d4 __attribute__((ext_vector_type(4)));
@@ -343,35 +348,65 @@ __device__ __forceinline__ void utv_mfma(const TdiConfig &tc, const FusedSource 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int nb = lane & 15, kq = lane >> 4;
     const size_t n = (size_t)src.num_pts;
-    for (int g = wave; g < ngc; g += TPB / 64) {
+    const bool sides = kUtvNodes<TPB> && kink && tc.utv_sides;
+    for (int w = __builtin_amdgcn_readfirstlane(wave); w < ngc + (sides ? 1 : 0); w += TPB / 64) {
+        const bool again = w == ngc;  // m's group a second time, for the samples after m
+        const int g = again ? (((m - T) >> 4) - q0) >> 4 : w;
         const int qb = q0 + 16 * g + nb;
         // window column of this lane's tap step 0 (>= -15: the tile's taps fit its window)
         const int w0 = T + 16 * min(qb, q1) + kmin - yw_lo + kq;
         int b[4];  // tap step j = 4a + i at b[i] + a
 #pragma unroll
         for (int i = 0; i < 4; ++i) b[i] = blk_col(w0 + 4 * i, R);
+        // the group's samples relative to m: before (lo < hi <= 0) and after, or on both sides of it
+        const int lo = max(first, T + 16 * (q0 + 16 * g)) - m;
+        const int hi = min(last, T + 16 * (q0 + 16 * g) + 255) - m;
+        const bool both = kUtvNodes<TPB> && kink && lo < 0 && hi > 0;
+        const int from = again ? m + 1 : first, to = sides && both && !again ? m : last;
         d4 a0[3], a1[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) a0[c] = a1[c] = d4{0.0, 0.0, 0.0, 0.0};
         const double *fl = filt + kFpadLo + kq - nb;  // fl[p * kFpad + 4j] = F0_p[4j + kq - nb]
+        // f(p, j): the F0 and F1 operands of pair p at tap step j
+        auto steps_of = [&](auto f) {
 #pragma unroll
-        for (int j = 0; j < kFirSteps; ++j) {
-            if (j >= kFirLeastSteps && j >= steps) break;
-            const int col = b[j & 3] + (j >> 2);
-            static_for<6>([&](auto l) {  // canonical link l: one operand for its two pairs
-                const double yv = ywin[l * pitch + col];
-                static_for<3>([&](auto c) {
-                    static_for<kUtvLinks>([&](auto q) {
-                        if constexpr (stock::canon(stock::cyc(kUtvLink[q], c)) == l) {
-                            constexpr int p = c * kUtvLinks + q;
-                            a0[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(fl[p * kFpad + 4 * j], yv,
-                                                                         a0[c], 0, 0, 0);
-                            a1[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                                fl[(kUtvPairs + p) * kFpad + 4 * j], yv, a1[c], 0, 0, 0);
-                        }
+            for (int j = 0; j < kFirSteps; ++j) {
+                if (j >= kFirLeastSteps && j >= steps) break;
+                const int col = b[j & 3] + (j >> 2);
+                static_for<6>([&](auto l) {  // canonical link l: one operand for its two pairs
+                    const double yv = ywin[l * pitch + col];
+                    static_for<3>([&](auto c) {
+                        static_for<kUtvLinks>([&](auto q) {
+                            if constexpr (stock::canon(stock::cyc(kUtvLink[q], c)) == l) {
+                                double f0, f1;
+                                f(c * kUtvLinks + q, j, f0, f1);
+                                a0[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(f0, yv, a0[c], 0, 0, 0);
+                                a1[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(f1, yv, a1[c], 0, 0, 0);
+                            }
+                        });
                     });
+                    __asm__ volatile("" ::: "memory");  // one link's operands in flight at a time
                 });
-                __asm__ volatile("" ::: "memory");  // one link's operands in flight at a time
+            }
+        };
+        if (both && !sides) {
+            // |i - m| over the group's samples by its least-squares line alpha + beta (i - m)
+            const double A = -lo, B = hi, N = A + B;
+            const double beta = (B - A) * (A * A + 4.0 * A * B + B * B) / (N * N * N);
+            const double half_alpha = 0.25 * ((A * A + B * B) / N - beta * (B - A));
+            const double part = 0.5 + 0.5 * beta;
+            steps_of([&](int p, int j, double &f0, double &f1) {
+                const double *x = fl + p * kFpad + 4 * j;
+                const double before = x[kUtvPairs * kFpad], d = x[2 * kUtvPairs * kFpad] - before;
+                f0 = __builtin_fma(half_alpha, d, x[0]);
+                f1 = __builtin_fma(part, d, before);
+            });
+        } else {
+            const bool after = kUtvNodes<TPB> && kink && (again || lo >= 0);
+            const double *fd = fl + (after ? 2 : 1) * kUtvPairs * kFpad;
+            steps_of([&](int p, int j, double &f0, double &f1) {
+                f0 = fl[p * kFpad + 4 * j];
+                f1 = fd[p * kFpad + 4 * j];
             });
         }
         InnerAcc ia;
@@ -379,7 +414,7 @@ __device__ __forceinline__ void utv_mfma(const TdiConfig &tc, const FusedSource 
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int i = T + 16 * qb + 4 * v + kq;
-            if (qb > q1 || i < first || i > last) continue;
+            if (qb > q1 || i < from || i > to) continue;
             const double di = (double)(i - m);
             const double X = __builtin_fma(di, a1[0][v], a0[0][v]);
             const double Y = __builtin_fma(di, a1[1][v], a0[1][v]);
@@ -652,8 +687,7 @@ void fused_lti_kernel(ProjConfig pc, TdiConfig tc, Batch<FusedSource> batch, Orb
 // rows canonical and padded), the tile's unit model (utv_unit) computed beside the projection,
 // then either the slowly-varying-arm filters on the matrix cores (utv_mfma) or, for a tile
 // that fails the model's tests, the per-sample stencils. LDS: the h window, whose space holds
-// the filters once the projection is done ([2][kUtvPairs][kFpad] doubles at most), then the
-// six padded rows.
+// the filters once the projection is done (utv_filter_doubles at most), then the six padded rows.
 template <int NX, typename HT, int PASSES, int TPB, bool STAGED>
 __device__ __forceinline__ void fused_tile_utv(const ProjConfig &pc, const TdiConfig &tc,
                                                const FusedSource &src, int tile,
@@ -703,16 +737,22 @@ __device__ __forceinline__ void fused_tile_utv(const ProjConfig &pc, const TdiCo
     const int hw_len = min(n, yw_lo + yw_len + pc.halo_hi) - hw_lo;
     double2 *hwin = reinterpret_cast<double2 *>(smem);
     double *filt = smem;  // after the projection
-    double *ywin = smem + max(2 * pc.win_cap, 2 * kUtvPairs * kFpad);  // [6][pitch]
+    double *ywin = smem + max(2 * pc.win_cap, utv_filter_doubles(TPB));  // [6][pitch]
     const double t0_offset = src.t0 + (double)0 * pc.dt;
-    const int m = (first + last) >> 1;
     // the times and light travel times at the tile's first, middle and last sample
-    if (tid < 3)
-        utv_reference_times(sh, tid, tid == 0 ? first : tid == 1 ? m : last, src.t0, tc.dt, orb, rm);
-    if (tid == 0) {
-        sh.kmin = 1 << 30;
-        sh.kmax = -(1 << 30);
-        sh.ok = 1;
+    if (tid < 3) {
+        bool node;
+        const int mid = utv_middle<kUtvNodes<TPB>>(orb, src.t0, tc.dt, first, last, node);
+        utv_reference_times(sh, tid, tid == 0 ? first : tid == 1 ? mid : last, src.t0, tc.dt, orb, rm);
+        if (tid == 0) {
+            sh.kmin = 1 << 30;
+            sh.kmax = -(1 << 30);
+            sh.ok = 1;
+            sh.m = mid;
+            sh.kink = node;
+            sh.per[0] = 1.0 / (double)(node ? mid - first : max(last - first, 1));
+            sh.per[1] = node ? 1.0 / (double)(last - mid) : 0.0;
+        }
     }
     for (int jj = tid; jj < hw_len; jj += TPB) hwin[jj] = load_h<HT>(src.h, hw_lo + jj);
     blk_zero(ywin, pitch, R, yw_len, tid, TPB);  // before the window's stores
@@ -722,7 +762,7 @@ __device__ __forceinline__ void fused_tile_utv(const ProjConfig &pc, const TdiCo
         ost = stage_orbit_nodes(orb, src.t0 + (double)yw_lo * pc.dt, s_orb, tid, TPB);
     }
     __syncthreads();
-    if (tid < 3 * NX) utv_unit<NX>(sh, tid, s_chain[tid], first, m, last, t0_offset, tc.fs, lg);
+    if (tid < 3 * NX) utv_unit<NX>(sh, tid, s_chain[tid], first, last, t0_offset, tc.fs, lg);
 
     bool bad = false;
     for (int w = tid; w < yw_len; w += TPB) {
@@ -752,17 +792,22 @@ __device__ __forceinline__ void fused_tile_utv(const ProjConfig &pc, const TdiCo
         // kernel's vector instructions less: 8 sources, 4.2e6 samples, 582 -> 539 us with fir_steps
         for (int x = tid; x < kUtvPairs * kFpad; x += TPB) {
             const int k = x % kFpad - kFpadLo;
-            if (k < 0 || k >= nt) filt[x] = filt[kUtvPairs * kFpad + x] = 0.0;
+            if (k < 0 || k >= nt) {
+                filt[x] = filt[kUtvPairs * kFpad + x] = 0.0;
+                if (kUtvNodes<TPB>) filt[2 * kUtvPairs * kFpad + x] = 0.0;
+            }
         }
         for (int x = tid; x < kUtvPairs * nt; x += TPB) {
             const int p = x / nt, k = x - p * nt;
-            double f0, f1;
+            double f0, f1[2];
             utv_filter_entry<NX>(sh, lg, s_E, p, k, f0, f1);
-            filt[p * kFpad + kFpadLo + k] = f0;
-            filt[(kUtvPairs + p) * kFpad + kFpadLo + k] = f1;
+            double *f = filt + p * kFpad + kFpadLo + k;
+            f[0] = f0;
+            f[kUtvPairs * kFpad] = f1[0];
+            if (kUtvNodes<TPB>) f[2 * kUtvPairs * kFpad] = f1[1];
         }
         __syncthreads();
-        utv_mfma<float, TPB>(tc, src, first, last, m, yw_lo, yw_len, kmin,
+        utv_mfma<float, TPB>(tc, src, first, last, sh.m, sh.kink, yw_lo, yw_len, kmin,
                              __builtin_amdgcn_readfirstlane(fir_steps(nt)), ywin, pitch, R, filt, ish);
     } else {
 #pragma unroll 1

@@ -122,6 +122,7 @@ struct TdiConfig {
     const char *inner_data = nullptr;
     int utv = 1;  // mixed stock tables, unequal arms: 1 = the slowly-varying-arm filter form,
                   // 0 = the per-sample kernel (utv_suitable)
+    int utv_sides = 0;  // the group of samples around an orbit node once for each side (kUtvTurn)
     int orbit_stage = 0;  // mixed matrix-core kernels: 1 = every tile's orbit nodes fit the LDS
                           // stage (orbit_stage_fits), so the staged variants run
 };
@@ -196,7 +197,7 @@ constexpr size_t kMaxLds = 160 * 1024;
 
 // Static LDS of a mixed matrix-core kernel at most: the E and orbit-node copies, the unit model of
 // the unequal-arm form, the inner-product slots.
-constexpr size_t kFusedStaticLds = 6656;
+constexpr size_t kFusedStaticLds = 6912;
 
 // CUs of the current device (looked up once).
 int compute_units();

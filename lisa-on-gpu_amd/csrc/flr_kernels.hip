@@ -472,7 +472,7 @@ size_t fused_lds_bytes(const ProjConfig &pc, const TdiConfig &tc, bool generic, 
                        int passes, bool utv)
 {
     if (utv)  // h window or the filters, then the padded rows (fused_tile_utv)
-        return ((size_t)std::max(2 * pc.win_cap, 2 * kUtvPairs * kFpad) +
+        return ((size_t)std::max(2 * pc.win_cap, utv_filter_doubles(passes == 4 ? 2 * kBlock : kBlock)) +
                 (size_t)kNLinks * blk_pitch(tc.win_cap)) *
                sizeof(double);
     const size_t doubles =

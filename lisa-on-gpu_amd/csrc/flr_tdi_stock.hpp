@@ -736,8 +736,15 @@ __device__ __forceinline__ bool lti_matches(double t, int i, double L, double t0
 //   F0_cq[k] = sum_{u in (c,q)} sign_u w_{k+kmin-off_u}(e_u),
 //   F1_cq[k] = -sum_{u in (c,q)} sign_u sigma_u w'_{k+kmin-off_u}(e_u),
 // with off_u = d_u - m and e_u taken at m: 24 composite filters per tile, applied on the matrix
-// cores. The reference positions are computed in double-double (utv_unit), so unlike the
-// per-sample delays they carry no FP64 rounding of the times. The weights are the fast stencil's
+// cores. Where a 1024-sample tile spans an orbit node, m is the sample at the node (the chains'
+// light travel times are all taken at the sample's own time, so every unit's slope changes there),
+// sigma_u the slope of the sample's side of it and F1 a filter for each side; the 256 samples around the
+// node that the matrix cores take together get the line closest to their two (utv_mfma; kUtvTurn). One line
+// through the tile was off the positions by up to 5.6e-10 samples in mid-tile on the cartwheel, which the
+// null channel T showed: at 2 mHz by 2.65e-8 of T (1.15e-8 with the line through the middle of a
+// 512-sample window), with the node followed by 3e-9. The reference positions are computed in
+// double-double (utv_unit), so unlike the per-sample delays they carry no FP64 rounding of the times. The
+// weights are the fast stencil's
 // (lagrange_weight_d), so the result differs from stencils at exact delays by the model's
 // position error (at most kLtiTol, tested per unit on the tile's two ends and middle), the
 // second-order term (|sigma| (b - a) / 2 <= kUtvDrift keeps it
@@ -746,8 +753,23 @@ __device__ __forceinline__ bool lti_matches(double t, int i, double L, double t0
 // takes the per-sample stencils instead.
 constexpr double kUtvDrift = 1e-4;
 constexpr double kUtvKnot = 3e-8;
+// The largest change of a position's slope at an orbit node, per sample, up to which the 256 samples around
+// it that the matrix cores take together get one line (tc.utv_sides otherwise): |i - m| is off its
+// least-squares line by at most 64 there, so a position by 32 times this, 1e-10 samples. On the cartwheel,
+// 2.3e-12, it leaves 4e-9 of the null channel T of a 2 mHz source.
+constexpr double kUtvTurn = 3e-12;
 constexpr int kUtvLinks = 4;                  // base links per channel (q)
 constexpr int kUtvPairs = 3 * kUtvLinks;      // (channel, base link) filters per kind
+// Whether the tiles of workgroups of `tpb` lanes follow an orbit node (the 1024-sample window): it holds a
+// third set of filters, which there takes the space of the h window, so two workgroups still share a
+// CU's LDS; the shorter windows, whose h windows are smaller, would lose one, and their line through the
+// tile is the closer one.
+template <int TPB>
+constexpr bool kUtvNodes = TPB > kBlock;
+__host__ __device__ constexpr int utv_filter_doubles(int tpb)
+{
+    return (tpb > kBlock ? 3 : 2) * kUtvPairs * kFpad;
+}
 constexpr int kUtvLink[kUtvLinks] = {13, 31, 12, 21};  // X's base links in order of first use
 
 // Base-link index q of X term x.
@@ -792,14 +814,42 @@ __device__ __forceinline__ DD dd_prod(double a, double b)
 
 // Per-tile model of the units, in LDS: the tile's first, middle and last sample time and the six
 // light travel times there (canonical order), in double-double; per unit (channel * NX + term)
-// off_u, e_u, sigma_u; the filters' tap range over all units and whether every unit passed.
+// off_u, e_u, sigma_u before and after the middle sample; the filters' tap range over all units and
+// whether every unit passed; the middle sample, whether an orbit node lies there (utv_middle), and the
+// reciprocals of the samples from the first to it and from it to the last (without a node: of all of them).
 struct UtvShared {
     double th[3], tl[3];
     double Lh[3][6], Ll[3][6];
-    double off[48], e[48], sigma[48];
+    double off[48], e[48], sigma[2][48];
     double A[48], dA[48];  // the interpolated A table at e_u and its slope in e
-    int kmin, kmax, ok;
+    int kmin, kmax, ok, m, kink;
+    double per[2];
 };
+
+// The window of the orbit tables that time t falls in, as orbit_node<kFast> picks it.
+__device__ __forceinline__ int utv_window(const OrbitView &orb, double t)
+{
+    const double q = t * orb.inv_dt;
+    return !(q >= 0.0) ? 0 : (q >= (double)(orb.N - 1) ? orb.N - 2 : (int)q);
+}
+
+// The model's middle sample of the tile [a, b]: with TWO, the sample nearest to the orbit node that the
+// tile spans if it spans one and that sample is not one of its ends (then kink), and otherwise half way.
+template <bool TWO>
+__device__ __forceinline__ int utv_middle(const OrbitView &orb, double t0, double dt, int a, int b,
+                                          bool &kink)
+{
+    kink = false;
+    if constexpr (TWO) {
+        const int wa = utv_window(orb, t0 + (double)a * dt), wb = utv_window(orb, t0 + (double)b * dt);
+        if (wb == wa + 1) {
+            const double at = rint((orb.dt * (double)wb - t0) / dt);
+            kink = at > (double)a && at < (double)b;
+            if (kink) return (int)at;
+        }
+    }
+    return (a + b) >> 1;
+}
 
 // Reference sample s (0: first, 1: middle, 2: last) of the tile at sample i: t0 + i dt and the
 // orbit tables' linear interpolant L_k(t) = v_k + slope_k (t - dt w) of every link, in
@@ -809,8 +859,7 @@ __device__ __forceinline__ void utv_reference_times(UtvShared &sh, int s, int i,
                                                     const RowMap &rm)
 {
     const DD t = dd_add({t0, 0.0}, dd_prod((double)i, dt));
-    const double q = t.hi * orb.inv_dt;
-    const int w = !(q >= 0.0) ? 0 : (q >= (double)(orb.N - 1) ? orb.N - 2 : (int)q);
+    const int w = utv_window(orb, t.hi);
     const DD tau = dd_add(t, dd_neg(dd_prod(orb.dt, (double)w)));
     const double *p = orb.table + (size_t)w * kOrbitStride;
     sh.th[s] = t.hi;
@@ -839,10 +888,12 @@ __device__ __forceinline__ int utv_chain_word(int u, int nx)
 }
 
 template <int NX>
-__device__ __forceinline__ void utv_unit(UtvShared &sh, int u, int chain, int a, int m, int b,
+__device__ __forceinline__ void utv_unit(UtvShared &sh, int u, int chain, int a, int b,
                                          double t0_offset, double fs, const LagrangeView &lg)
 {
     constexpr int H = 13;
+    const int m = sh.m;
+    const bool kink = sh.kink;
     double pos[3];
     int off_m = 0;
     double e_m = 0.0;
@@ -875,46 +926,62 @@ __device__ __forceinline__ void utv_unit(UtvShared &sh, int u, int chain, int a,
             e_m = e;
         }
     }
-    const double sigma = b > a ? (pos[2] - pos[0]) / (double)(b - a) : 0.0;
-    // (1) the line through the middle position with the chord's slope is off the positions at
-    // a and b by dev, and off any position in between by at most 3 dev (the positions are
-    // piecewise linear in i between the orbit nodes); the model takes the line half way between it
-    // and the chord, whose mean error over the tile is about zero: the rms error of a kink anywhere in
-    // the tile drops to 0.75 of the line's through the middle (null channel T against
-    // extended-precision delays, kinks of 1.5e-12 s/s: 9.9e-8 -> 7.6e-8 at the 512-sample window)
-    const double off_chord = pos[0] + sigma * (double)(m - a) - pos[1];
-    const double dev = fabs(off_chord);
-    bool ok = 3.0 * dev <= kLtiTol;
-    e_m -= 0.5 * off_chord;
+    double before, after;  // the drift per sample on either side of m
+    bool ok;
+    if (kink) {
+        // (1) the positions are linear from a to the node and from there to b, so two lines meeting at
+        // m, half a sample from the node at most, are off them by at most half the change of the drift
+        before = (pos[1] - pos[0]) * sh.per[0];
+        after = (pos[2] - pos[1]) * sh.per[1];
+        ok = 0.5 * fabs(after - before) <= kLtiTol;
+    } else {
+        // (1) the line through the middle position with the chord's slope is off the positions at
+        // a and b by dev, and off any position in between by at most 3 dev (the positions are
+        // piecewise linear in i between the orbit nodes); the model takes the line half way between it
+        // and the chord, whose mean error over the tile is about zero: the rms error of a kink anywhere in
+        // the tile drops to 0.75 of the line's through the middle (null channel T against
+        // extended-precision delays, kinks of 1.5e-12 s/s: 9.9e-8 -> 7.6e-8 at the 512-sample window)
+        before = after = (pos[2] - pos[0]) * sh.per[0];
+        const double off_chord = pos[0] + before * (double)(m - a) - pos[1];
+        ok = 3.0 * fabs(off_chord) <= kLtiTol;
+        e_m -= 0.5 * off_chord;
+    }
     // (2) drift across the tile
-    const double drift = fabs(sigma) * (double)max(m - a, b - m);
-    ok = ok && drift <= kUtvDrift;
-    // (3) e over the tile, [e_m - drift, e_m + drift], within the A-table segment of e_m, or past one of
-    // its nodes by `over`: then A's chord over that range, moved half way to A(e_m), is off A by at most
-    // (3/4 - over / (2 drift)) over <= 0.28 drift times the change of slope at the node. (At the ends of
-    // [0, 1] the stencil itself moves by a sample: there `over` counts in full.) On the cartwheel no
-    // tile of 1024 samples fails any more; before, about 1 in 150 did, and one tile's per-sample
-    // path takes ~100 us (2nd generation, dt = 5 s, 1024-sample window: 262,144 samples 161 -> 77 us,
-    // 2,000,000 375 -> 297 us)
-    const double s_m = e_m * lg.inv_deps, s_d = drift * lg.inv_deps;
+    const double da = before * (double)(m - a), db = -after * (double)(b - m);  // e at a, b less e_m
+    ok = ok && fmax(fabs(da), fabs(db)) <= kUtvDrift;
+    // (3) e over the tile, from e_m + lo to e_m + hi, within the A-table segment of e_m, or past one of
+    // its nodes: then A's chord over that range, moved half way to A(e_m), is off A by half the chord's
+    // error at e_m, or at the node by the chord's error there less that half: within 0.28 of half the
+    // range times the change of slope at the node when e_m is its middle. (At the ends of
+    // [0, 1] the stencil itself moves by a sample: there the part past the node counts in full.) On the
+    // cartwheel no tile of 1024 samples fails any more; before, about 1 in 150 did, and one tile's
+    // per-sample path takes ~100 us (2nd generation, dt = 5 s, 1024-sample window: 262,144 samples
+    // 161 -> 77 us, 2,000,000 375 -> 297 us)
+    const double lo = fmin(0.0, fmin(da, db)), hi = fmax(0.0, fmax(da, db));
+    const double s_m = e_m * lg.inv_deps, s_lo = s_m + lo * lg.inv_deps, s_hi = s_m + hi * lg.inv_deps;
     const int ind = min(max((int)s_m, 0), lg.num_A - 2);
-    const double over = fmax(fmax((double)ind - (s_m - s_d), (s_m + s_d) - (double)(ind + 1)),
-                             0.0) / lg.inv_deps;
     const double2 as = lg.Aslope[ind];  // A as lagrange_A_fast interpolates it, and its slope
     double A_m = __builtin_fma(as.y, s_m - (double)ind, as.x), dA_m = as.y * lg.inv_deps;
-    if (over > 0.0) {
-        if (s_m - s_d < 0.0 || s_m + s_d > (double)(lg.num_A - 1)) {
-            ok = ok && over <= kUtvKnot;
+    const double under = (double)ind - s_lo, over = s_hi - (double)(ind + 1);
+    const double past = fmax(fmax(under, over), 0.0);
+    if (past > 0.0) {
+        if (s_lo < 0.0 || s_hi > (double)(lg.num_A - 1)) {
+            ok = ok && past / lg.inv_deps <= kUtvKnot;
         } else {
-            const double lo = lagrange_A_fast(lg, e_m - drift), hi = lagrange_A_fast(lg, e_m + drift);
-            ok = ok && over * (0.75 - over / (2.0 * drift)) <= kUtvKnot;
-            A_m = 0.5 * A_m + 0.25 * (lo + hi);
-            dA_m = (hi - lo) / (2.0 * drift);
+            // the chord's error at the node and at e_m, for a unit change of slope there
+            const double W = s_hi - s_lo;
+            const double far = (under > over ? s_hi - s_m : s_m - s_lo) / W;  // e_m's end opposite the node
+            const double at_node = past * (W - past) / W, at_m = past * far;
+            ok = ok && fmax(0.5 * at_m, at_node - 0.5 * at_m) / lg.inv_deps <= kUtvKnot;
+            const double A_lo = lagrange_A_fast(lg, e_m + lo), A_hi = lagrange_A_fast(lg, e_m + hi);
+            dA_m = (A_hi - A_lo) / (hi - lo);
+            A_m = 0.5 * (A_m + __builtin_fma(-lo, dA_m, A_lo));
         }
     }
     sh.off[u] = (double)off_m;
     sh.e[u] = e_m;
-    sh.sigma[u] = sigma;
+    sh.sigma[0][u] = before;
+    sh.sigma[1][u] = after;
     sh.A[u] = A_m;
     sh.dA[u] = dA_m;
     atomicMin(&sh.kmin, off_m - (H - 1));
@@ -970,17 +1037,17 @@ constexpr unsigned kUtvNegative = [] {
     return w;
 }();
 
-// Entry k (0 <= k < kFir) of both filters of pair p = c * kUtvLinks + q of the tile's model. Lanes of
-// any pairs share the loop over their links' terms.
+// Entry k (0 <= k < kFir) of the filters of pair p = c * kUtvLinks + q of the tile's model: F0, and F1
+// before (f1[0]) and after (f1[1]) the middle sample. Lanes of any pairs share the loop over their
+// links' terms.
 template <int NX>
 __device__ __forceinline__ void utv_filter_entry(const UtvShared &sh, const LagrangeView &lg,
                                                  const double *E_lds, int p, int k, double &f0,
-                                                 double &f1)
+                                                 double (&f1)[2])
 {
     constexpr int H = 13;
     const int c = p / kUtvLinks, q = p - c * kUtvLinks;
-    f0 = 0.0;
-    f1 = 0.0;
+    f0 = f1[0] = f1[1] = 0.0;
     const unsigned terms = (unsigned)(kUtvTerms >> (16 * q));
     for (int n = 0; n < NX / kUtvLinks; ++n) {  // the pair's units in index order
         const int x = (terms >> (4 * n)) & 15;
@@ -991,7 +1058,8 @@ __device__ __forceinline__ void utv_filter_entry(const UtvShared &sh, const Lagr
         lagrange_weight_d(sh.A[u], sh.dA[u], E_lds, sh.e[u], r, w, dw);
         const double sg = (kUtvNegative >> x) & 1 ? -1.0 : 1.0;
         f0 = __builtin_fma(sg, w, f0);
-        f1 = __builtin_fma(-sg * sh.sigma[u], dw, f1);
+        f1[0] = __builtin_fma(-sg * sh.sigma[0][u], dw, f1[0]);
+        f1[1] = __builtin_fma(-sg * sh.sigma[1][u], dw, f1[1]);
     }
 }
 
