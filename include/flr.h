@@ -221,7 +221,9 @@ int flr_batch_run(flr_batch *batch, void *stream);
  * h. From these the white-noise inner products and log-likelihood follow, and the real part of
  * get_overlap's rfft overlap by Parseval (the DC and Nyquist bins from sums 2 and 3). Mixed
  * fused batches (FLR_FLAG_MIXED) with a stock TDI table at order 25 (FLR_ERR_UNSUPPORTED
- * otherwise); deterministic (fixed reduction order). The per-tile sums live in a device buffer
+ * otherwise); deterministic (fixed reduction order), and a source's sums are the same bits
+ * whatever other sources the batch holds and whatever its launch shape: the inner products'
+ * window follows the response and the sampling alone. The per-tile sums live in a device buffer
  * of the batch, allocated at the first call and when the batch's tile count grows (so the
  * first call must not be under stream capture); later calls allocate nothing. */
 int flr_fused_inner(flr_batch *batch, const void *data_all, double *sums, void *stream);

@@ -147,6 +147,15 @@ struct flr_response {
     }
 };
 
+// The tiles of a fused launch over a batch's sources.
+struct FusedTiling {
+    int passes = kFusedPasses;  // the tile's window is passes * kBlock samples
+    int len = 0;                // output samples per tile (make_fused_config; 0: not tiled yet)
+    int total = 0;
+    int *d = nullptr;           // [num_sources + 1] prefix sums
+    int *h = nullptr;           // their pinned staging copy
+};
+
 struct flr_batch {
     flr_response *r = nullptr;
     int flags = 0;
@@ -160,26 +169,22 @@ struct flr_batch {
     int proj_tiles = 0, tdi_tiles = 0;
     int proj_min_start = 0, tdi_min_start = 0;  // smallest start index over the sources
     int fused_min_start = 0;      // smallest tdi_start over the bound sources
-    bool fused = false;           // one fused launch over d_fused / d_fused_tiles
+    bool fused = false;           // one fused launch over d_fused and tiles.d
     FusedSource *d_fused = nullptr;
-    int *d_fused_tiles = nullptr;
-    int fused_tiles = 0;
     int capacity = 0;             // fused: sources the tables hold
-    int tile_passes = kFusedPasses;  // fused: the tile's window is tile_passes * kBlock samples
-    bool auto_shape = true;          // ... chosen by auto_passes until flr_batch_set_launch sets it
-    uint64_t shape_version = ~0ull;  // response version auto_passes chose it for
-    int tile_len = 0;                // fused: output samples per tile (make_fused_config)
+    FusedTiling tiles;            // fused: the runs' tiles, their window chosen by auto_passes until
+    bool auto_shape = true;       // flr_batch_set_launch sets it
+    FusedTiling inner;            // ... and the inner products' (inner_passes)
+    uint64_t shape_version = ~0ull;  // response version the windows were chosen for
     int grid_per_cu = 32;            // persistent workgroups per CU (the autotuner's usual pick)
-    FusedSource *h_fused = nullptr;  // pinned staging of the source table and tile prefix
-    int *h_fused_tiles = nullptr;
+    FusedSource *h_fused = nullptr;  // pinned staging of the source table
     hipEvent_t uploaded = nullptr;   // the last bind's upload
     hipEvent_t ran = nullptr;        // the last run's launch: a bind on any stream waits for it
     bool ran_recorded = false;       // `ran` has been recorded at least once
     double *d_lti = nullptr;         // mixed fused: [capacity][kLtiRecord] composite TDI filters
     uint64_t lti_version = ~0ull;    // response version the filters were built for (none yet)
     bool lti_uniform = false;        // every bound source clears the composite-filter tile test
-    uint64_t uniform_version = ~0ull;  // response version and tile length lti_uniform holds for
-    int uniform_tile = 0;
+    uint64_t uniform_version = ~0ull;  // response version lti_uniform holds for
     const void *out_base = nullptr;  // fused: the bound out_all (inner-product launches)
     double *d_inner = nullptr;       // fused inner products: per tile [3][kInnerSums] sums
     int64_t inner_cap = 0;           // tiles d_inner holds
@@ -550,7 +555,33 @@ int make_fused_config(const flr_response *r, double dt, double fs, int flags, in
     return FLR_OK;
 }
 
-// Window of a fused launch nobody chose a shape for, in units of kBlock samples: 1, 2 or 4 for the
+// The inner products' window in units of kBlock samples, 0 where a batch has none. A source's sums are
+// grouped by tile, so the window follows the response and the sampling alone: a walker's sums and
+// likelihood are the same bits alone and in any batch. 1024 where the filters fit their taps, the
+// orbits suit long tiles (unequal arms: utv_long_tiles) and two workgroups share a CU's LDS, 512
+// otherwise: equal arms, 32 sources of 131,072 samples 299 (1024), 371 (512) and 475 us (256), 4 of 32,768 32.4,
+// 33.9 and 28.2, 1 of 8,192 32.3, 28.8 and 21.5; unequal arms, as a run's: 8 of 524,288 577 (1024) and
+// 823 us (512).
+int inner_passes(const flr_response *r, double dt, double fs, int flags)
+{
+    if (!(flags & FLR_FLAG_MIXED) || r->order != 25 || r->stock_gen == 0) return 0;
+    const int nx = r->stock_gen == 1 ? 8 : 16;
+    const int chain = (int)std::ceil(r->max_chain * r->orbits->max_ltt * fs);
+    const bool equal = r->orbits->equal_arm;
+    ProjConfig pc;
+    TdiConfig tc;
+    StockTdi stock;
+    return chain + r->order + 3 <= kFir &&
+                   make_fused_config(r, dt, fs, flags, 4, pc, tc, stock) == FLR_OK &&
+                   2 * fused_lds_bytes(pc, tc, false, equal, 4, !equal) + 2 * kFusedStaticLds <= kMaxLds &&
+                   (equal ? r->orbits->constant_arm
+                          : utv_suitable(r->orbits, nx, tc.tile, dt, fs, r->deps) &&
+                                utv_long_tiles(r->orbits, nx, tc.tile, dt, fs, r->deps))
+               ? 4
+               : kFusedPasses;
+}
+
+// Window of a run of a fused batch nobody chose a shape for, in units of kBlock samples: 1, 2 or 4 for the
 // mixed matrix-core forms, kFusedPasses otherwise. src: the sources; uniform: every one clears the
 // composite-filter test as a whole.
 //
@@ -562,29 +593,19 @@ int make_fused_config(const flr_response *r, double dt, double fs, int flags, in
 // (1024) against 243 us; 64 sources, 1.06e8 samples: 6.53 against 7.20 ms. The results do not depend
 // on the choice.
 // Unequal arms: the per-tile filters make a tile's fixed cost larger, and their results depend on
-// the tile's length (within the float32 rounding), so the choice must not depend on a batch's size:
-// 1024 wherever the filters fit their taps, the orbits suit long tiles (utv_long_tiles) and two
-// workgroups share a CU's LDS. 8 sources, 4.3e6 samples: 578 against 876 us; 131,072: 48.7 against
-// 63.8; below 65,536 samples the two are equal within 4%.
+// the tile's length (within the float32 rounding), so the choice must not depend on a batch's size: that
+// of inner_passes. 8 sources, 4.3e6 samples: 535 us (1024) against 765 (512); 131,072: 48.7 against
+// 58.5; below 65,536 samples the two are equal within 6%.
 int auto_passes(const flr_response *r, double dt, double fs, int flags, const FusedSource *src,
                 int num_sources, bool uniform)
 {
-    if (!(flags & FLR_FLAG_MIXED) || r->order != 25 || r->stock_gen == 0) return kFusedPasses;
+    const int fixed = inner_passes(r, dt, fs, flags);
+    if (fixed == 0) return kFusedPasses;
+    if (!r->orbits->equal_arm) return fixed;
     const int zero_edges = (flags & FLR_FLAG_ZERO_EDGES) ? 1 : 0;
-    const int nx = r->stock_gen == 1 ? 8 : 16;
     ProjConfig pc;
     TdiConfig tc;
     StockTdi stock;
-    if (!r->orbits->equal_arm) {
-        const int chain = (int)std::ceil(r->max_chain * r->orbits->max_ltt * fs);
-        return chain + r->order + 3 <= kFir &&
-                       make_fused_config(r, dt, fs, flags, 4, pc, tc, stock) == FLR_OK &&
-                       2 * fused_lds_bytes(pc, tc, false, false, 4, true) + 2 * kFusedStaticLds <= kMaxLds &&
-                       utv_suitable(r->orbits, nx, tc.tile, dt, fs, r->deps) &&
-                       utv_long_tiles(r->orbits, nx, tc.tile, dt, fs, r->deps)
-                   ? 4
-                   : kFusedPasses;
-    }
     if (!uniform) return kFusedPasses;
     const double cost[3] = {4.4, 8.75, 16.3};
     const int cus = compute_units();
@@ -1011,11 +1032,11 @@ void flr_batch_destroy(flr_batch *b)
         (void)hipEventDestroy(b->ran);
     }
     if (b->d_fused) (void)hipFree(b->d_fused);
-    if (b->d_fused_tiles) (void)hipFree(b->d_fused_tiles);
+    if (b->tiles.d) (void)hipFree(b->tiles.d);  // (inner.d lies behind it)
     if (b->d_lti) (void)hipFree(b->d_lti);
     if (b->d_inner) (void)hipFree(b->d_inner);
     if (b->h_fused) (void)hipHostFree(b->h_fused);
-    if (b->h_fused_tiles) (void)hipHostFree(b->h_fused_tiles);
+    if (b->tiles.h) (void)hipHostFree(b->tiles.h);
     delete b;
 }
 
@@ -1127,11 +1148,12 @@ int flr_fused_reserve(flr_response *r, int capacity, double dt, double sampling_
     b->fs = sampling_frequency;
     b->fused = true;
     b->capacity = capacity;
-    b->tile_len = tc.tile;
+    b->tiles.len = tc.tile;
+    const size_t prefixes = sizeof(int) * 2 * ((size_t)capacity + 1);
     hipError_t e = hipMalloc(&b->d_fused, sizeof(FusedSource) * capacity);
-    if (e == hipSuccess) e = hipMalloc(&b->d_fused_tiles, sizeof(int) * (capacity + 1));
+    if (e == hipSuccess) e = hipMalloc(&b->tiles.d, prefixes);
     if (e == hipSuccess) e = hipHostMalloc((void **)&b->h_fused, sizeof(FusedSource) * capacity);
-    if (e == hipSuccess) e = hipHostMalloc((void **)&b->h_fused_tiles, sizeof(int) * (capacity + 1));
+    if (e == hipSuccess) e = hipHostMalloc((void **)&b->tiles.h, prefixes);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->uploaded, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&b->ran, hipEventDisableTiming);
     if (e == hipSuccess && (flags & FLR_FLAG_MIXED))
@@ -1140,6 +1162,8 @@ int flr_fused_reserve(flr_response *r, int capacity, double dt, double sampling_
         flr_batch_destroy(b);
         return hip_fail(e, "fused batch reserve");
     }
+    b->inner.d = b->tiles.d + capacity + 1;
+    b->inner.h = b->tiles.h + capacity + 1;
     *out = b;
     return FLR_OK;
 }
@@ -1194,9 +1218,9 @@ int fused_tile_prefix(const FusedSource *src, int num_sources, int zero_edges, i
 // set too (a TDI table with longer delay chains has wider halos and so shorter tiles). When the
 // configuration's tile differs from the one the bound sources were tiled for, re-tile them from
 // the pinned staging copy and upload the prefix on `stream` (after any run still reading it).
-int fused_retile(flr_batch *b, int tile_len, hipStream_t stream)
+int fused_retile(flr_batch *b, FusedTiling &t, int tile_len, hipStream_t stream)
 {
-    if (tile_len == b->tile_len) return FLR_OK;
+    if (tile_len == t.len) return FLR_OK;
     bool cap = false;
     int cst = stream_capturing(stream, cap);
     if (cst) return cst;
@@ -1206,16 +1230,15 @@ int fused_retile(flr_batch *b, int tile_len, hipStream_t stream)
     if (b->num_sources > 0) {
         FLR_HIP(hipEventSynchronize(b->uploaded));  // the staging copy is no longer being read
         const int zero_edges = (b->flags & FLR_FLAG_ZERO_EDGES) ? 1 : 0;
-        int st = fused_tile_prefix(b->h_fused, b->num_sources, zero_edges, tile_len,
-                                   b->h_fused_tiles);
+        int st = fused_tile_prefix(b->h_fused, b->num_sources, zero_edges, tile_len, t.h);
         if (st) return st;
         if (b->ran_recorded) FLR_HIP(hipStreamWaitEvent(stream, b->ran, 0));
-        FLR_HIP(hipMemcpyAsync(b->d_fused_tiles, b->h_fused_tiles,
-                               sizeof(int) * (b->num_sources + 1), hipMemcpyHostToDevice, stream));
+        FLR_HIP(hipMemcpyAsync(t.d, t.h, sizeof(int) * (b->num_sources + 1), hipMemcpyHostToDevice,
+                               stream));
         FLR_HIP(hipEventRecord(b->uploaded, stream));
-        b->fused_tiles = b->h_fused_tiles[b->num_sources];
+        t.total = t.h[b->num_sources];
     }
-    b->tile_len = tile_len;
+    t.len = tile_len;
     return FLR_OK;
 }
 
@@ -1231,10 +1254,10 @@ int lti_refresh(flr_batch *b, hipStream_t stream)
     ProjConfig pc;
     TdiConfig tc;
     StockTdi stock;
-    int st = make_fused_config(r, b->dt, b->fs, b->flags, b->tile_passes, pc, tc, stock);
+    int st = make_fused_config(r, b->dt, b->fs, b->flags, b->tiles.passes, pc, tc, stock);
     if (st) return st;
     tc.lti_fir = b->d_lti;
-    Batch<FusedSource> bf{b->d_fused, b->d_fused_tiles, b->num_sources, b->fused_tiles};
+    Batch<FusedSource> bf{b->d_fused, b->tiles.d, b->num_sources, b->tiles.total};
     hipError_t e = launch_lti_filters(tc, bf, r->orbits->view(), r->lagrange(), stock, stream);
     if (e != hipSuccess) return hip_fail(e, "composite filter launch");
     b->lti_version = r->version;
@@ -1255,7 +1278,7 @@ int flr_fused_bind(flr_batch *b, const flr_source *sources, int num_sources, con
     const int flags = b->flags;
     const int zero_edges = (flags & FLR_FLAG_ZERO_EDGES) ? 1 : 0;
     std::vector<FusedSource> fs(num_sources);
-    std::vector<int> ft(num_sources + 1, 0);
+    std::vector<int> ft(num_sources + 1, 0), fi;
     int64_t samples = 0;
     int cst;
     for (int s = 0; s < num_sources; ++s) {
@@ -1273,19 +1296,31 @@ int flr_fused_bind(flr_batch *b, const flr_source *sources, int num_sources, con
         choose = b->h_fused[s].num_pts != fs[s].num_pts ||
                  b->h_fused[s].tdi_start != fs[s].tdi_start;
     const int passes = choose ? auto_passes(b->r, b->dt, b->fs, flags, fs.data(), num_sources, uniform)
-                              : b->tile_passes;
+                              : b->tiles.passes;
     ProjConfig pc;
     TdiConfig tc;
     StockTdi stock;
     if ((cst = make_fused_config(b->r, b->dt, b->fs, flags, passes, pc, tc, stock))) return cst;
     if ((cst = fused_tile_prefix(fs.data(), num_sources, zero_edges, tc.tile, ft.data()))) return cst;
+    const int tile_len = tc.tile;
+    // the inner products' tiles, where the batch has them (at the launch if they cannot be made now)
+    const int inner_window = inner_passes(b->r, b->dt, b->fs, flags);
+    int inner_len = 0;
+    if (inner_window != 0 &&
+        make_fused_config(b->r, b->dt, b->fs, flags, inner_window, pc, tc, stock) == FLR_OK) {
+        fi.resize(num_sources + 1);
+        if (fused_tile_prefix(fs.data(), num_sources, zero_edges, tc.tile, fi.data()) == FLR_OK)
+            inner_len = tc.tile;
+    }
     hipStream_t st = (hipStream_t)stream;
     FLR_HIP(hipEventSynchronize(b->uploaded));  // the staging buffers are free again
     // a run still in flight (possibly on another stream) reads the tables about to be replaced
     if (b->ran_recorded) FLR_HIP(hipStreamWaitEvent(st, b->ran, 0));
-    b->tile_passes = passes;
+    b->tiles.passes = passes;
+    b->tiles.len = tile_len;
+    b->inner.passes = inner_window != 0 ? inner_window : kFusedPasses;
+    b->inner.len = inner_len;
     b->shape_version = b->r->version;
-    b->tile_len = tc.tile;
     // A source's composite filters depend on its first time and first TDI sample (and on the
     // response's tables, tracked by lti_version), not on its sky position or input: when these
     // match the previous bind's (still in the staging copy), the filters built then -- already
@@ -1294,22 +1329,24 @@ int flr_fused_bind(flr_batch *b, const flr_source *sources, int num_sources, con
     for (int s = 0; same_refs && s < num_sources; ++s)
         same_refs = b->h_fused[s].t0 == fs[s].t0 && b->h_fused[s].tdi_start == fs[s].tdi_start;
     std::memcpy(b->h_fused, fs.data(), sizeof(FusedSource) * num_sources);
-    std::memcpy(b->h_fused_tiles, ft.data(), sizeof(int) * (num_sources + 1));
+    std::memcpy(b->tiles.h, ft.data(), sizeof(int) * (num_sources + 1));
+    if (inner_len != 0) std::memcpy(b->inner.h, fi.data(), sizeof(int) * (num_sources + 1));
     FLR_HIP(hipMemcpyAsync(b->d_fused, b->h_fused, sizeof(FusedSource) * num_sources,
                            hipMemcpyHostToDevice, st));
-    FLR_HIP(hipMemcpyAsync(b->d_fused_tiles, b->h_fused_tiles, sizeof(int) * (num_sources + 1),
-                           hipMemcpyHostToDevice, st));
+    // both prefixes in one copy: the second lies behind the first's capacity
+    const size_t prefix = (inner_len != 0 ? (size_t)b->capacity + 1 : 0) + num_sources + 1;
+    FLR_HIP(hipMemcpyAsync(b->tiles.d, b->tiles.h, sizeof(int) * prefix, hipMemcpyHostToDevice, st));
     b->num_sources = num_sources;
     b->samples = samples;
     b->fused_min_start = fs[0].tdi_start;
     for (int s = 1; s < num_sources; ++s)
         b->fused_min_start = std::min(b->fused_min_start, fs[s].tdi_start);
-    b->fused_tiles = ft[num_sources];
+    b->tiles.total = ft[num_sources];
+    b->inner.total = inner_len != 0 ? fi[num_sources] : 0;
     b->out_base = out_all;
     if (!same_refs) b->lti_version = ~0ull;  // new sources: their filters are built now
     b->lti_uniform = uniform;                 // the tile-test proof for these sources
     b->uniform_version = b->r->version;
-    b->uniform_tile = tc.tile;
     const int fst = lti_refresh(b, st);
     // recorded after the filters too: flr_fused_create waits on it before returning
     FLR_HIP(hipEventRecord(b->uploaded, st));
@@ -1352,14 +1389,17 @@ int fused_launch(flr_batch *b, hipStream_t s, const void *data, double *sums)
     StockTdi stock;
     int st;
     if (b->num_sources < 1) return fail(FLR_ERR_INVALID_ARGUMENT, "no sources bound to the batch");
-    if (b->auto_shape && b->shape_version != r->version) {  // the tables changed since the bind
-        b->tile_passes = auto_passes(r, b->dt, b->fs, b->flags, b->h_fused, b->num_sources,
-                                     sources_uniform(r, b->dt, b->fs, b->flags, b->h_fused,
-                                                     b->num_sources));
+    if (b->shape_version != r->version) {  // the tables changed since the bind
+        if (b->auto_shape)
+            b->tiles.passes = auto_passes(r, b->dt, b->fs, b->flags, b->h_fused, b->num_sources,
+                                          sources_uniform(r, b->dt, b->fs, b->flags, b->h_fused,
+                                                          b->num_sources));
+        const int inner_window = inner_passes(r, b->dt, b->fs, b->flags);
+        b->inner.passes = inner_window != 0 ? inner_window : kFusedPasses;
         b->shape_version = r->version;
     }
-    if ((st = make_fused_config(r, b->dt, b->fs, b->flags, b->tile_passes, pc, tc, stock)))
-        return st;
+    FusedTiling &tiles = data ? b->inner : b->tiles;
+    if ((st = make_fused_config(r, b->dt, b->fs, b->flags, tiles.passes, pc, tc, stock))) return st;
     bool cap = false;
     if ((st = stream_capturing(s, cap))) return st;
     if (data) {
@@ -1367,8 +1407,8 @@ int fused_launch(flr_batch *b, hipStream_t s, const void *data, double *sums)
             return fail(FLR_ERR_UNSUPPORTED, "fused inner products run in the mixed-precision "
                                              "kernels with a stock TDI table at order 25");
     }
-    if ((st = fused_retile(b, tc.tile, s))) return st;
-    if (data && b->fused_tiles > b->inner_cap) {
+    if ((st = fused_retile(b, tiles, tc.tile, s))) return st;
+    if (data && tiles.total > b->inner_cap) {
         if (cap)
             return fail(FLR_ERR_UNSUPPORTED, "the inner-product buffer must grow: call "
                                              "flr_fused_inner once outside stream capture first");
@@ -1379,21 +1419,20 @@ int fused_launch(flr_batch *b, hipStream_t s, const void *data, double *sums)
             b->d_inner = nullptr;
             b->inner_cap = 0;
         }
-        FLR_HIP(hipMalloc(&b->d_inner, sizeof(double) * 3 * kInnerSums * (size_t)b->fused_tiles));
-        b->inner_cap = b->fused_tiles;
+        FLR_HIP(hipMalloc(&b->d_inner, sizeof(double) * 3 * kInnerSums * (size_t)tiles.total));
+        b->inner_cap = tiles.total;
     }
     if ((st = lti_refresh(b, s))) return st;
-    Batch<FusedSource> bf{b->d_fused, b->d_fused_tiles, b->num_sources, b->fused_tiles,
+    Batch<FusedSource> bf{b->d_fused, tiles.d, b->num_sources, tiles.total,
                           b->fused_min_start};
     tc.lti_fir = b->d_lti;
     if ((b->flags & FLR_FLAG_MIXED) && stock.generation != 0 && stock.equal_arm &&
         r->order == 25) {
-        if (b->uniform_version != r->version || b->uniform_tile != tc.tile) {
+        if (b->uniform_version != r->version) {
             // the staging copy holds the bound sources (its upload may still be in flight:
             // reading it on the host is fine)
             b->lti_uniform = sources_uniform(r, b->dt, b->fs, b->flags, b->h_fused, b->num_sources);
             b->uniform_version = r->version;
-            b->uniform_tile = tc.tile;
         }
         tc.lti_uniform = b->lti_uniform ? 1 : 0;
     }
@@ -1412,10 +1451,10 @@ int fused_launch(flr_batch *b, hipStream_t s, const void *data, double *sums)
                                       (b->flags & FLR_FLAG_MIXED) != 0,
                                       (b->flags & FLR_FLAG_Q31) ? kInQ31
                                       : (b->flags & FLR_FLAG_C128) ? kInC128 : kInC64,
-                                      b->tile_passes, b->grid_per_cu, stock, s);
+                                      tiles.passes, b->grid_per_cu, stock, s);
     if (e != hipSuccess) return hip_fail(e, "fused batch launch");
     if (data) {
-        e = launch_inner_reduce(b->d_inner, b->d_fused_tiles, b->num_sources, sums, s);
+        e = launch_inner_reduce(b->d_inner, tiles.d, b->num_sources, sums, s);
         if (e != hipSuccess) return hip_fail(e, "inner-product reduction launch");
     }
     // an event recorded inside a capture cannot be waited on outside it: replays of a
@@ -1469,7 +1508,7 @@ int flr_batch_set_launch(flr_batch *b, int tile_samples, int grid_per_cu)
     if (!b || !b->r) return fail(FLR_ERR_INVALID_ARGUMENT, "batch is NULL");
     if (grid_per_cu < 0 || grid_per_cu > 64)
         return fail(FLR_ERR_INVALID_ARGUMENT, "grid_per_cu must be in [1, 64] (0 keeps it)");
-    int passes = b->tile_passes;
+    int passes = b->tiles.passes;
     if (tile_samples != 0) {
         if (!b->fused) {
             if (tile_samples != kBlock)
@@ -1485,16 +1524,16 @@ int flr_batch_set_launch(flr_batch *b, int tile_samples, int grid_per_cu)
         }
     }
     DeviceGuard g(b->r->device);
-    if (b->fused && passes != b->tile_passes) {
+    if (b->fused && passes != b->tiles.passes) {
         ProjConfig pc;
         TdiConfig tc;
         StockTdi stock;
         int st = make_fused_config(b->r, b->dt, b->fs, b->flags, passes, pc, tc, stock);
         if (st) return st;
         // re-tile the bound sources (host copy in the staging buffer), then wait for the upload
-        if ((st = fused_retile(b, tc.tile, nullptr))) return st;
+        if ((st = fused_retile(b, b->tiles, tc.tile, nullptr))) return st;
         FLR_HIP(hipEventSynchronize(b->uploaded));
-        b->tile_passes = passes;
+        b->tiles.passes = passes;
     }
     if (tile_samples != 0) b->auto_shape = false;
     if (grid_per_cu != 0) b->grid_per_cu = grid_per_cu;
@@ -1504,7 +1543,7 @@ int flr_batch_set_launch(flr_batch *b, int tile_samples, int grid_per_cu)
 int flr_batch_launch(const flr_batch *b, int *tile_samples, int *grid_per_cu)
 {
     if (!b) return fail(FLR_ERR_INVALID_ARGUMENT, "batch is NULL");
-    if (tile_samples) *tile_samples = b->fused ? b->tile_passes * kBlock : kBlock;
+    if (tile_samples) *tile_samples = b->fused ? b->tiles.passes * kBlock : kBlock;
     if (grid_per_cu) *grid_per_cu = b->grid_per_cu;
     return FLR_OK;
 }
