@@ -325,10 +325,16 @@ int compute_units()
     return cus;
 }
 
+// Persistent grid of total_tiles: as many workgroups as take one tile count each (but the last), at most
+// grid_per_cu per CU. With some of them taking one tile more than the rest, spread evenly among them, a
+// launch of 1.43 tiles a workgroup took 30% longer than its share: 16 sources of 700,000 samples, 11,747
+// tiles of the 1024-sample window, 975 us with 8,192 workgroups, 765 with 5,874.
 int batch_grid(int total_tiles, int grid_per_cu)
 {
     const int grid = compute_units() * (grid_per_cu > 0 ? grid_per_cu : 16);
-    return total_tiles < grid ? total_tiles : grid;
+    if (total_tiles <= grid) return total_tiles;
+    const int each = (total_tiles + grid - 1) / grid;
+    return (total_tiles + each - 1) / each;
 }
 
 static size_t proj_lds(const ProjConfig &cfg) { return (size_t)cfg.win_cap * sizeof(double2); }
