@@ -555,6 +555,18 @@ int make_fused_config(const flr_response *r, double dt, double fs, int flags, in
     return FLR_OK;
 }
 
+// Whether the composite filters of constant equal arms fit their taps and the mixed kernels' halos,
+// whatever the start time and the sources: the positions of the chains' delays relative to the sample.
+bool lti_filters_fit(const flr_orbits *o, double fs, int nx, const TdiConfig &tc)
+{
+    constexpr int H = 13;
+    const int M = nx == 8 ? 3 : 7;  // longest chain
+    const int lo = (int)std::ceil(-M * o->ltt0 * fs) - 1, hi = -1;
+    const int kmin = lo - (H - 1);
+    return o->constant_arm && hi + H - kmin + 1 <= kFir && kmin + tc.halo_lo >= 0 &&
+           kmin + kFir <= tc.halo_hi + 1;
+}
+
 // The inner products' window in units of kBlock samples, 0 where a batch has none. A source's sums are
 // grouped by tile, so the window follows the response and the sampling alone: a walker's sums and
 // likelihood are the same bits alone and in any batch. 1024 where the filters fit their taps, the
@@ -571,19 +583,19 @@ int inner_passes(const flr_response *r, double dt, double fs, int flags)
     ProjConfig pc;
     TdiConfig tc;
     StockTdi stock;
-    return chain + r->order + 3 <= kFir &&
-                   make_fused_config(r, dt, fs, flags, 4, pc, tc, stock) == FLR_OK &&
+    return make_fused_config(r, dt, fs, flags, 4, pc, tc, stock) == FLR_OK &&
                    2 * fused_lds_bytes(pc, tc, false, equal, 4, !equal) + 2 * kFusedStaticLds <= kMaxLds &&
-                   (equal ? r->orbits->constant_arm
-                          : utv_suitable(r->orbits, nx, tc.tile, dt, fs, r->deps) &&
+                   (equal ? lti_filters_fit(r->orbits, fs, nx, tc)
+                          : chain + r->order + 3 <= kFir &&
+                                utv_suitable(r->orbits, nx, tc.tile, dt, fs, r->deps) &&
                                 utv_long_tiles(r->orbits, nx, tc.tile, dt, fs, r->deps))
                ? 4
                : kFusedPasses;
 }
 
 // Window of a run of a fused batch nobody chose a shape for, in units of kBlock samples: 1, 2 or 4 for the
-// mixed matrix-core forms, kFusedPasses otherwise. src: the sources; uniform: every one clears the
-// composite-filter test as a whole.
+// mixed matrix-core forms, kFusedPasses otherwise. src: the sources, of which only the lengths and start
+// indexes count: a bound plan keeps its window while its start times change.
 //
 // Equal arms: a launch takes about 8 us plus, per tile that the busiest CU works through, 4.4, 8.75
 // or 16.3 us for the 256-, 512- and 1024-sample windows (MI355X; within 5% from 8,192 to 3,153,600
@@ -591,13 +603,17 @@ int inner_passes(const flr_response *r, double dt, double fs, int flags)
 // taken: long tiles recompute less halo and share one barrier among more work, short ones spread a
 // small launch over the CUs. 131,072 samples: 21.7 (256) against 26.7 us (512); 1-yr source: 219
 // (1024) against 243 us; 64 sources, 1.06e8 samples: 6.53 against 7.20 ms. The results do not depend
-// on the choice.
+// on the choice. At start times where the tiles cannot be cleared as a whole (from about 2e7 s on) every
+// window takes 9 to 14% longer, so the choice is the same: from 3.5e7 to 2.8e8 s 8,192 samples 16.3 us (256), 24.2
+// (512) and 28.2 (1024), 32 sources of 131,072 samples 476, 375 and 302, a 1-yr source 306, 264 and 234.
+// Filters that do not fit (fine sampling, arms that change) leave every tile to the per-sample stencils:
+// 512.
 // Unequal arms: the per-tile filters make a tile's fixed cost larger, and their results depend on
 // the tile's length (within the float32 rounding), so the choice must not depend on a batch's size: that
 // of inner_passes. 8 sources, 4.3e6 samples: 535 us (1024) against 765 (512); 131,072: 48.7 against
 // 58.5; below 65,536 samples the two are equal within 6%.
 int auto_passes(const flr_response *r, double dt, double fs, int flags, const FusedSource *src,
-                int num_sources, bool uniform)
+                int num_sources)
 {
     const int fixed = inner_passes(r, dt, fs, flags);
     if (fixed == 0) return kFusedPasses;
@@ -606,7 +622,9 @@ int auto_passes(const flr_response *r, double dt, double fs, int flags, const Fu
     ProjConfig pc;
     TdiConfig tc;
     StockTdi stock;
-    if (!uniform) return kFusedPasses;
+    if (make_fused_config(r, dt, fs, flags, kFusedPasses, pc, tc, stock) != FLR_OK ||
+        !lti_filters_fit(r->orbits, fs, r->stock_gen == 1 ? 8 : 16, tc))
+        return kFusedPasses;
     const double cost[3] = {4.4, 8.75, 16.3};
     const int cus = compute_units();
     int best = kFusedPasses;
@@ -1295,7 +1313,7 @@ int flr_fused_bind(flr_batch *b, const flr_source *sources, int num_sources, con
     for (int s = 0; b->auto_shape && !choose && s < num_sources; ++s)
         choose = b->h_fused[s].num_pts != fs[s].num_pts ||
                  b->h_fused[s].tdi_start != fs[s].tdi_start;
-    const int passes = choose ? auto_passes(b->r, b->dt, b->fs, flags, fs.data(), num_sources, uniform)
+    const int passes = choose ? auto_passes(b->r, b->dt, b->fs, flags, fs.data(), num_sources)
                               : b->tiles.passes;
     ProjConfig pc;
     TdiConfig tc;
@@ -1391,9 +1409,7 @@ int fused_launch(flr_batch *b, hipStream_t s, const void *data, double *sums)
     if (b->num_sources < 1) return fail(FLR_ERR_INVALID_ARGUMENT, "no sources bound to the batch");
     if (b->shape_version != r->version) {  // the tables changed since the bind
         if (b->auto_shape)
-            b->tiles.passes = auto_passes(r, b->dt, b->fs, b->flags, b->h_fused, b->num_sources,
-                                          sources_uniform(r, b->dt, b->fs, b->flags, b->h_fused,
-                                                          b->num_sources));
+            b->tiles.passes = auto_passes(r, b->dt, b->fs, b->flags, b->h_fused, b->num_sources);
         const int inner_window = inner_passes(r, b->dt, b->fs, b->flags);
         b->inner.passes = inner_window != 0 ? inner_window : kFusedPasses;
         b->shape_version = r->version;
@@ -1745,7 +1761,7 @@ int flr_fused_run_static(flr_response *r, const flr_source *sources, int num_sou
         if ((st = fused_source_record(sources[q], q, flags, h_all, out_all, recs[q]))) return st;
     const bool uniform = sources_uniform(r, dt, sampling_frequency, flags, recs.data(), num_sources);
     if (tile_samples == 0)
-        passes = auto_passes(r, dt, sampling_frequency, flags, recs.data(), num_sources, uniform);
+        passes = auto_passes(r, dt, sampling_frequency, flags, recs.data(), num_sources);
     ProjConfig pc;
     TdiConfig tc;
     StockTdi stock;

@@ -121,3 +121,28 @@ def test_a_replay_without_its_proof_reports(torch_gpu, orbits):
     plan.run()
     plan.check_errors()
     assert not bool(plan.out_all.isnan().any())
+
+
+@pytest.mark.parametrize("lengths", [[9_001], [90_001, 5_003, 40_011], [700_001, 20_000]])
+def test_window_of_any_start_time(torch_gpu, orbits, lengths):
+    """The rule counts tiles: plans of the same sources take the same window at any start time, and their
+    outputs are those of every explicit window."""
+    from fastlisaresponse_amd.autotune import apply
+    from fastlisaresponse_amd.batch import BatchedResponse
+    torch = torch_gpu
+    br = BatchedResponse(0.1, tdi="2nd generation", orbits=orbits, precision="mixed-c128")
+    m = len(lengths)
+    h = torch.as_tensor(np.concatenate([gb_waveform(n, 10.0, f=4e-3) for n in lengths]), device="cuda")
+    shapes = set()
+    for t0 in (EARLY, LATE, 2.8e8):
+        plan = br.plan(h, lengths, [0.3] * m, [0.2] * m, [t0] * m)
+        shapes.add(_shape(plan))
+        plan.run()
+        plan.check_errors()
+        got = plan.out_all.clone()
+        for window in (256, 512, 1024):
+            apply(plan, window, 32)
+            plan.run()
+            plan.check_errors()
+            assert torch.equal(plan.out_all, got), (t0, window)
+    assert len(shapes) == 1
