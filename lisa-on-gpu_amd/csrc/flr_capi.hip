@@ -597,17 +597,20 @@ int inner_passes(const flr_response *r, double dt, double fs, int flags)
 // mixed matrix-core forms, kFusedPasses otherwise. src: the sources, of which only the lengths and start
 // indexes count: a bound plan keeps its window while its start times change.
 //
-// Equal arms: a launch takes about 8 us plus, per tile that the busiest CU works through, 4.4, 8.75
-// or 16.3 us for the 256-, 512- and 1024-sample windows (MI355X; within 5% from 8,192 to 3,153,600
-// samples, both generations, dt 5 and 10 s). So the window with the least rounds times cost is
-// taken: long tiles recompute less halo and share one barrier among more work, short ones spread a
-// small launch over the CUs. 131,072 samples: 21.7 (256) against 26.7 us (512); 1-yr source: 219
-// (1024) against 243 us; 64 sources, 1.06e8 samples: 6.53 against 7.20 ms. The results do not depend
-// on the choice. At start times where the tiles cannot be cleared as a whole (from about 2e7 s on) every
-// window takes 9 to 14% longer, so the choice is the same: from 3.5e7 to 2.8e8 s 8,192 samples 16.3 us (256), 24.2
-// (512) and 28.2 (1024), 32 sources of 131,072 samples 476, 375 and 302, a 1-yr source 306, 264 and 234.
-// Filters that do not fit (fine sampling, arms that change) leave every tile to the per-sample stencils:
-// 512.
+// Equal arms: a launch takes about 8 us plus 4.4, 8.75 or 16.3 us (256-, 512- and 1024-sample windows)
+// times the tiles a CU has to work through, one at least; tiles in the zeroed edges count nothing (MI355X;
+// within 10%: which CU gets the last tiles is not in it). Long tiles recompute less halo and share one
+// barrier among more work, short ones spread a small launch over the CUs; 512 is left where that
+// promises a tenth or more. Over 220 batches of 1 to 48 sources (dt 5 to 15 s, both generations, early and
+// late start times) the choice is at worst 1.2% slower than 512 (with whole rounds over the CUs, the edges
+// counted and no margin 14.7%: 48 sources of 8,552 samples 39.2 against 34.7 us) and on average 4.5%
+// slower than the fastest window; 512 throughout is 14% slower. 131,072 samples: 21.7 (256) against 26.7
+// us (512); 1-yr source: 219 (1024) against 243; 64 sources, 1.06e8 samples: 6.53 against 7.20 ms. The
+// results do not depend on the choice. At start times where the tiles cannot be cleared as a whole (from
+// about 2e7 s on) every window takes 9 to 14% longer, so the choice is the same: from 3.5e7 to 2.8e8 s
+// 8,192 samples 16.3 us (256), 24.2 (512) and 28.2 (1024), 32 sources of 131,072 samples 476, 375 and 302, a
+// 1-yr source 306, 264 and 234. Filters that do not fit (fine sampling, arms that change) leave every
+// tile to the per-sample stencils: 512.
 // Unequal arms: the per-tile filters make a tile's fixed cost larger, and their results depend on
 // the tile's length (within the float32 rounding), so the choice must not depend on a batch's size: that
 // of inner_passes. 8 sources, 4.3e6 samples: 535 us (1024) against 765 (512); 131,072: 48.7 against
@@ -618,7 +621,6 @@ int auto_passes(const flr_response *r, double dt, double fs, int flags, const Fu
     const int fixed = inner_passes(r, dt, fs, flags);
     if (fixed == 0) return kFusedPasses;
     if (!r->orbits->equal_arm) return fixed;
-    const int zero_edges = (flags & FLR_FLAG_ZERO_EDGES) ? 1 : 0;
     ProjConfig pc;
     TdiConfig tc;
     StockTdi stock;
@@ -626,18 +628,20 @@ int auto_passes(const flr_response *r, double dt, double fs, int flags, const Fu
         !lti_filters_fit(r->orbits, fs, r->stock_gen == 1 ? 8 : 16, tc))
         return kFusedPasses;
     const double cost[3] = {4.4, 8.75, 16.3};
-    const int cus = compute_units();
+    const double cus = compute_units();
     int best = kFusedPasses;
     double least = 0.0;
-    for (int k = 2; k >= 0; --k) {  // the longer window where two cost the same
+    for (int k : {1, 2, 0}) {  // 512 first
         const int passes = 1 << k;
         if (make_fused_config(r, dt, fs, flags, passes, pc, tc, stock) != FLR_OK) continue;
         if (k == 2 && 2 * fused_lds_bytes(pc, tc, false, true, 4) + 2 * kFusedStaticLds > kMaxLds) continue;
         int64_t tiles = 0;
         for (int s = 0; s < num_sources; ++s)
-            tiles += tiles_for(src[s].num_pts, src[s].tdi_start, zero_edges, tc.tile);
-        const double c = cost[k] * (double)((tiles + cus - 1) / cus);
-        if (least == 0.0 || c < least) {
+            tiles += std::max(0, tiles_for(src[s].num_pts, src[s].tdi_start, 0, tc.tile));
+        const double c = 8.0 + cost[k] * std::max(1.0, (double)tiles / cus);
+        if (k == 1)
+            least = 0.9 * c;
+        else if (c <= least) {
             least = c;
             best = passes;
         }

@@ -146,3 +146,16 @@ def test_window_of_any_start_time(torch_gpu, orbits, lengths):
             plan.check_errors()
             assert torch.equal(plan.out_all, got), (t0, window)
     assert len(shapes) == 1
+
+
+@pytest.mark.parametrize("lengths,dt,window", [([8_552] * 48, 7.0, 512), ([74_783] * 8, 10.0, 512),
+                                               ([131_072] * 32, 10.0, 1024), ([9_001], 10.0, 256)])
+def test_window_by_the_computed_tiles(torch_gpu, orbits, lengths, dt, window):
+    """Tiles in the zeroed edges count nothing, and 512 samples are left only for a tenth or more."""
+    from fastlisaresponse_amd.batch import BatchedResponse
+    torch = torch_gpu
+    br = BatchedResponse(1 / dt, tdi="2nd generation", orbits=orbits, precision="mixed-c128")
+    m = len(lengths)
+    h = torch.zeros(sum(lengths), dtype=torch.complex128, device="cuda")
+    plan = br.plan(h, lengths, [0.3] * m, [0.2] * m)
+    assert _shape(plan)[0] == window
