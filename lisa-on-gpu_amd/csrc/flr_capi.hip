@@ -598,15 +598,16 @@ int inner_passes(const flr_response *r, double dt, double fs, int flags)
 // indexes count: a bound plan keeps its window while its start times change.
 //
 // Equal arms: a launch takes about 8 us plus 4.4, 8.75 or 16.3 us (256-, 512- and 1024-sample windows)
-// times the tiles a CU has to work through, one at least; tiles in the zeroed edges count nothing (MI355X;
-// within 10%: which CU gets the last tiles is not in it). Long tiles recompute less halo and share one
-// barrier among more work, short ones spread a small launch over the CUs; 512 is left where that
-// promises a tenth or more. Over 220 batches of 1 to 48 sources (dt 5 to 15 s, both generations, early and
-// late start times) the choice is at worst 1.2% slower than 512 (with whole rounds over the CUs, the edges
-// counted and no margin 14.7%: 48 sources of 8,552 samples 39.2 against 34.7 us) and on average 4.5%
-// slower than the fastest window; 512 throughout is 14% slower. 131,072 samples: 21.7 (256) against 26.7
-// us (512); 1-yr source: 219 (1024) against 243; 64 sources, 1.06e8 samples: 6.53 against 7.20 ms. The
-// results do not depend on the choice. At start times where the tiles cannot be cleared as a whole (from
+// times the tiles a CU has to work through, one at least and whole ones of 1024; tiles in the zeroed edges
+// count nothing (MI355X; within 10%: which CU gets the last tiles is not in it). Long tiles recompute less
+// halo and share one barrier among more work, short ones spread a small launch over the CUs; 512 is
+// left where that promises 8% or more. Over 620 batches of 1 to 48 sources (dt 5 to 15 s, both
+// generations, early and late start times) the choice is never slower than 512 (with whole rounds for
+// every window, the edges counted and no margin 13 are, by up to 14.7%: 48 sources of 8,552 samples 39.2
+// against 34.7 us) and on average 5% slower than the fastest window; 512 throughout is 15% slower.
+// 131,072 samples: 21.7 (256) against 26.7 us (512); 1-yr source: 219 (1024) against 243; 64 sources,
+// 1.06e8 samples: 6.53 against 7.20 ms. The results do not depend on the choice. At start times where the
+// tiles cannot be cleared as a whole (from
 // about 2e7 s on) every window takes 9 to 14% longer, so the choice is the same: from 3.5e7 to 2.8e8 s
 // 8,192 samples 16.3 us (256), 24.2 (512) and 28.2 (1024), 32 sources of 131,072 samples 476, 375 and 302, a
 // 1-yr source 306, 264 and 234. Filters that do not fit (fine sampling, arms that change) leave every
@@ -638,9 +639,10 @@ int auto_passes(const flr_response *r, double dt, double fs, int flags, const Fu
         int64_t tiles = 0;
         for (int s = 0; s < num_sources; ++s)
             tiles += std::max(0, tiles_for(src[s].num_pts, src[s].tdi_start, 0, tc.tile));
-        const double c = 8.0 + cost[k] * std::max(1.0, (double)tiles / cus);
+        const double rounds = std::max(1.0, (double)tiles / cus);
+        const double c = 8.0 + cost[k] * (k == 2 ? std::ceil(rounds) : rounds);
         if (k == 1)
-            least = 0.9 * c;
+            least = 0.92 * c;
         else if (c <= least) {
             least = c;
             best = passes;
