@@ -269,15 +269,17 @@ def pack_q31(h: torch.Tensor, lengths: Sequence[int]):
     return out, scales
 
 
-def _host_values(x) -> np.ndarray:
-    """Per-source numbers (a list, array or tensor) as a host array."""
-    if isinstance(x, torch.Tensor):
-        return x.detach().cpu().numpy()
-    if isinstance(x, np.ndarray):
-        return x
-    if any(isinstance(v, torch.Tensor) for v in x):
-        return np.array([float(v) for v in x])
-    return np.asarray(x)
+def _plain_values(x) -> Optional[np.ndarray]:
+    """Per-source numbers that are float64 as they stand (a flat array, a CPU tensor without gradient or
+    a list of floats) as a host array; None for anything else, which is taken entry by entry."""
+    if type(x) is np.ndarray:
+        return x if x.dtype == np.float64 and x.ndim == 1 else None
+    if type(x) is torch.Tensor:
+        plain = x.dtype == torch.float64 and x.dim() == 1 and not x.is_cuda and not x.requires_grad
+        return x.numpy() if plain else None
+    if type(x) in (list, tuple) and all(type(v) in (float, np.float64) for v in x):
+        return np.array(x, dtype=np.float64)
+    return None
 
 
 class BatchedResponse:
@@ -406,16 +408,38 @@ class BatchPlan:
         if (len(lams) != n or len(betas) != n or (t0s is not None and len(t0s) != n)
                 or (scales is not None and len(scales) != n)):
             raise ValueError("lams, betas (and t0s, scales) must have one entry per source")
+        given = [x for x in (lams, betas, t0s, scales) if x is not None]
+        plain = [_plain_values(x) for x in given]
+        if any(x is None for x in plain):
+            return self._records_by_entry(lams, betas, t0s, scales)
+        lams, betas = plain[:2]
         rec = np.zeros(n, dtype=_SOURCE_DTYPE)
         rec["offset"], rec["num_pts"] = self.offsets, self.lengths
         rec["projections_start_ind"] = self.br.projections_start_ind
         rec["tdi_start_ind"] = self.br.tdi_start_ind
-        rec["t0"] = 0.0 if t0s is None else _host_values(t0s)
-        rec["scale"] = 1.0 if scales is None else _host_values(scales)
-        k, u, v = sky_basis(_host_values(lams), _host_values(betas))
+        rec["t0"] = 0.0 if t0s is None else plain[2]
+        rec["scale"] = 1.0 if scales is None else plain[-1]
+        k, u, v = sky_basis(lams, betas)
         for c in range(3):
             rec["k"][:, c], rec["u"][:, c], rec["v"][:, c] = k[c], u[c], v[c]
         return rec
+
+    def _records_by_entry(self, lams, betas, t0s, scales):
+        """_records of numbers of any kind that indexes and converts to a float."""
+        n = len(self.lengths)
+        srcs = (_capi.FlrSource * n)()
+        for s in range(n):
+            k, u, v = sky_basis(lams[s], betas[s])
+            q = srcs[s]
+            q.offset = int(self.offsets[s])
+            q.num_pts = int(self.lengths[s])
+            q.projections_start_ind = self.br.projections_start_ind
+            q.tdi_start_ind = self.br.tdi_start_ind
+            q.t0 = 0.0 if t0s is None else float(t0s[s])
+            q.scale = 1.0 if scales is None else float(scales[s])
+            for c in range(3):
+                q.k[c], q.u[c], q.v[c] = k[c], u[c], v[c]
+        return np.frombuffer(srcs, dtype=_SOURCE_DTYPE)
 
     def rebind(self, lams, betas, t0s=None, scales=None, h_all: Optional[torch.Tensor] = None,
                stream: Optional[int] = None) -> None:

@@ -131,6 +131,6 @@ def sky_basis(lam: float, beta: float):
     cb, sb = np.cos(beta), np.sin(beta)
     cl, sl = np.cos(lam), np.sin(lam)
     k = np.array([-cb * cl, -cb * sl, -sb])
-    u = np.array([sl, -cl, np.zeros_like(sl)])
+    u = np.array([sl, -cl, np.zeros_like(sl) if np.ndim(sl) else 0.0])
     v = np.array([-sb * cl, -sb * sl, cb])
     return k, u, v
