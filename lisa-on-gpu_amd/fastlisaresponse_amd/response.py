@@ -291,11 +291,12 @@ class pyResponseTDI:
 
     def _data_time_check(self, t0: float, n: int, input_in):
         t_last = t0 + (n - 1) * self.dt
-        if t_last > self.response_orbits.t[-1]:  # an increasing grid
+        t = self.response_orbits.t
+        if t_last > t[-1] and t_last > t.max():  # the last time first: the maximum takes a pass
             warnings.warn("Input waveform is longer than available orbital information. "
                           "Trimming to fit orbital information.")
             t_data = t0 + np.arange(n) * self.dt
-            max_ind = np.where(t_data <= self.response_orbits.t.max())[0][-1]
+            max_ind = np.where(t_data <= t.max())[0][-1]
             input_in = input_in[:max_ind]
         return input_in
 
