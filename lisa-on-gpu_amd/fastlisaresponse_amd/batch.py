@@ -139,8 +139,8 @@ def rms_frequencies(h: torch.Tensor, lengths: Sequence[int], dt: float) -> np.nd
     single complex sinusoid. One pass over the samples (flr_series_stats on the device, sums by
     index for host tensors), one host sync."""
     lengths = np.asarray([int(n) for n in lengths], dtype=np.int64)
-    if _on_device(h) and len(lengths) and lengths.min() > 0 and \
-            int(lengths.sum()) == h.numel() // (2 if h.dtype == torch.int32 else 1):
+    per = 2 if h.dtype == torch.int32 else 1
+    if _on_device(h) and len(lengths) and lengths.min() > 0 and per * int(lengths.sum()) == h.numel():
         st = _SeriesStats(h, lengths.tolist()).stats.cpu().numpy()
         return _rms(st[:, 2], st[:, 3], lengths, dt)
     if h.dtype == torch.int32:  # q31 pairs
@@ -159,13 +159,17 @@ def rms_frequencies(h: torch.Tensor, lengths: Sequence[int], dt: float) -> np.nd
     return _rms(p.cpu().numpy(), d.cpu().numpy(), lengths, dt)
 
 
+def _known_action(action: str) -> None:
+    if action not in ("warn", "raise", "off"):
+        raise ValueError("action must be 'warn', 'raise' or 'off'")
+
+
 def check_storage(h: torch.Tensor, lengths: Sequence[int], dt: float, precision: str,
                   armlength: float = 2.5e9, tol: float = STORAGE_TOL, action: str = "warn"):
     """Estimate each source's storage error (storage_error_estimate at its RMS frequency) and
     warn (StorageErrorWarning) or raise (ValueError, action="raise") when one exceeds tol;
     returns the estimates. action="off" or a format without storage error skips the pass."""
-    if action not in ("warn", "raise", "off"):
-        raise ValueError("action must be 'warn', 'raise' or 'off'")
+    _known_action(action)
     if action == "off" or STORAGE_K[precision] == 0.0:
         return np.zeros(len(lengths))
     return _storage_verdict(rms_frequencies(h, lengths, dt), precision, armlength, tol, action, 4)
@@ -192,10 +196,12 @@ def pack_checked(h: torch.Tensor, dt: float, precision: str, armlength: float, a
     """One source's complex128 series in the 8-byte format of `precision` ("mixed" or "mixed-q31")
     and its scale, after check_storage's verdict on it: one pass for the statistics, one for the
     conversion, one transfer to the host."""
+    _known_action(action)
     pack = pack_q31 if precision == "mixed-q31" else pack_mixed
     n = len(h)
     if not (_on_device(h) and h.dtype == torch.complex128 and n):
-        check_storage(h, [n], dt, precision, armlength, action=action)
+        if action != "off":
+            _storage_verdict(rms_frequencies(h, [n], dt), precision, armlength, STORAGE_TOL, action, 4)
         stored, scales = pack(h, [n])
         return stored, scales[0]
     series = _SeriesStats(h, [n])
