@@ -152,8 +152,9 @@ __global__ __launch_bounds__(kBlock) void series_pack_kernel(const double2 *__re
                 reinterpret_cast<int2 *>(out)[i] =
                     make_int2((int)rint(v.x * mul), (int)rint(v.y * mul));
             else
-                reinterpret_cast<float2 *>(out)[i] =
-                    make_float2((float)(v.x * mul), (float)(v.y * mul));
+                // the product by the complex number mul: a component that is not finite makes both NaN
+                reinterpret_cast<float2 *>(out)[i] = make_float2(
+                    (float)(v.x * mul - v.y * 0.0), (float)(v.y * mul + v.x * 0.0));
         }
     }
 }
