@@ -229,12 +229,13 @@ int flr_batch_run(flr_batch *batch, void *stream);
 int flr_fused_inner(flr_batch *batch, const void *data_all, double *sums, void *stream);
 /* Launch shape of a batch (no counterpart in the reference): tile_samples window samples per
  * workgroup tile (fused mixed: 256, 512 or 1024; fused FP64: 512; unfused: 256; 0 keeps the
- * current -- for a mixed batch at first the one its sources' sizes, or with unequal arms the orbits,
- * suggest; a fused tile outputs tile_samples minus the TDI delay halos, so that its projection
+ * current -- for a mixed batch the one its sources' sizes, or with unequal arms the orbits, suggest
+ * when they are first bound, kept while later binds have the same lengths; a fused tile outputs tile_samples minus the TDI delay halos, so that its projection
  * window is whole rounds of the workgroup) and grid_per_cu persistent workgroups per CU
- * (1..64; 0 keeps the current, default 32). Results do not depend on either. Call it when no
- * launch of the batch is in flight; the autotuner (fastlisaresponse_amd.autotune) times the
- * candidates and keeps the fastest. */
+ * (1..64; 0 keeps the current, default 32). Only the window of a mixed batch with unequal arms
+ * shows in results: its outputs at two windows differ within their float32 rounding (the null
+ * channel T by some 1e-7 of itself). Call it when no launch of the batch is in flight; the
+ * autotuner (fastlisaresponse_amd.autotune) times the candidates and keeps the fastest. */
 int flr_batch_set_launch(flr_batch *batch, int tile_samples, int grid_per_cu);
 /* The batch's launch shape (either pointer may be NULL). */
 int flr_batch_launch(const flr_batch *batch, int *tile_samples, int *grid_per_cu);

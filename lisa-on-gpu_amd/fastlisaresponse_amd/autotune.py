@@ -1,6 +1,10 @@
 """Launch-shape autotuner for batched and fused response launches.
 
-The kernels' results do not depend on the launch shape, only their speed does: the tile
+The launch shape is a matter of speed: the FP64 forms, the mixed forms with equal arms and every inner
+product give the same bits at any. With unequal arms the mixed forms' filters are made per tile, so A, E
+(and X, Y, Z) of two tile lengths differ within their float32 rounding and the null channel T by some
+1e-7 of itself; a
+plan that must reproduce another's bits keeps its shape instead of being tuned. The shape is the tile
 length (output samples per workgroup tile, i.e. samples per lane x 256) and the persistent grid
 density (workgroups per CU). `tune(plan)` times every candidate on the plan itself with HIP
 events, keeps the fastest on the plan and remembers it per workload key (precision, fused,
@@ -71,7 +75,6 @@ def apply(plan, tile_samples: int, grid_per_cu: int) -> None:
     """Set a plan's launch shape (no launch of the plan may be in flight)."""
     torch.cuda.synchronize()
     check(lib().flr_batch_set_launch(plan._h, int(tile_samples), int(grid_per_cu)))
-    plan.launch_shape = (int(tile_samples), int(grid_per_cu))
 
 
 def tune(plan, reps: int = 3, use_cache: bool = True) -> dict:

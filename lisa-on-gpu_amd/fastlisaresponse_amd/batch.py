@@ -404,9 +404,14 @@ class BatchPlan:
         self._h = h
         self.num_sources = n
         self.samples = int(lib().flr_batch_samples(h))
+
+    @property
+    def launch_shape(self):
+        """(tile window samples, workgroups per CU) of the plan's runs as the library has it now: it keeps
+        a chosen window through every rebind, and chooses anew if the response's tables change."""
         tile, grid = ctypes.c_int(), ctypes.c_int()
-        check(lib().flr_batch_launch(h, ctypes.byref(tile), ctypes.byref(grid)))
-        self.launch_shape = (tile.value, grid.value)  # (tile window samples, WGs per CU)
+        check(lib().flr_batch_launch(self._h, ctypes.byref(tile), ctypes.byref(grid)))
+        return tile.value, grid.value
 
     def _records(self, lams, betas, t0s=None, scales=None):
         """flr_source records of the plan's sources (packed offsets, the lengths of the plan)."""
@@ -454,8 +459,11 @@ class BatchPlan:
         outputs and the launch shape -- the MCMC pattern of many steps over fixed-length
         sources. Enqueued on `stream` (default: the current one) without allocating; the
         composite TDI filters are rebuilt only if a start time changed. A graph captured from
-        run() keeps replaying correctly after a rebind, since the kernel reads the rebound
-        tables at run time."""
+        run() or inner_products() keeps replaying correctly after a rebind, since the kernels read
+        the rebound tables at run time -- except that, with equal arms, a graph captured where
+        every tile cleared the composite filters' test (early start times) holds no per-sample
+        stencils: replayed with start times that need them it writes NaN, and check_errors
+        raises."""
         if not self.br.fused:
             raise ValueError("rebind needs a fused plan (fused=True or a mixed precision)")
         if h_all is not None:
@@ -482,7 +490,8 @@ class BatchPlan:
         (utility.inner_from_sums, overlap_from_sums and log_likelihood_from_sums turn them into
         inner products, get_overlap's overlap and a white-noise log-likelihood). Mixed plans
         with the stock TDI tables. Enqueued on `stream` (default: the current one); the first
-        call allocates the per-tile buffer, later ones nothing (graph-capturable after it)."""
+        call allocates the per-tile buffer, later ones nothing (graph-capturable after it). A
+        source's sums are the same bits in any batch and at any launch shape."""
         if self.br.precision == "fp64":
             raise ValueError("fused inner products run in the mixed-precision kernels "
                              "(precision='mixed-c128', 'mixed' or 'mixed-q31')")
