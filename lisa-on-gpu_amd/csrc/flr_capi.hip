@@ -597,14 +597,15 @@ int inner_passes(const flr_response *r, double dt, double fs, int flags)
 // mixed matrix-core forms, kFusedPasses otherwise. src: the sources, of which only the lengths and start
 // indexes count: a bound plan keeps its window while its start times change.
 //
-// Equal arms: a launch takes about 8 us plus 4.4, 8.75 or 16.3 us (256-, 512- and 1024-sample windows)
-// times the tiles a CU has to work through, one at least and whole ones of 1024; tiles in the zeroed edges
-// count nothing (MI355X; within 10%: which CU gets the last tiles is not in it). Long tiles recompute less
-// halo and share one barrier among more work, short ones spread a small launch over the CUs; 512 is
-// left where that promises 8% or more. Over 620 batches of 1 to 48 sources (dt 5 to 15 s, both
-// generations, early and late start times) the choice is never slower than 512 (with whole rounds for
-// every window, the edges counted and no margin 13 are, by up to 14.7%: 48 sources of 8,552 samples 39.2
-// against 34.7 us) and on average 5% slower than the fastest window; 512 throughout is 15% slower.
+// Equal arms: a launch takes about fixed + per_tile r microseconds (MI355X; 5 to 7% rms over 620 batches of 1
+// to 48 sources, dt 5 to 15 s, both generations, early and late start times), r being the tiles a CU has to
+// work through -- at least one, a share of what it lacks to a whole number added, the more the longer
+// the tile; tiles in the zeroed edges count half, or whole for the 1024-sample window. Long tiles
+// recompute less halo and share one barrier among more work, short ones spread a small launch over the CUs;
+// 512 is left where that promises 9% or more. Over those batches the choice is at worst 2% slower than 512
+// and on average 2.5% slower than the fastest window; 512 throughout is 15% slower, and with whole rounds for
+// every window, a fixed 8 us and no margin 13 are slower than 512 by 3 to 14.7% (48 sources of 8,552 samples
+// 39.2 against 34.7 us) and the average is 4%.
 // 131,072 samples: 21.7 (256) against 26.7 us (512); 1-yr source: 219 (1024) against 243; 64 sources,
 // 1.06e8 samples: 6.53 against 7.20 ms. The results do not depend on the choice. At start times where the
 // tiles cannot be cleared as a whole (from
@@ -628,21 +629,28 @@ int auto_passes(const flr_response *r, double dt, double fs, int flags, const Fu
     if (make_fused_config(r, dt, fs, flags, kFusedPasses, pc, tc, stock) != FLR_OK ||
         !lti_filters_fit(r->orbits, fs, r->stock_gen == 1 ? 8 : 16, tc))
         return kFusedPasses;
-    const double cost[3] = {4.4, 8.75, 16.3};
-    const double cus = compute_units();
+    struct Cost {
+        double fixed, per_tile, whole, edge;
+    };
+    const Cost cost[3] = {{11.0, 4.25, 0.0, 0.5}, {13.0, 8.1, 0.5, 0.5}, {10.0, 15.0, 0.75, 1.0}};
+    const int zero_edges = (flags & FLR_FLAG_ZERO_EDGES) ? 1 : 0;
     int best = kFusedPasses;
     double least = 0.0;
     for (int k : {1, 2, 0}) {  // 512 first
         const int passes = 1 << k;
         if (make_fused_config(r, dt, fs, flags, passes, pc, tc, stock) != FLR_OK) continue;
         if (k == 2 && 2 * fused_lds_bytes(pc, tc, false, true, 4) + 2 * kFusedStaticLds > kMaxLds) continue;
-        int64_t tiles = 0;
-        for (int s = 0; s < num_sources; ++s)
-            tiles += std::max(0, tiles_for(src[s].num_pts, src[s].tdi_start, 0, tc.tile));
-        const double rounds = std::max(1.0, (double)tiles / cus);
-        const double c = 8.0 + cost[k] * (k == 2 ? std::ceil(rounds) : rounds);
+        double tiles = 0.0;
+        for (int s = 0; s < num_sources; ++s) {
+            const int n = src[s].num_pts, start = src[s].tdi_start;
+            const int computed = tiles_for(n, start, 0, tc.tile);
+            tiles += computed + cost[k].edge * (tiles_for(n, start, zero_edges, tc.tile) - computed);
+        }
+        const double rounds = std::max(1.0, tiles / compute_units());
+        const double c = cost[k].fixed +
+                         cost[k].per_tile * (rounds + cost[k].whole * (std::ceil(rounds) - rounds));
         if (k == 1)
-            least = 0.92 * c;
+            least = 0.91 * c;
         else if (c <= least) {
             least = c;
             best = passes;
