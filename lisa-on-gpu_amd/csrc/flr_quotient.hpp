@@ -30,7 +30,9 @@ struct Recip {
 // F G, of its reciprocal and of the product by the other factor), 1 - b y = e1 comes out exactly, and
 // l = e1 y leaves e1^2 = 9 u^2 and its own rounding, 3 u^2; the product l a adds 3 u^2. Together
 // 15 u^2 = 15 2^-106, below that distance when h <= 2^c / 15: c = 8 for h <= 16, 9 up to
-// kMaxHalf (exact2_min_position). Two operations per quotient instead of div_rcp's three, and one
+// kMaxHalf (exact2_min_position). That is for a of 2^-967 or more, whose l a is a normal number; smaller
+// ones are off by units of the smallest double, and an infinite a gives an infinity or NaN where
+// div_rcp gives NaN. Two operations per quotient instead of div_rcp's three, and one
 // v_rcp_f64 (4 issue slots) per tap pair instead of two: 58 issue slots instead of 72 per tap pair of
 // six units with one fraction, 30 instead of 36 of a complex stencil, 23 instead of 27 of one unit.
 // The exact forms are bound by these FP64 operations: 1-yr FP64 drop-in (3,153,600 samples) 1.125 ->
