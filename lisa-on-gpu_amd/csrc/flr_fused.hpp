@@ -362,6 +362,7 @@ __device__ __forceinline__ void utv_mfma(const TdiConfig &tc, const FusedSource 
         const int lo = max(first, T + 16 * (q0 + 16 * g)) - m;
         const int hi = min(last, T + 16 * (q0 + 16 * g) + 255) - m;
         const bool both = kUtvNodes<TPB> && kink && lo < 0 && hi > 0;
+        if (again && !both) continue;  // m is the group's first or last sample: one side took all of it
         const int from = again ? m + 1 : first, to = sides && both && !again ? m : last;
         d4 a0[3], a1[3];
 #pragma unroll

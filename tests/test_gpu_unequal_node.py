@@ -65,3 +65,27 @@ def test_long_tiles_span_one_node_at_most(torch_gpu, dt, window):
     n = 20_000
     plan = _plan(torch_gpu, _cartwheel(), gb_waveform(n, dt), n, dt, 0.0, "2nd generation")
     assert plan.launch_shape[0] == window
+
+
+@pytest.mark.parametrize("chan", ["AET", "XYZ"])
+def test_inner_products_of_long_tiles_around_large_kinks(torch_gpu, chan):
+    """Where the samples around a node are done once for each side of it, every sample meets the data
+    once: the sums against those of the stored outputs, up to their float32 rounding."""
+    from fastlisaresponse_amd.batch import BatchedResponse
+    torch = torch_gpu
+    n, dt, t0 = 1 << 17, 10.0, 2e6
+    h = torch.as_tensor(gb_waveform(n, dt, f=4e-3, fdot=1e-16, t0=t0), device="cuda")
+    br = BatchedResponse(1 / dt, orbits=wobbly_orbits(3e-8, 1e5), tdi_chan=chan, precision="mixed-c128")
+    plan = br.plan(h, [n], [1.2], [0.3], [t0])
+    assert plan.launch_shape[0] == 1024
+    plan.run()
+    T = br.tdi_start_ind
+    g = torch.Generator(device="cuda").manual_seed(4)
+    data = torch.randn(plan.out_all.shape, generator=g, device="cuda") * plan.out_all.abs().max()
+    sums = plan.inner_products(data)[0]
+    plan.check_errors()
+    out = plan.out_all.view(3, n).double()[:, T:n - T]
+    d = data.view(3, n).double()[:, T:n - T]
+    hh, dd = out.square().sum(1), d.square().sum(1)
+    assert bool(((sums[:, 1] - hh).abs() <= 2.0 ** -23 * hh).all())
+    assert bool(((sums[:, 0] - (d * out).sum(1)).abs() <= 2.0 ** -24 * (dd * hh).sqrt()).all())
