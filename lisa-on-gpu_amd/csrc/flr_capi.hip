@@ -584,7 +584,8 @@ int inner_passes(const flr_response *r, double dt, double fs, int flags)
     TdiConfig tc;
     StockTdi stock;
     return make_fused_config(r, dt, fs, flags, 4, pc, tc, stock) == FLR_OK &&
-                   2 * fused_lds_bytes(pc, tc, false, equal, 4, !equal) + 2 * kFusedStaticLds <= kMaxLds &&
+                   2 * (fused_lds_bytes(pc, tc, false, equal, 4, !equal) +
+                        (equal ? kFusedStaticLds : kUtvStaticLds)) <= kMaxLds &&
                    (equal ? lti_filters_fit(r->orbits, fs, nx, tc)
                           : chain + r->order + 3 <= kFir &&
                                 utv_suitable(r->orbits, nx, tc.tile, dt, fs, r->deps) &&

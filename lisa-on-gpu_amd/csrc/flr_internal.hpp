@@ -195,9 +195,10 @@ struct FusedSource {
 // LDS a workgroup may take.
 constexpr size_t kMaxLds = 160 * 1024;
 
-// Static LDS of a mixed matrix-core kernel at most: the E and orbit-node copies, the unit model of
-// the unequal-arm form, the inner-product slots.
-constexpr size_t kFusedStaticLds = 6912;
+// Static LDS of a mixed matrix-core kernel at most: the E and orbit-node copies and the inner-product
+// slots; in the unequal-arm form (kUtvStaticLds) the unit model too.
+constexpr size_t kFusedStaticLds = 6656;
+constexpr size_t kUtvStaticLds = 6912;
 
 // CUs of the current device (looked up once).
 int compute_units();

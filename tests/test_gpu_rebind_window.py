@@ -149,7 +149,8 @@ def test_window_of_any_start_time(torch_gpu, orbits, lengths):
 
 
 @pytest.mark.parametrize("lengths,dt,window", [([8_552] * 48, 7.0, 512), ([74_783] * 8, 10.0, 512),
-                                               ([131_072] * 32, 10.0, 1024), ([9_001], 10.0, 256)])
+                                               ([131_072] * 32, 10.0, 1024), ([9_001], 10.0, 256),
+                                               ([131_072] * 32, 5.3, 1024)])
 def test_window_by_the_computed_tiles(torch_gpu, orbits, lengths, dt, window):
     """Tiles in the zeroed edges count nothing, and 512 samples are left only for a tenth or more."""
     from fastlisaresponse_amd.batch import BatchedResponse
